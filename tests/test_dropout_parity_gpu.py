@@ -135,6 +135,25 @@ def test_c_abi_direct_in_place_offsets_and_tails(dtype):
         assert same_bits(inplace.cpu(), whole) and same_bits(parts.cpu(), whole), f"n={n}"
 
 
+@pytest.mark.parametrize("beyond", [0, 1, 5000])
+def test_offsets_around_the_32_bit_boundary(beyond):
+    """The kernel that takes the second counter word as zero serves calls whose last offset is 2^32 - 1 at most; one more
+    element, or the boundary in the middle of a vector, takes the other one."""
+    announce(f"dropout around 2^32, beyond={beyond}")
+    lib = _native.lib()
+    st = torch.cuda.current_stream().cuda_stream
+    n, seed = 10007, 4242
+    first = 2 ** 32 - n + beyond
+    for dtype in DTYPES:
+        x = (torch.randn(n, generator=torch.Generator().manual_seed(beyond)) * 2).to(dtype)
+        xg = x.cuda()
+        out = torch.empty_like(xg)
+        for p in (1e-9, 0.37, 1.0 - 2.0 ** -24):
+            assert lib.thn_dropout(xg.data_ptr(), out.data_ptr(), n, first, p, seed, _native.dtype_code(dtype), st) == 0
+            torch.cuda.synchronize()
+            assert same_bits(out.cpu(), expected(x, p, seed, first)), f"{dtype} p={p}"
+
+
 def test_non_finite_inputs_and_extreme_p():
     announce("dropout non-finite")
     lib = _native.lib()

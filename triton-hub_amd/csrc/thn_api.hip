@@ -2388,6 +2388,7 @@ int thn_dropout(const void* x, void* out, int64_t n, int64_t first_offset, float
     a.p = p;
     a.key_lo = static_cast<uint32_t>(seed);
     a.key_hi = static_cast<uint32_t>(seed >> 32);
+    a.threshold = thn::dropout_threshold(p);
     // Bound by integer arithmetic: as many waves as a compute unit holds (8 workgroups of 256 threads).
     const int64_t blocks = (a.total_vecs + thn::kDropoutBlock - 1) / thn::kDropoutBlock;
     const int64_t cap = static_cast<int64_t>(cus) * 8;
