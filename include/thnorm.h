@@ -372,6 +372,8 @@ int thn_dropout(const void* x, void* out, int64_t n, int64_t first_offset, float
  * block_threads 0 or 256 and vecs_per_thread 0, 2 or, softmax only, 4 rows per lane and step) keeps them, any other
  * shape selects the row kernels for such rows too.  Off the 128-bit path (rows of at least one vector) they take 2 rows
  * per lane only.
+ * The softmax family's rows wider than 64 KiB: threads_per_row = 1024 with vecs_per_thread >= 8 holds every row that fits
+ * (up to 384 KiB, not float64, streams in step) in the registers of a compute unit, whatever the row count.
  * Process-wide; meant for benchmarks, not for concurrent production use.  Returns THN_E_SHAPE when no
  * compiled kernel has that shape.
  */

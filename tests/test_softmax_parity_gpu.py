@@ -22,6 +22,7 @@ from TritonHub.Activations import LogSoftmax, Softmax, Softmin, _launch
 from TritonHub.Activations.logsoftmax import logsoftmax
 from TritonHub.Activations.softmax import softmax
 from TritonHub.Activations.softmin import softmin
+from TritonHub.Normalization._launch import query_launch
 
 pytestmark = pytest.mark.gpu
 KINDS = ["softmax", "softmin", "logsoftmax"]
@@ -148,6 +149,64 @@ def test_rows_wider_than_64_kib(kind, dtype, widths):
         else:
             x[:, :17] = -3.0e4                  # log-softmax of -inf is -inf: keep the outputs finite
         run_and_compare(kind, x, dy, f"{kind} wide N={n}")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("kind", KINDS)
+def test_rows_held_by_a_compute_unit(kind, dtype):
+    """Rows of 64 KiB to 384 KiB in the registers of one workgroup: both sides of every change of the vectors per thread,
+    rows that start at every offset from a 16-byte boundary, more rows than compute units, fewer rows than those; streams
+    that do not start in step, which the looping kernels take."""
+    vec = 16 // torch.empty((), dtype=dtype).element_size()
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    lib = _native.lib()
+    log = kind == "logsoftmax"
+    # by default: float32 forwards and log-softmax backwards at any row count, the others from 24 MiB per tensor on
+    m = 24 * 2 ** 20 // (4097 * 16)
+    for which, always in ((2, dtype == torch.float32), (3, log)):
+        for rows, wide in ((3, always), (m, always), (m + 1, True)):
+            assert query_launch(which, log, rows, 4097 * vec, dtype)[0] == (8 if wide else 4), (which, rows)
+    try:
+        for which in (2, 3):
+            assert lib.thn_norm_set_launch_override(which, 8, 1024, 0, 0) == 0
+        for k, nxt in ((4, 8), (8, 12), (12, 16), (16, 20), (20, 24), (24, 0)):
+            for n in (k * 1024 * vec - 1, k * 1024 * vec, k * 1024 * vec + vec - 1, k * 1024 * vec + vec):
+                if n <= 4096 * vec:
+                    continue
+                want = max(8, k) if n // vec <= k * 1024 else nxt
+                for which in (2, 3):
+                    assert query_launch(which, log, 3, n, dtype)[:3] == ((want, 1024, 1024) if want else (4, 1024, 1024)), n
+                announce(f"rows in a compute unit {kind} {dtype} N={n}")
+                x, dy = make((3, n), dtype, seed=n, scale=3.0)
+                run_and_compare(kind, x, dy, f"{kind} N={n}")
+    finally:
+        for which in (2, 3):
+            lib.thn_norm_set_launch_override(which, 0, 0, 0, 0)
+    n = 4096 * vec + 5
+    announce(f"rows in a compute unit {kind} {dtype} {2 * cus - 3} x {n}")
+    x, dy = make((2 * cus - 3, n), dtype, seed=1, scale=3.0)
+    run_and_compare(kind, x, dy, f"{kind} {2 * cus - 3} x {n}")
+    x, dy = (t.to("cuda") for t in make((2 * cus - 3, n), dtype, seed=1, scale=3.0))
+    module = MODULE[kind]()
+    apart = torch.empty(x.numel() + 1, dtype=dtype, device="cuda")[1:].view_as(x).copy_(x).requires_grad_(True)
+    y0 = module(apart)
+    y1 = module(x.requires_grad_(True))
+    dx0, dx1 = torch.autograd.grad(y0, apart, dy)[0], torch.autograd.grad(y1, x, dy)[0]
+    eps = torch.finfo(dtype).eps                            # both are within an ulp and a few float32 roundings of the same value
+    assert torch.allclose(y0.double(), y1.double(), rtol=2 * eps + 2e-6, atol=1e-6)
+    assert torch.allclose(dx0.double(), dx1.double(), rtol=2 * eps + 1e-5, atol=1e-6)
+
+
+@pytest.mark.parametrize("n", [32768 + 8, 400000])
+def test_a_nan_spoils_its_wide_row_and_no_other(n):
+    """A NaN in a row wider than 64 KiB, in registers or walked twice: the row is NaN, as a narrow row is; -inf is not."""
+    for kind, rows in (("softmax", 4), ("logsoftmax", 400)):
+        x = torch.randn(rows, n, dtype=torch.bfloat16, device="cuda")
+        x[1, 77] = float("nan")
+        x[2, ::2] = float("-inf")
+        y = MODULE[kind]()(x)
+        assert bool(torch.isnan(y[1]).all())
+        assert not bool(torch.isnan(y[0]).any()) and not bool(torch.isnan(y[2:]).any())
 
 
 @pytest.mark.parametrize("kind", KINDS)

@@ -6,6 +6,7 @@
 #include <initializer_list>
 #include <mutex>
 #include <unordered_map>
+#include <utility>
 
 #include "thn_dispatch.h"
 #include "thn_flat.h"
@@ -17,6 +18,7 @@
 #include "thn_pnorm_dispatch.h"
 #include "thn_softmax_dispatch.h"
 #include "thn_softmax_flat.h"
+#include "thn_softmax_wide.h"
 #include "thn_pnorm_flat.h"
 #include "thn_tiny.h"
 
@@ -403,6 +405,54 @@ int default_blocks_per_cu(int which, int flavour, int block) {
     // as many workgroups per compute unit as their registers allow, up to four.
     if ((which == kFusedFwd || which == kFusedBwd) && ((flavour >> 1) == thn::kGelu || (flavour >> 1) == thn::kGeluTanh)) return 4;
     return kDefaultBlocksPerCu;
+}
+
+// Vectors per thread of the register-resident softmax kernels (thn_softmax_wide.h) for M rows of N columns, 0 where the
+// looping kernels run: float64, rows of more than 24 x 1024 vectors, an overridden launch shape of those kernels, and where
+// the second walk costs nothing, because what it reads still lies in the eight 4-MiB L2s:
+//   forward, 16-bit: x of less than 24 MiB (bfloat16 looping -> registers, softmax: 64 x 40000 9.1 -> 9.9 us, 192 x 40000 10.0 ->
+//     10.6, 64 x 90001 16.2 -> 17.5, 192 x 90001 21.5 -> 18.7, 512 x 151936 75.5 -> 63.7).  float32 rows have half the
+//     elements per byte and gain at every row count (32 x 40000 10.1 -> 8.9, 256 x 40000 18.8 -> 15.4);
+//   softmax backward (which reads y twice either way): y and dy of less than 48 MiB together (bfloat16 64 x 40000 7.9 -> 8.3,
+//     300 x 40000 19.1 -> 19.8, 256 x 90001 37.2 -> 26.8), and float32 rows that need 24 vectors per thread (spills).
+//     The log-softmax backward gains everywhere (bfloat16 16 x 40000 8.5 -> 7.8, 300 x 90001 45.2 -> 39.7).
+int softmax_wide_vecs(int which, bool is_log, int64_t M, int64_t N, int dtype) {
+    const int bytes = elem_bytes(dtype);
+    const int64_t vecs = N / (16 / bytes);
+    if (dtype == THN_F64 || vecs > thn::kWideMaxVecs) return 0;
+    int k = static_cast<int>((vecs + 4 * thn::kWideBlock - 1) / (4 * thn::kWideBlock)) * 4;
+    if (k < 8) k = 8;
+    const Override& ov = g_override[which];
+    if (ov.k.load() >= 8 && ov.tpr.load() == thn::kWideBlock) return k;
+    if (ov.block.load() > 0 || ov.bpc.load() > 0) return 0;
+    const int64_t mib = M * N * bytes >> 20;
+    if (which == kSoftmaxFwd && bytes == 2 && mib < 24) return 0;
+    if (which == kSoftmaxBwd && !is_log && (mib < 24 || (bytes == 4 && k == 24))) return 0;
+    return k;
+}
+
+// Every row of every stream starts at the same offset from a 16-byte boundary, on an element.
+bool same_phase(std::initializer_list<std::pair<const void*, int64_t>> streams, int64_t M, int bytes) {
+    const uintptr_t base = reinterpret_cast<uintptr_t>(streams.begin()->first);
+    const int64_t stride = streams.begin()->second;
+    if (base % static_cast<uintptr_t>(bytes) != 0) return false;
+    for (const auto& s : streams) {
+        if ((reinterpret_cast<uintptr_t>(s.first) - base) % 16 != 0 || (M > 1 && (s.second - stride) % 16 != 0)) return false;
+    }
+    return true;
+}
+
+#define THN_WIDE_SWITCH(CALL)                                                                                  \
+    switch (dtype) {                                                                                           \
+        case THN_F32: return thn::CALL##_f32(is_log, k, a, grid, st);                                          \
+        case THN_F16: return thn::CALL##_f16(is_log, k, a, grid, st);                                          \
+        default: return thn::CALL##_bf16(is_log, k, a, grid, st);                                              \
+    }
+int launch_softmax_fwd_wide(int dtype, bool is_log, int k, const SoftmaxFwdArgs& a, int grid, hipStream_t st) {
+    THN_WIDE_SWITCH(launch_softmax_fwd_wide)
+}
+int launch_softmax_bwd_wide(int dtype, bool is_log, int k, const SoftmaxBwdArgs& a, int grid, hipStream_t st) {
+    THN_WIDE_SWITCH(launch_softmax_bwd_wide)
 }
 
 void softmax_loop_launch(int which, int* block, int* bpc) {
@@ -1791,6 +1841,14 @@ int thn_norm_query_launch(int which, int is_layernorm, int64_t M, int64_t N, int
             softmax_loop_launch(which, &block, &bpc);
             const int64_t cap = static_cast<int64_t>(cus) * bpc;
             grid = static_cast<int>(M < cap ? M : cap);
+            const int k = softmax_wide_vecs(which, flavour & 1, M, N, x_dtype);
+            if (k > 0) {                            // rows in the registers of a compute unit (dense tensors)
+                shape[0] = k;
+                shape[1] = shape[2] = thn::kWideBlock;
+                shape[3] = static_cast<int>(M < cus ? M : cus);
+                shape[4] = 1;
+                return THN_OK;
+            }
         }
         shape[0] = thn::kWalkVecs;
         shape[1] = block;
@@ -2048,11 +2106,17 @@ int thn_softmax_fwd(const void* x, int64_t x_row_stride, void* y, int64_t y_row_
         a.M = M;
         a.n_cols = static_cast<int>(N);
         a.sign = kind == THN_SOFTMIN ? -1.0f : 1.0f;
-        int block, bpc;
+        int block, bpc, lrc;
         softmax_loop_launch(kSoftmaxFwd, &block, &bpc);
-        const int64_t cap = static_cast<int64_t>(cus) * bpc;
-        const int grid = static_cast<int>(M < cap ? M : cap);
-        const int lrc = launch_softmax_fwd_loop(dtype, kind == THN_LOGSOFTMAX, block, a, grid, static_cast<hipStream_t>(stream));
+        const int k = softmax_wide_vecs(kSoftmaxFwd, kind == THN_LOGSOFTMAX, M, N, dtype);
+        if (k > 0 && same_phase({{x, a.x_stride_bytes}, {y, a.y_stride_bytes}}, M, bytes)) {
+            const int grid = static_cast<int>(M < cus ? M : cus);
+            lrc = launch_softmax_fwd_wide(dtype, kind == THN_LOGSOFTMAX, k, a, grid, static_cast<hipStream_t>(stream));
+        } else {
+            const int64_t cap = static_cast<int64_t>(cus) * bpc;
+            const int grid = static_cast<int>(M < cap ? M : cap);
+            lrc = launch_softmax_fwd_loop(dtype, kind == THN_LOGSOFTMAX, block, a, grid, static_cast<hipStream_t>(stream));
+        }
         if (lrc > 0) return THN_E_SHAPE;
         return lrc == 0 ? THN_OK : THN_E_LAUNCH;
     }
@@ -2135,11 +2199,17 @@ int thn_softmax_bwd(const void* y, int64_t y_row_stride, const void* dy, int64_t
         a.M = M;
         a.n_cols = static_cast<int>(N);
         a.sign = kind == THN_SOFTMIN ? -1.0f : 1.0f;
-        int block, bpc;
+        int block, bpc, lrc;
         softmax_loop_launch(kSoftmaxBwd, &block, &bpc);
-        const int64_t cap = static_cast<int64_t>(cus) * bpc;
-        const int grid = static_cast<int>(M < cap ? M : cap);
-        const int lrc = launch_softmax_bwd_loop(dtype, kind == THN_LOGSOFTMAX, block, a, grid, static_cast<hipStream_t>(stream));
+        const int k = softmax_wide_vecs(kSoftmaxBwd, kind == THN_LOGSOFTMAX, M, N, dtype);
+        if (k > 0 && same_phase({{y, a.y_stride_bytes}, {dy, a.dy_stride_bytes}, {dx, a.dx_stride_bytes}}, M, bytes)) {
+            const int grid = static_cast<int>(M < cus ? M : cus);
+            lrc = launch_softmax_bwd_wide(dtype, kind == THN_LOGSOFTMAX, k, a, grid, static_cast<hipStream_t>(stream));
+        } else {
+            const int64_t cap = static_cast<int64_t>(cus) * bpc;
+            const int grid = static_cast<int>(M < cap ? M : cap);
+            lrc = launch_softmax_bwd_loop(dtype, kind == THN_LOGSOFTMAX, block, a, grid, static_cast<hipStream_t>(stream));
+        }
         if (lrc > 0) return THN_E_SHAPE;
         return lrc == 0 ? THN_OK : THN_E_LAUNCH;
     }

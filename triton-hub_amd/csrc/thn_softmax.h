@@ -259,7 +259,8 @@ __global__ void __launch_bounds__(BLOCK) softmax_bwd_kernel(const SoftmaxBwdArgs
 // ---------------------------------------------------------------------------------------------------
 // Rows wider than 64 KiB (the reference cuts such a row into 64 KiB chunks and normalises each chunk by itself,
 // softmax.py:34-40 -- which is not a softmax of the row; here the row is one softmax).  One 1024-thread workgroup
-// per row, grid-stride over rows, two walks per row (thn_walk.h); the second comes from the L2 / Infinity Cache.
+// per row, grid-stride over rows, two walks per row (thn_walk.h); the second comes from the L2 / Infinity Cache.  Rows that
+// a compute unit can hold in its registers run thn_softmax_wide.h instead where that is faster (softmax_wide_vecs()).
 //   forward:  walk 1 keeps a running maximum m and sum(exp(x - m)) per thread (the sum is rescaled whenever the
 //             maximum moves: a few times per thread), combined over the workgroup; walk 2 writes y;
 //   backward: walk 1 sum(y*g) (log-softmax: sum(g)); walk 2 writes dx.
@@ -285,7 +286,7 @@ __global__ void __launch_bounds__(kSoftmaxLoopBlock) softmax_fwd_loop_kernel(con
                 acc *= static_cast<double>(exp_c(m - v));          // m = -inf: 0
                 m = v;
             }
-            acc += v > neg_inf ? static_cast<double>(exp_c(v - m)) : 0.0;   // -inf - -inf must not poison the sum
+            acc += v == neg_inf ? 0.0 : static_cast<double>(exp_c(v - m));   // -inf - -inf must not poison the sum (a NaN does)
             return C(0);
         };
         walk_row_vec<T, C, kSoftmaxLoopBlock, 1, false, true, true>(
@@ -304,13 +305,13 @@ __global__ void __launch_bounds__(kSoftmaxLoopBlock) softmax_fwd_loop_kernel(con
                 }
                 C part = C(0);
 #pragma unroll
-                for (int e = 0; e < T::VEC; ++e) part += v[e] > neg_inf ? exp_c(v[e] - m) : C(0);
+                for (int e = 0; e < T::VEC; ++e) part += v[e] == neg_inf ? C(0) : exp_c(v[e] - m);
                 acc += static_cast<double>(part);
             },
             one);
         C mx[1] = {m};
         row_allreduce<kSoftmaxLoopBlock, 1, 1, OpMax, C>(mx, red, phase, 0, t);
-        double s[1] = {m > neg_inf ? acc * static_cast<double>(exp_c(m - mx[0])) : 0.0};
+        double s[1] = {acc == 0.0 ? 0.0 : acc * static_cast<double>(exp_c(m - mx[0]))};
         row_allreduce<kSoftmaxLoopBlock, 1, 1, OpSum, double>(s, red_sum, phase_sum, 0, t);
         const C row_max = mx[0];
         C scale;
