@@ -583,7 +583,8 @@ __global__ void __launch_bounds__(BLOCK) norm_bwd_kernel(const BwdArgs a) {
         for (int i = 0; i < NV; ++i) s[i] = 0.0f;
         float dlt_fused = 0.0f;
         if constexpr (FUSED && LN) {
-            // first round: dlt = sum(u)/N, so that z below is built from the corrected xhat
+            // first round: sum(x - mean), so that z below is built from the corrected xhat (x - mean)*rstd - dlt with
+            // dlt = sum(x - mean)*rstd/N, one multiply-add per element
             float su[1] = {0.0f};
 #pragma unroll
             for (int k = 0; k < K; ++k) {
@@ -591,14 +592,13 @@ __global__ void __launch_bounds__(BLOCK) norm_bwd_kernel(const BwdArgs a) {
                 float sk = 0.0f;
 #pragma unroll
                 for (int e = 0; e < VEC; ++e) {
-                    const float v = (u[k][e] - c_mean) * c_rstd;
-                    u[k][e] = v;
-                    sk += counts(k, e) ? v : 0.0f;
+                    u[k][e] -= c_mean;
+                    sk += counts(k, e) ? u[k][e] : 0.0f;
                 }
                 su[0] += own[k] ? sk : 0.0f;
             }
             row_allreduce<TPR, G, 1>(su, red, phase, g, t);
-            dlt_fused = su[0] * a.inv_n;
+            dlt_fused = su[0] * a.inv_n * c_rstd;
         }
 #pragma unroll
         for (int k = 0; k < K; ++k) {
@@ -608,7 +608,7 @@ __global__ void __launch_bounds__(BLOCK) norm_bwd_kernel(const BwdArgs a) {
 #pragma unroll
             for (int e = 0; e < VEC; ++e) {
                 if constexpr (FUSED && LN) {
-                    u[k][e] -= dlt_fused;                               // the corrected xhat
+                    u[k][e] = fmaf(u[k][e], c_rstd, -dlt_fused);        // the corrected xhat
                 } else if constexpr (LN) {
                     u[k][e] = (u[k][e] - c_mean) * c_rstd;
                 } else {
