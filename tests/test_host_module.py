@@ -1,0 +1,80 @@
+"""The native host module (TritonHub/_host.so) against the Python wrappers' general way: the same bits for every form of call
+that it takes, and None for what it leaves to them."""
+import pytest
+import torch
+
+from TritonHub import _native
+from TritonHub.Activations import _launch as act_launch
+from TritonHub.Normalization import _launch as norm_launch
+
+
+class _General:
+    """Stands in for the host module: everything goes the general way."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
+def test_host_tensors_and_wrong_argument_counts():
+    host, x = _native.host(), torch.randn(4, 8)
+    assert host.norm_fwd(x, None, None, 1e-5, True, -1, 0) is None
+    assert host.norm_bwd(x, x, None, None, None, x, False, -1, True, True) is None
+    assert host.softmax_fwd(x, 0) is None and host.softmax_bwd(x, x, 0) is None
+    assert host.act_fwd(x, 0, 0.0, 0.0) is None and host.act_bwd(x, x, 0, 0.0, 0.0) is None
+    assert host.softmax_fwd(None, 0) is None and host.softmax_fwd("x", 0) is None
+    for name, count in (("norm_fwd", 7), ("norm_bwd", 10), ("softmax_fwd", 2), ("softmax_bwd", 3), ("act_fwd", 4), ("act_bwd", 5)):
+        with pytest.raises(TypeError):
+            getattr(host, name)(*[x] * (count - 1))
+
+
+def _same(a, b):
+    if a is None or b is None:
+        return a is None and b is None
+    return a.dtype == b.dtype and a.shape == b.shape and a.stride() == b.stride() and torch.equal(a, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16, torch.float64])
+@pytest.mark.parametrize("shape", [(1,), (7,), (3, 1, 5), (2, 100, 128), (65, 4098)])
+def test_same_bits_as_the_general_way(shape, dtype, monkeypatch):
+    host, n = _native.host(), shape[-1]
+    g = torch.Generator(device="cuda").manual_seed(n)
+    x, dy = (torch.randn(*shape, device="cuda", generator=g).to(dtype) for _ in range(2))
+    w, b = (torch.randn(n, device="cuda", generator=g).to(dtype) for _ in range(2))
+    w32 = w.float()
+
+    def norms(act):
+        for layernorm in (True, False):
+            for weight, bias in ((w, b), (w, None), (None, None), (w32, None), (None, b), (w32, b)):
+                if bias is not None and not layernorm:
+                    continue
+                y, mean, rstd = norm_launch.norm_fwd(x, weight, bias, 1e-5, layernorm, act)
+                yield from (y, mean, rstd)
+                for need_dw, need_db in ((True, True), (False, True), (True, False), (False, False)):
+                    yield from norm_launch.norm_bwd(x, dy, weight, bias, mean, rstd, layernorm, act, need_dw, need_db)
+
+    def everything():
+        yield from norms(-1)
+        yield from norms(_native.ACT_SILU)
+        for kind in (_native.SOFTMAX, _native.SOFTMIN, _native.LOGSOFTMAX):
+            y = act_launch.softmax_fwd(x, kind)
+            yield from (y, act_launch.softmax_bwd(y, dy, kind))
+        for act, p0, p1 in ((_native.ACT_GELU, 0.0, 0.0), (_native.ACT_LEAKY_RELU, 0.1, 0.0), (_native.ACT_THRESHOLD, 0.2, -1)):
+            yield from (act_launch.act_fwd(x, act, p0, p1), act_launch.act_bwd(x, dy, act, p0, p1))
+
+    here = list(everything())
+    monkeypatch.setattr(_native, "host", lambda: _General())
+    general = list(everything())
+    assert len(here) == len(general) and all(_same(a, c) for a, c in zip(here, general))
+    # what it takes, and what it leaves to the wrappers
+    assert host.norm_fwd(x, w, b, 1e-5, True, -1, 0) is not None and host.softmax_fwd(x, 0) is not None
+    assert host.norm_fwd(x, w32, b, 1e-5, True, -1, 0) is None or dtype == torch.float32
+    rstd = torch.ones(x.numel() // n, device="cuda")
+    assert host.norm_bwd(x, dy.double() if dtype != torch.float64 else dy.float(), w, None, None, rstd, False, -1, True, True) is None
+    assert host.norm_bwd(x, dy, w, None, None, rstd.double(), False, -1, True, True) is None
+    assert host.norm_fwd(x, torch.ones(n + 1, device="cuda", dtype=dtype), None, 1e-5, True, -1, 0) is None
+    assert host.softmax_fwd(x[..., :0], 0) is None and host.softmax_fwd(x.expand(2, *shape), 0) is None
+    assert host.softmax_fwd(torch.ones(4, 4, device="cuda", dtype=torch.int32), 0) is None
+    assert host.softmax_bwd(x, dy.reshape(-1, 1), 0) is None or n == 1
+    with pytest.raises(RuntimeError, match="libthnorm"):
+        host.softmax_fwd(x, 9)

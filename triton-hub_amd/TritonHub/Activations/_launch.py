@@ -46,6 +46,9 @@ def _call(device, fn_name, *args):
 
 
 def softmax_fwd(x: torch.Tensor, kind: int) -> torch.Tensor:
+    done = _native.host().softmax_fwd(x, kind)
+    if done is not None:
+        return done
     if not x.is_cuda:
         _native.require_gpu(x)
     x2, m, n, x_stride, reshaped = _flatten(x)
@@ -60,6 +63,9 @@ def softmax_fwd(x: torch.Tensor, kind: int) -> torch.Tensor:
 
 def softmax_bwd(y: torch.Tensor, dout: torch.Tensor, kind: int) -> torch.Tensor:
     """`y` is the saved OUTPUT of the forward (softmax.py:86-97)."""
+    done = _native.host().softmax_bwd(y, dout, kind)
+    if done is not None:
+        return done
     if not y.is_cuda:
         _native.require_gpu(y)
     y2, m, n, y_stride, reshaped = _flatten(y)
@@ -78,6 +84,9 @@ def softmax_bwd(y: torch.Tensor, dout: torch.Tensor, kind: int) -> torch.Tensor:
 def act_fwd(x: torch.Tensor, act: int, param0: float = 0.0, param1: float = 0.0) -> torch.Tensor:
     """Element-wise forward: what the reference's ``_<name>_fwd`` wrappers do on the host (e.g. gelu.py:31-49) --
     last dimension contiguous, flatten to (M, N), allocate the output with the same assertions -- then the C ABI."""
+    done = _native.host().act_fwd(x, act, param0, param1)
+    if done is not None:
+        return done
     if not x.is_cuda:
         _native.require_gpu(x)
     x2, m, n, x_stride, reshaped = _flatten(x)
@@ -92,6 +101,9 @@ def act_fwd(x: torch.Tensor, act: int, param0: float = 0.0, param1: float = 0.0)
 
 def act_bwd(saved: torch.Tensor, dout: torch.Tensor, act: int, param0: float = 0.0, param1: float = 0.0) -> torch.Tensor:
     """Element-wise backward (e.g. gelu.py:83-105); ``saved`` is what the reference's Function saved."""
+    done = _native.host().act_bwd(saved, dout, act, param0, param1)
+    if done is not None:
+        return done
     if not saved.is_cuda:
         _native.require_gpu(saved)
     s2, m, n, s_stride, reshaped = _flatten(saved)

@@ -125,6 +125,9 @@ def norm_fwd(x: torch.Tensor, weight, bias, eps: float, layernorm: bool, act: in
     """Returns (y like x, mean (M,) float32 or None, rstd (M,) float32).  `act` >= 0: the activation with that
     code is applied in the same pass (thn_norm_act_fwd).  `backward_follows`: whether autograd will run a backward
     for this call (it decides the cache policy of the read of x under set_cache_policy('auto'))."""
+    done = _native.host().norm_fwd(x, weight, bias, eps, layernorm, act, _x_policy_flag(backward_follows))
+    if done is not None:
+        return done
     if not x.is_cuda:
         _native.require_gpu(x)
     x2, m, n, x_stride, reshaped = _flatten(x, 'input')
@@ -182,6 +185,9 @@ def norm_bwd(x: torch.Tensor, dout: torch.Tensor, weight, bias, mean, rstd, laye
     `act` >= 0: the backward of norm_fwd(..., act) (thn_norm_act_bwd).  `need_dw` / `need_db` False: that parameter
     is frozen (autograd's needs_input_grad): its sums are not stored, and with both False the backward is the row
     kernel alone, without partial sums and without the second stage."""
+    done = _native.host().norm_bwd(x, dout, weight, bias, mean, rstd, layernorm, act, need_dw, need_db)
+    if done is not None:
+        return done
     if not x.is_cuda:
         _native.require_gpu(x)
     x2, m, n, x_stride, reshaped = _flatten(x, 'input')

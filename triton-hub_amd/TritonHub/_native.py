@@ -1,4 +1,4 @@
-"""ctypes binding of ``libthnorm.so`` -- the only way the Python layer reaches the GPU.
+"""ctypes binding of ``libthnorm.so`` and the native host module over it -- the only ways the Python layer reaches the GPU.
 
 There is no fallback: if the shared library is missing or a call fails, an exception is raised.  The
 library is built by ``triton-hub_amd/csrc/Makefile`` (``python __graft_entry__.py`` at the repository
@@ -7,6 +7,7 @@ root drives it) and lives next to this file.
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import os
 import threading
 
@@ -14,6 +15,7 @@ import torch
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, 'libthnorm.so')
+HOST_PATH = os.path.join(_HERE, '_host.so')
 
 F32, F16, BF16, F64 = 0, 1, 2, 3
 SOFTMAX, SOFTMIN, LOGSOFTMAX = 0, 1, 2
@@ -81,6 +83,28 @@ def lib():
                     fn.argtypes = argtypes
                 _lib = handle
     return _lib
+
+
+_host = None
+
+
+def host():
+    """The native host module (csrc/thn_host.cpp): one function per launch wrapper, which makes the whole call for ordinary
+    tensors and returns None for any other; raises if it has not been built."""
+    global _host
+    if _host is None:
+        with _lock:
+            if _host is None:
+                for path in (LIB_PATH, HOST_PATH):
+                    if not os.path.exists(path):
+                        raise RuntimeError(
+                            f'{path} is missing: build the HIP extension first '
+                            '(make -C triton-hub_amd/csrc, or __graft_entry__.build()). There is no CPU fallback.')
+                spec = importlib.util.spec_from_file_location('TritonHub._host', HOST_PATH)
+                module = importlib.util.module_from_spec(spec)
+                spec.loader.exec_module(module)
+                _host = module
+    return _host
 
 
 def strerror(status: int) -> str:
