@@ -226,3 +226,39 @@ def test_random_sizes_offsets_seeds_and_alignments():
         what = f"case {case}: {dtype} n={n} skew=({skew_in},{skew_out}) first={first} seed={seed} p={p:.3f}"
         assert same_bits(got[skew_out:skew_out + n].contiguous(), expected(x[skew_in:].contiguous(), p, seed, first)), what
         assert bool((got[:skew_out] == 7).all()) and bool((got[skew_out + n:] == 7).all()), what + " (wrote outside)"
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16, torch.float64])
+@pytest.mark.parametrize("n", [(1 << 22) - 1, 1 << 22, (1 << 22) + 1, (1 << 22) + 13, (1 << 22) + 5000])
+def test_kept_decisions_give_the_bits_of_drawn_ones(n, dtype):
+    """From 2^22 elements on the backward reads the decisions that the forward kept: both directions against thn_dropout
+    with the same seed, for whole vectors and tails, every p that keeps something, gradients off the 16-byte path, a
+    strided gradient (drawn again) and a second backward through the same graph."""
+    g = torch.Generator(device="cuda").manual_seed(n)
+    x, dy = (torch.randn(n, device="cuda", generator=g, dtype=torch.float32).to(dtype) for _ in range(2))
+    x[3], x[8], dy[5], dy[7] = float("inf"), float("nan"), float("-inf"), float("nan")
+
+    def drawn(t, p, seed):
+        out = torch.empty_like(t)
+        assert _native.lib().thn_dropout(t.data_ptr(), out.data_ptr(), n, 0, p, seed, _native.dtype_code(dtype), 0) == 0
+        return out
+
+    bits = {2: torch.int16, 4: torch.int32, 8: torch.int64}[x.element_size()]
+    same = lambda a, b: torch.equal(a.view(bits), b.view(bits))
+    for p in (1e-3, 0.1, 0.5, 0.999, 1.0 - 2.0 ** -24):
+        random.seed(n)
+        seed = random.randint(0, 2 ** 16)
+        random.seed(n)
+        module, xg = Dropout(p), x.clone().requires_grad_(True)
+        y = module(xg)
+        assert len(y.grad_fn.saved_tensors) == (1 if n >= 1 << 22 else 0)
+        want = drawn(dy, p, seed)
+        assert same(y.detach(), drawn(x, p, seed))
+        assert same(torch.autograd.grad(y, xg, dy, retain_graph=True)[0], want)
+        off = torch.empty(n + 1, dtype=dtype, device="cuda")[1:].copy_(dy)
+        assert same(torch.autograd.grad(y, xg, off, retain_graph=True)[0], want)
+        wide = torch.empty(n, 2, dtype=dtype, device="cuda")[:, 0].copy_(dy)
+        assert same(torch.autograd.grad(y, xg, wide)[0], want)
+        random.seed(n)
+        with torch.no_grad():
+            assert same(module(x), drawn(x, p, seed))

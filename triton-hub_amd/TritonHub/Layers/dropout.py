@@ -36,20 +36,31 @@ def _dropout_apply(t: torch.Tensor, p, seed, training, what: str) -> torch.Tenso
 
 
 class dropout(torch.autograd.Function):
-    """forward(ctx, input, p, training) -> output; keeps (p, seed, training) on ctx and no tensor: the backward
-    regenerates the mask from the seed."""
+    """forward(ctx, input, p, training) -> output; keeps (p, seed, training) on ctx.  A large input that requires a gradient
+    also saves which elements were dropped (one byte per 16 bytes of input), and the backward reads them; every other
+    backward regenerates the mask from the seed.  The two give the same bits."""
 
     @staticmethod
     def forward(ctx, input, p, training):
         seed = random.randint(0, 2**16)
-        output = _dropout_apply(input, p, seed, training, 'input')
         ctx.p = p
         ctx.seed = seed
         ctx.training = training
+        done = _native.host().dropout_fwd(input, p, seed, ctx.needs_input_grad[0]) if training else None
+        if done is None:
+            return _dropout_apply(input, p, seed, training, 'input')
+        output, mask = done
+        if mask is not None:
+            ctx.save_for_backward(mask)
         return output
 
     @staticmethod
     def backward(ctx, d_out):
+        if ctx.training:
+            saved = ctx.saved_tensors
+            grad = _native.host().dropout_bwd(d_out, ctx.p, ctx.seed, saved[0] if saved else None)
+            if grad is not None:
+                return grad, None, None
         grad = _dropout_apply(d_out, ctx.p, ctx.seed, ctx.training, 'gradient')
         return grad, None, None
 

@@ -15,6 +15,7 @@
 #include "thn_reduce.h"
 #include "thn_act_dispatch.h"
 #include "thn_dropout.h"
+#include "thn_dropout_mask.h"
 #include "thn_pnorm_dispatch.h"
 #include "thn_softmax_dispatch.h"
 #include "thn_softmax_flat.h"
@@ -1700,6 +1701,41 @@ int act_blocks_per_cu(int act, bool bwd, int bytes) {
     return 2;
 }
 
+int dropout_launch(thn::DropoutMask mode, const void* x, void* out, uint32_t* mask, int64_t n, int64_t first_offset, float p,
+                   uint64_t seed, int dtype, void* stream) {
+    const int bytes = elem_bytes(dtype);
+    if (bytes == 0) return THN_E_DTYPE;
+    if (n < 0 || first_offset < 0 || !(p >= 0.0f && p <= 1.0f)) return THN_E_SHAPE;
+    if (n == 0) return THN_OK;
+    if (x == nullptr || out == nullptr || (mode != thn::DropoutMask::kNone && mask == nullptr)) return THN_E_NULL;
+    if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(out)) % static_cast<uintptr_t>(bytes) != 0) {
+        return THN_E_SHAPE;
+    }
+    const int cus = current_cu_count();
+    if (cus <= 0) return THN_E_DEVICE;
+    thn::DropoutArgs a{};
+    a.x = static_cast<const char*>(x);
+    a.out = static_cast<char*>(out);
+    a.total_elems = n;
+    a.total_vecs = n / (16 / bytes);
+    a.first_offset = first_offset;
+    a.p = p;
+    a.key_lo = static_cast<uint32_t>(seed);
+    a.key_hi = static_cast<uint32_t>(seed >> 32);
+    a.threshold = thn::dropout_threshold(p);
+    a.mask = mask;
+    if (mode != thn::DropoutMask::kNone && (a.threshold == thn::kDropAll || a.total_vecs > thn::kMaskedMost)) return THN_E_SHAPE;
+    // Bound by integer arithmetic: as many waves as a compute unit holds (8 workgroups of 256 threads).  From a mask, by
+    // memory: 4 workgroups, as the element-wise kernels.
+    const int64_t per_block = static_cast<int64_t>(thn::kDropoutBlock) * (mode == thn::DropoutMask::kNone ? 1 : thn::kMaskedVecs);
+    const int64_t blocks = (a.total_vecs + per_block - 1) / per_block;
+    const int64_t cap = static_cast<int64_t>(cus) * (mode == thn::DropoutMask::kRead ? 4 : 8);
+    const int grid = static_cast<int>(blocks < 1 ? 1 : (blocks < cap ? blocks : cap));
+    const int rc = thn::launch_dropout(dtype, mode, a, grid, static_cast<hipStream_t>(stream));
+    if (rc > 0) return THN_E_DTYPE;
+    return rc == 0 ? THN_OK : THN_E_LAUNCH;
+}
+
 int act_launch(const void* x, int64_t x_row_stride, const void* g, int64_t g_row_stride, void* out,
                int64_t out_row_stride, int64_t M, int64_t N, int act, float p0, float p1, int dtype, bool bwd,
                void* stream) {
@@ -2439,33 +2475,19 @@ int thn_act_bwd(const void* saved, int64_t saved_row_stride, const void* dy, int
 
 int thn_dropout(const void* x, void* out, int64_t n, int64_t first_offset, float p, uint64_t seed, int dtype,
                 void* stream) {
-    const int bytes = elem_bytes(dtype);
-    if (bytes == 0) return THN_E_DTYPE;
-    if (n < 0 || first_offset < 0 || !(p >= 0.0f && p <= 1.0f)) return THN_E_SHAPE;
-    if (n == 0) return THN_OK;
-    if (x == nullptr || out == nullptr) return THN_E_NULL;
-    if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(out)) % static_cast<uintptr_t>(bytes) != 0) {
-        return THN_E_SHAPE;
-    }
-    const int cus = current_cu_count();
-    if (cus <= 0) return THN_E_DEVICE;
-    thn::DropoutArgs a{};
-    a.x = static_cast<const char*>(x);
-    a.out = static_cast<char*>(out);
-    a.total_elems = n;
-    a.total_vecs = n / (16 / bytes);
-    a.first_offset = first_offset;
-    a.p = p;
-    a.key_lo = static_cast<uint32_t>(seed);
-    a.key_hi = static_cast<uint32_t>(seed >> 32);
-    a.threshold = thn::dropout_threshold(p);
-    // Bound by integer arithmetic: as many waves as a compute unit holds (8 workgroups of 256 threads).
-    const int64_t blocks = (a.total_vecs + thn::kDropoutBlock - 1) / thn::kDropoutBlock;
-    const int64_t cap = static_cast<int64_t>(cus) * 8;
-    const int grid = static_cast<int>(blocks < 1 ? 1 : (blocks < cap ? blocks : cap));
-    const int rc = thn::launch_dropout(dtype, a, grid, static_cast<hipStream_t>(stream));
-    if (rc > 0) return THN_E_DTYPE;
-    return rc == 0 ? THN_OK : THN_E_LAUNCH;
+    return dropout_launch(thn::DropoutMask::kNone, x, out, nullptr, n, first_offset, p, seed, dtype, stream);
 }
 
 }  // extern "C"
+
+namespace thn {
+
+int dropout_keep_mask(const void* x, void* out, uint32_t* mask, int64_t n, float p, uint64_t seed, int dtype, void* stream) {
+    return dropout_launch(DropoutMask::kWrite, x, out, mask, n, 0, p, seed, dtype, stream);
+}
+
+int dropout_from_mask(const void* x, void* out, const uint32_t* mask, int64_t n, float p, uint64_t seed, int dtype, void* stream) {
+    return dropout_launch(DropoutMask::kRead, x, out, const_cast<uint32_t*>(mask), n, 0, p, seed, dtype, stream);
+}
+
+}  // namespace thn

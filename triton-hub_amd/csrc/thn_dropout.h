@@ -16,7 +16,8 @@
 //    [-T, T - 1] exactly if uint32(v + T) < 2 T;
 //  * a dropped element is selected before it is scaled (0 scales to +0), which leaves no branch.
 // Issue costs measured for one wave (cycles): v_mad_u64_u32 / v_mul_hi_u32 4.2, v_bitop3_b32 and v_xor_b32 2.5, v_cmp_u32 4.2,
-// v_mul_f64 and the float64 conversions 4.2-4.5.  bfloat16 16384 x 4096, one launch (134 MB in, 134 MB out): 113 -> 86.5 us.
+// v_mul_f64 and the float64 conversions 4.2-4.5.  bfloat16 16384 x 4096 (134 MB in, 134 MB out),
+// launches of one direction after another: 123 -> 92 us.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -36,6 +37,7 @@ struct DropoutArgs {
     float p;
     uint32_t key_lo, key_hi;
     uint32_t threshold;    // dropout_threshold(p)
+    uint32_t* mask;        // dropout_masked_kernel: see there
 };
 
 constexpr float kDropoutScale = 4.6566127342e-10f;
@@ -129,7 +131,29 @@ __device__ __forceinline__ float keep_div(float x, const KeepDivisor& d) {
 __device__ __forceinline__ double keep_div(double x, const KeepDivisor& d) { return x / d.keep64; }
 
 constexpr int kDropoutBlock = 256;
+constexpr int kMaskedVecs = 4;                   // vectors per thread and step of dropout_masked_kernel
+constexpr int64_t kMaskedMost = int64_t{1} << 31;  // vectors at most
 constexpr uint32_t kDropAll = 0x80000000u;      // the threshold at which no element is kept (2 T does not fit a word there)
+
+// What a step of the kernels does with one element: the value it stores, `dropped` being the decision.  The float32 value is
+// selected before it is widened (the asm keeps the compiler from selecting both halves of the float64 instead).
+__device__ __forceinline__ float dropout_value(float x, bool dropped, const KeepDivisor& keep) {
+    float kept = dropped ? 0.0f : x;
+    asm("" : "+v"(kept));
+    return keep_div(kept, keep);
+}
+__device__ __forceinline__ double dropout_value(double x, bool dropped, const KeepDivisor& keep) { return keep_div(dropped ? 0.0 : x, keep); }
+
+// the tail that does not fill a vector
+template <typename T, bool kWide>
+__device__ __forceinline__ void dropout_tail(const DropoutArgs& a, const KeepDivisor& keep, bool all) {
+    using C = typename std::conditional<T::kBytes == 8, double, float>::type;
+    const int64_t i = a.total_vecs * T::VEC + threadIdx.x;
+    if (blockIdx.x == 0 && i < a.total_elems) {
+        const C x = load_elem<T, C>(a.x, i);
+        store_elem<T, C>(a.out, i, all || is_dropped<kWide>(a.first_offset + i, a) ? C(0) : keep_div(x, keep));
+    }
+}
 
 template <typename T, bool kWide>
 __global__ void __launch_bounds__(kDropoutBlock) dropout_flat_kernel(const DropoutArgs a) {
@@ -148,17 +172,77 @@ __global__ void __launch_bounds__(kDropoutBlock) dropout_flat_kernel(const Dropo
         unpack_as<T>(raw, xf);
         const int64_t e0 = a.first_offset + v * VEC;
 #pragma unroll
-        for (int e = 0; e < VEC; ++e) of[e] = keep_div(is_dropped<kWide>(e0 + e, a) ? C(0) : xf[e], keep);
+        for (int e = 0; e < VEC; ++e) of[e] = dropout_value(xf[e], is_dropped<kWide>(e0 + e, a), keep);
         st128u(a.out + v * 16, pack_as<T, C>(of));
     }
-    // the tail that does not fill a vector
-    const int64_t i = a.total_vecs * VEC + threadIdx.x;
-    if (blockIdx.x == 0 && i < a.total_elems) {
-        const C x = load_elem<T, C>(a.x, i);
-        store_elem<T, C>(a.out, i, all || is_dropped<kWide>(a.first_offset + i, a) ? C(0) : keep_div(x, keep));
-    }
+    dropout_tail<T, kWide>(a, keep, all);
 }
 
-int launch_dropout(int dtype, const DropoutArgs& a, int grid, hipStream_t st);
+// A forward that keeps its decisions (kRead = false) and the backward that reads them instead of drawing them again.  A
+// workgroup takes pieces of 256 x 4 vectors, thread t of it vectors t, t + 256, t + 512 and t + 768 of a piece; word t of the
+// piece's 256 words of mask holds their decisions, a byte per vector with the first in the highest byte, the first element of a
+// vector in the highest of the byte's VEC low bits.  (One byte per thread and vector cost the forward 14 us.)  The next
+// piece is requested before the present one is used, as in act_flat_kernel; slots past the end repeat the last vector, so
+// that no branch stands around a load or a store.  The threshold is below kDropAll (p < 1 in float32) and
+// the vectors have 32-bit numbers.
+// bfloat16 16384 x 4096: forward 95 us (92 without a mask: two instructions per element and 8 MiB more), backward 46, which is
+// what two plain streams take (80 drawn again); both directions of a pass 174 -> 136.
+template <typename T, bool kWide, bool kRead>
+__global__ void __launch_bounds__(kDropoutBlock) dropout_masked_kernel(const DropoutArgs a) {
+    using C = typename std::conditional<T::kBytes == 8, double, float>::type;
+    constexpr int VEC = T::VEC, U = kMaskedVecs;
+    const KeepDivisor keep = make_keep_divisor(1.0f - a.p);
+    const uint32_t pieces = static_cast<uint32_t>((a.total_vecs + kDropoutBlock * U - 1) / (kDropoutBlock * U));
+    const uint32_t last = static_cast<uint32_t>(a.total_vecs - 1);
+    const auto place = [&](uint32_t piece, int u) -> uint32_t {
+        const uint32_t v = piece * (kDropoutBlock * U) + u * kDropoutBlock + threadIdx.x;
+        return v < last ? v : last;
+    };
+    const auto load = [&](uint32_t v) { return ld128u(a.x + static_cast<uint64_t>(v) * 16); };
+    if (blockIdx.x < pieces) {
+        u32x4 cur[U], nxt[U];
+        uint32_t word = 0u, next_word = 0u;
+#pragma unroll
+        for (int u = 0; u < U; ++u) cur[u] = load(place(blockIdx.x, u));
+        if constexpr (kRead) word = a.mask[static_cast<uint64_t>(blockIdx.x * kDropoutBlock + threadIdx.x)];
+        drain_vector_memory(cur);
+        for (uint32_t piece = blockIdx.x; piece < pieces; piece += gridDim.x) {
+            const uint32_t next = piece + gridDim.x < pieces ? piece + gridDim.x : piece;
+#pragma unroll
+            for (int u = 0; u < U; ++u) nxt[u] = load(place(next, u));
+            if constexpr (kRead) next_word = a.mask[static_cast<uint64_t>(next * kDropoutBlock + threadIdx.x)];
+            else word = 0u;
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const uint32_t v = place(piece, u);
+                const int64_t e0 = a.first_offset + static_cast<int64_t>(v) * VEC;
+                C xf[VEC], of[VEC];
+                unpack_as<T>(cur[u], xf);
+                if constexpr (!kRead && VEC < 8) word <<= 8 - VEC;
+#pragma unroll
+                for (int e = 0; e < VEC; ++e) {
+                    bool dropped;
+                    if constexpr (kRead) {
+                        dropped = (word >> (8 * (U - 1 - u) + VEC - 1 - e) & 1u) != 0u;
+                    } else {
+                        dropped = is_dropped<kWide>(e0 + e, a);
+                        word = word << 1 | (dropped ? 1u : 0u);
+                    }
+                    of[e] = dropout_value(xf[e], dropped, keep);
+                }
+                st128u(a.out + static_cast<uint64_t>(v) * 16, pack_as<T, C>(of));
+            }
+            if constexpr (!kRead) a.mask[static_cast<uint64_t>(piece * kDropoutBlock + threadIdx.x)] = word;
+#pragma unroll
+            for (int u = 0; u < U; ++u) cur[u] = nxt[u];
+            word = next_word;
+        }
+    }
+    dropout_tail<T, kWide>(a, keep, false);
+}
+
+enum class DropoutMask { kNone, kWrite, kRead };
+
+int launch_dropout(int dtype, DropoutMask mode, const DropoutArgs& a, int grid, hipStream_t st);
 
 }  // namespace thn

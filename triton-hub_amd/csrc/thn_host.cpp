@@ -19,6 +19,7 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include "thn_dropout_mask.h"
 #include "thnorm.h"
 
 namespace {
@@ -256,9 +257,68 @@ PyObject* act_bwd(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     END_HANDLE_TH_ERRORS
 }
 
+// From this many elements on a dropout that will be differentiated keeps its decisions (one byte per 16 bytes of input, in 32-bit words) instead of
+// drawing them again in the backward.  Below it the kernels take less time than the host needs for the extra tensor.  (The masked kernels number up to 2^31 vectors.)
+constexpr int64_t kMaskFrom = int64_t{1} << 22, kMaskTo = int64_t{1} << 32;
+
+// dropout_fwd(x, p, seed, backward_follows) -> (out, mask or None), for 0 < p < 1 (in float32, as the kernels compare)
+PyObject* dropout_fwd(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+    HANDLE_TH_ERRORS
+    if (wrong_count(nargs, 4)) return nullptr;
+    const at::Tensor* x = plain(args[0]);
+    double p;
+    long long seed;
+    if (x == nullptr || !number(args[1], &p) || !(p > 0.0 && static_cast<float>(p) < 1.0f) || !whole(args[2], &seed)) Py_RETURN_NONE;
+    const int64_t n = x->numel();
+    const bool keep = PyObject_IsTrue(args[3]) == 1 && n >= kMaskFrom && n < kMaskTo;
+    at::Tensor results[2] = {at::empty_like(*x), keep ? at::empty({thn::dropout_mask_words(n, static_cast<int>(x->element_size()))}, x->options().dtype(at::kInt)) : at::Tensor()};
+    void *xp = x->data_ptr(), *yp = results[0].data_ptr(), *stream = stream_of(*x);
+    uint32_t* mask = keep ? reinterpret_cast<uint32_t*>(results[1].data_ptr<int32_t>()) : nullptr;
+    const int code = type_code(*x);
+    const int status = unlocked([&] {
+        if (keep) return thn::dropout_keep_mask(xp, yp, mask, n, static_cast<float>(p), static_cast<uint64_t>(seed), code, stream);
+        return thn_dropout(xp, yp, n, 0, static_cast<float>(p), static_cast<uint64_t>(seed), code, stream);
+    });
+    if (status != THN_OK) return failed(status);
+    return as_tuple(results);
+    END_HANDLE_TH_ERRORS
+}
+
+// dropout_bwd(dout, p, seed, mask or None) -> dx; a mask of another size belongs to another type of storage
+PyObject* dropout_bwd(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+    HANDLE_TH_ERRORS
+    if (wrong_count(nargs, 4)) return nullptr;
+    const at::Tensor* g = plain(args[0]);
+    double p;
+    long long seed;
+    if (g == nullptr || !number(args[1], &p) || !(p > 0.0 && static_cast<float>(p) < 1.0f) || !whole(args[2], &seed)) Py_RETURN_NONE;
+    const int64_t n = g->numel();
+    const uint32_t* mask = nullptr;
+    if (args[3] != Py_None) {
+        if (!THPVariable_CheckExact(args[3])) Py_RETURN_NONE;
+        const at::Tensor& t = THPVariable_Unpack(args[3]);
+        if (!t.defined() || t.device() != g->device() || t.scalar_type() != at::kInt || !t.is_contiguous() ||
+            t.numel() != thn::dropout_mask_words(n, static_cast<int>(g->element_size()))) {
+            Py_RETURN_NONE;
+        }
+        mask = reinterpret_cast<const uint32_t*>(t.data_ptr<int32_t>());
+    }
+    const at::Tensor dx = at::empty_like(*g);
+    void *gp = g->data_ptr(), *dxp = dx.data_ptr(), *stream = stream_of(*g);
+    const int code = type_code(*g);
+    const int status = unlocked([&] {
+        if (mask != nullptr) return thn::dropout_from_mask(gp, dxp, mask, n, static_cast<float>(p), static_cast<uint64_t>(seed), code, stream);
+        return thn_dropout(gp, dxp, n, 0, static_cast<float>(p), static_cast<uint64_t>(seed), code, stream);
+    });
+    if (status != THN_OK) return failed(status);
+    return THPVariable_Wrap(dx);
+    END_HANDLE_TH_ERRORS
+}
+
 #define THN_METHOD(NAME) {#NAME, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(NAME)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {THN_METHOD(norm_fwd),    THN_METHOD(norm_bwd), THN_METHOD(softmax_fwd), THN_METHOD(softmax_bwd),
-                         THN_METHOD(act_fwd),     THN_METHOD(act_bwd),  {nullptr, nullptr, 0, nullptr}};
+                         THN_METHOD(act_fwd),     THN_METHOD(act_bwd),
+                         THN_METHOD(dropout_fwd), THN_METHOD(dropout_bwd), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", "Host side of the operator calls in native code.", -1, methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace
