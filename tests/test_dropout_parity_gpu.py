@@ -233,7 +233,7 @@ def test_random_sizes_offsets_seeds_and_alignments():
 def test_kept_decisions_give_the_bits_of_drawn_ones(n, dtype):
     """From 2^22 elements on the backward reads the decisions that the forward kept: both directions against thn_dropout
     with the same seed, for whole vectors and tails, every p that keeps something, gradients off the 16-byte path, a
-    strided gradient (drawn again) and a second backward through the same graph."""
+    strided gradient (drawn again) and further backwards through the same graph, which saves no tensor and so is not freed."""
     g = torch.Generator(device="cuda").manual_seed(n)
     x, dy = (torch.randn(n, device="cuda", generator=g, dtype=torch.float32).to(dtype) for _ in range(2))
     x[3], x[8], dy[5], dy[7] = float("inf"), float("nan"), float("-inf"), float("nan")
@@ -251,14 +251,30 @@ def test_kept_decisions_give_the_bits_of_drawn_ones(n, dtype):
         random.seed(n)
         module, xg = Dropout(p), x.clone().requires_grad_(True)
         y = module(xg)
-        assert len(y.grad_fn.saved_tensors) == (1 if n >= 1 << 22 else 0)
+        assert (y.grad_fn.mask is not None) == (n >= 1 << 22)
         want = drawn(dy, p, seed)
         assert same(y.detach(), drawn(x, p, seed))
-        assert same(torch.autograd.grad(y, xg, dy, retain_graph=True)[0], want)
+        assert same(torch.autograd.grad(y, xg, dy)[0], want)
         off = torch.empty(n + 1, dtype=dtype, device="cuda")[1:].copy_(dy)
-        assert same(torch.autograd.grad(y, xg, off, retain_graph=True)[0], want)
+        assert same(torch.autograd.grad(y, xg, off)[0], want)
         wide = torch.empty(n, 2, dtype=dtype, device="cuda")[:, 0].copy_(dy)
         assert same(torch.autograd.grad(y, xg, wide)[0], want)
         random.seed(n)
         with torch.no_grad():
             assert same(module(x), drawn(x, p, seed))
+
+
+@pytest.mark.parametrize("n", [(1 << 22) - 8, 1 << 22])
+def test_backward_under_a_checkpoint_keeps_the_decisions_of_its_output(n):
+    """A checkpoint runs the forward a second time, which draws another seed from Python's random numbers: the gradient is
+    that of the output the caller has, as it is when the mask is drawn from the seed."""
+    from torch.utils.checkpoint import checkpoint
+    x = torch.ones(n, device="cuda", requires_grad=True)
+    double = lambda t: Dropout(0.5)(t) * x           # the product saves a tensor, so the checkpoint does run again
+    y = checkpoint(double, x, use_reentrant=False)
+    kept = y.detach() != 0
+    inner = y.grad_fn.next_functions[0][0]
+    seen = []
+    inner.register_hook(lambda gin, gout: seen.append(gin[0]))
+    y.backward(torch.ones_like(y))
+    assert len(seen) == 1 and torch.equal(seen[0] != 0, kept)

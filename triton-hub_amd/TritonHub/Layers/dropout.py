@@ -37,8 +37,10 @@ def _dropout_apply(t: torch.Tensor, p, seed, training, what: str) -> torch.Tenso
 
 class dropout(torch.autograd.Function):
     """forward(ctx, input, p, training) -> output; keeps (p, seed, training) on ctx.  A large input that requires a gradient
-    also saves which elements were dropped (one byte per 16 bytes of input), and the backward reads them; every other
-    backward regenerates the mask from the seed.  The two give the same bits."""
+    also keeps there which elements were dropped (``mask``, one byte per 16 bytes of input), and the backward reads them;
+    every other backward regenerates the mask from the seed.  The two give the same bits.  The mask is no saved tensor, as
+    the seed is none: a graph can be walked again without retain_graph, and a checkpoint that runs the forward once more,
+    with another seed, leaves the backward the decisions of the output it belongs to."""
 
     @staticmethod
     def forward(ctx, input, p, training):
@@ -46,19 +48,17 @@ class dropout(torch.autograd.Function):
         ctx.p = p
         ctx.seed = seed
         ctx.training = training
+        ctx.mask = None
         done = _native.host().dropout_fwd(input, p, seed, ctx.needs_input_grad[0]) if training else None
         if done is None:
             return _dropout_apply(input, p, seed, training, 'input')
-        output, mask = done
-        if mask is not None:
-            ctx.save_for_backward(mask)
+        output, ctx.mask = done
         return output
 
     @staticmethod
     def backward(ctx, d_out):
         if ctx.training:
-            saved = ctx.saved_tensors
-            grad = _native.host().dropout_bwd(d_out, ctx.p, ctx.seed, saved[0] if saved else None)
+            grad = _native.host().dropout_bwd(d_out, ctx.p, ctx.seed, ctx.mask)
             if grad is not None:
                 return grad, None, None
         grad = _dropout_apply(d_out, ctx.p, ctx.seed, ctx.training, 'gradient')
