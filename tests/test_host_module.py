@@ -1,10 +1,14 @@
 """The native host module (TritonHub/_host.so) against the Python wrappers' general way: the same bits for every form of call
 that it takes, and None for what it leaves to them."""
+import types
+
 import pytest
 import torch
 
 from TritonHub import _native
 from TritonHub.Activations import _launch as act_launch
+from TritonHub.Layers import Dropout
+from TritonHub.Layers import dropout as dropout_layer
 from TritonHub.Normalization import _launch as norm_launch
 
 
@@ -25,6 +29,44 @@ def test_host_tensors_and_wrong_argument_counts():
     for name, count in (("norm_fwd", 7), ("norm_bwd", 10), ("softmax_fwd", 2), ("softmax_bwd", 3), ("act_fwd", 4), ("act_bwd", 5)):
         with pytest.raises(TypeError):
             getattr(host, name)(*[x] * (count - 1))
+
+
+@pytest.fixture
+def dropout_calls(monkeypatch):
+    """Dropout over a host module that only notes what it is asked for, for tensors of four elements and more; the "mask" is
+    the tensor 7."""
+    calls = types.SimpleNamespace(keep=[], masks=[], gradients=[])
+
+    class Host:
+        def dropout_fwd(self, x, p, seed, keep):
+            calls.keep.append(keep)
+            return x.clone(), torch.tensor(7) if keep else None
+
+        def dropout_bwd(self, g, p, seed, mask):
+            calls.masks.append(mask)
+            calls.gradients.append(g)
+            return g.clone()
+
+    monkeypatch.setattr(_native, "host", lambda: Host())
+    monkeypatch.setattr(dropout_layer, "KEEP_FROM", 4)
+    return calls
+
+
+def test_dropout_keeps_decisions_only_for_a_backward(dropout_calls):
+    """Not under no_grad or in inference mode, nor in the first forward of a reentrant checkpoint, whatever the input says."""
+    from torch.utils.checkpoint import checkpoint
+    module, x = Dropout(0.5), torch.ones(4, requires_grad=True)
+    with torch.no_grad():
+        assert module(x).grad_fn is None
+    with torch.inference_mode():
+        module(x)
+    module(x.detach())
+    module(x[:3])
+    assert dropout_calls.keep == [False] * 4
+    assert module(x).grad_fn.mask is not None and module(x * 2).grad_fn.mask is not None
+    assert dropout_calls.keep[4:] == [True, True]
+    checkpoint(lambda t: module(t) * t, x, use_reentrant=True).sum().backward()
+    assert dropout_calls.keep[6:] == [False, True] and len(dropout_calls.masks) == 1 and dropout_calls.masks[0] is not None
 
 
 def _same(a, b):

@@ -35,9 +35,14 @@ def _dropout_apply(t: torch.Tensor, p, seed, training, what: str) -> torch.Tenso
     return out.reshape(t.shape)
 
 
+# From this many elements on a dropout that will be differentiated keeps its decisions instead of drawing them again in the
+# backward.  Below it the kernels take less time than the host needs for the extra tensor.
+KEEP_FROM = 1 << 22
+
+
 class dropout(torch.autograd.Function):
-    """forward(ctx, input, p, training) -> output; keeps (p, seed, training) on ctx.  A large input that requires a gradient
-    also keeps there which elements were dropped (``mask``, one byte per 16 bytes of input), and the backward reads them;
+    """forward(ctx, input, p, training) -> output; keeps (p, seed, training) on ctx.  The forward of a large input also
+    keeps there which elements were dropped (``mask``, one byte per 16 bytes of input) if a backward can follow, which reads them;
     every other backward regenerates the mask from the seed.  The two give the same bits.  The mask is no saved tensor, as
     the seed is none: a graph can be walked again without retain_graph, and a checkpoint that runs the forward once more,
     with another seed, leaves the backward the decisions of the output it belongs to."""
@@ -49,7 +54,10 @@ class dropout(torch.autograd.Function):
         ctx.seed = seed
         ctx.training = training
         ctx.mask = None
-        done = _native.host().dropout_fwd(input, p, seed, ctx.needs_input_grad[0]) if training else None
+        # needs_input_grad says that the input requires a gradient, also where gradients are off (no_grad, inference mode, the
+        # first forward of a reentrant checkpoint): only a node with somewhere to pass a gradient on to has a backward
+        keep = ctx.needs_input_grad[0] and input.numel() >= KEEP_FROM and len(ctx.next_functions) > 0
+        done = _native.host().dropout_fwd(input, p, seed, keep) if training else None
         if done is None:
             return _dropout_apply(input, p, seed, training, 'input')
         output, ctx.mask = done

@@ -257,11 +257,10 @@ PyObject* act_bwd(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     END_HANDLE_TH_ERRORS
 }
 
-// From this many elements on a dropout that will be differentiated keeps its decisions (one byte per 16 bytes of input, in 32-bit words) instead of
-// drawing them again in the backward.  Below it the kernels take less time than the host needs for the extra tensor.  (The masked kernels number up to 2^31 vectors.)
-constexpr int64_t kMaskFrom = int64_t{1} << 22, kMaskTo = int64_t{1} << 32;
+constexpr int64_t kMaskTo = int64_t{1} << 32;        // the masked kernels number up to 2^31 vectors
 
-// dropout_fwd(x, p, seed, backward_follows) -> (out, mask or None), for 0 < p < 1 (in float32, as the kernels compare)
+// dropout_fwd(x, p, seed, keep) -> (out, mask or None), for 0 < p < 1 (in float32, as the kernels compare); keep: the decisions
+// are wanted for a backward (one byte per 16 bytes of input, in 32-bit words)
 PyObject* dropout_fwd(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     HANDLE_TH_ERRORS
     if (wrong_count(nargs, 4)) return nullptr;
@@ -270,7 +269,7 @@ PyObject* dropout_fwd(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     long long seed;
     if (x == nullptr || !number(args[1], &p) || !(p > 0.0 && static_cast<float>(p) < 1.0f) || !whole(args[2], &seed)) Py_RETURN_NONE;
     const int64_t n = x->numel();
-    const bool keep = PyObject_IsTrue(args[3]) == 1 && n >= kMaskFrom && n < kMaskTo;
+    const bool keep = PyObject_IsTrue(args[3]) == 1 && n < kMaskTo;
     at::Tensor results[2] = {at::empty_like(*x), keep ? at::empty({thn::dropout_mask_words(n, static_cast<int>(x->element_size()))}, x->options().dtype(at::kInt)) : at::Tensor()};
     void *xp = x->data_ptr(), *yp = results[0].data_ptr(), *stream = stream_of(*x);
     uint32_t* mask = keep ? reinterpret_cast<uint32_t*>(results[1].data_ptr<int32_t>()) : nullptr;
