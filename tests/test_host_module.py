@@ -69,6 +69,17 @@ def test_dropout_keeps_decisions_only_for_a_backward(dropout_calls):
     assert dropout_calls.keep[6:] == [False, True] and len(dropout_calls.masks) == 1 and dropout_calls.masks[0] is not None
 
 
+def test_dropout_gives_its_decisions_back(dropout_calls):
+    """The first backward reads them and lets them go, although the graph (here through y) lives on; the second draws."""
+    x = torch.ones(4, requires_grad=True)
+    y = Dropout(0.5)(x)
+    assert y.grad_fn.mask is not None
+    y.backward(torch.ones(4))
+    assert y.grad_fn.mask is None
+    y.backward(torch.ones(4))
+    assert [m is None for m in dropout_calls.masks] == [False, True]
+
+
 def _same(a, b):
     if a is None or b is None:
         return a is None and b is None

@@ -42,8 +42,8 @@ KEEP_FROM = 1 << 22
 
 class dropout(torch.autograd.Function):
     """forward(ctx, input, p, training) -> output; keeps (p, seed, training) on ctx.  The forward of a large input also
-    keeps there which elements were dropped (``mask``, one byte per 16 bytes of input) if a backward can follow, which reads them;
-    every other backward regenerates the mask from the seed.  The two give the same bits.  The mask is no saved tensor, as
+    keeps there which elements were dropped (``mask``, one byte per 16 bytes of input) if a backward can follow, which reads them
+    and gives them back; every other backward, a second one among them, regenerates the mask from the seed.  The two give the same bits.  The mask is no saved tensor, as
     the seed is none: a graph can be walked again without retain_graph, and a checkpoint that runs the forward once more,
     with another seed, leaves the backward the decisions of the output it belongs to."""
 
@@ -66,7 +66,8 @@ class dropout(torch.autograd.Function):
     @staticmethod
     def backward(ctx, d_out):
         if ctx.training:
-            grad = _native.host().dropout_bwd(d_out, ctx.p, ctx.seed, ctx.mask)
+            mask, ctx.mask = ctx.mask, None          # given back as saved tensors are; another backward draws the same bits
+            grad = _native.host().dropout_bwd(d_out, ctx.p, ctx.seed, mask)
             if grad is not None:
                 return grad, None, None
         grad = _dropout_apply(d_out, ctx.p, ctx.seed, ctx.training, 'gradient')
