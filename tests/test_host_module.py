@@ -80,6 +80,15 @@ def test_dropout_gives_its_decisions_back(dropout_calls):
     assert [m is None for m in dropout_calls.masks] == [False, True]
 
 
+def test_dropout_reads_its_decisions_for_any_gradient(dropout_calls):
+    """The expanded gradient of a sum and a strided one meet the mask as a contiguous copy; without a mask they are passed on."""
+    for backward in (lambda y: y.sum().backward(), lambda y: y.backward(torch.ones(4, 2)[:, 0])):
+        backward(Dropout(0.5)(torch.ones(4, requires_grad=True)))
+        assert dropout_calls.masks[-1] is not None and dropout_calls.gradients[-1].is_contiguous()
+    Dropout(0.5)(torch.ones(3, requires_grad=True)).sum().backward()
+    assert dropout_calls.masks[-1] is None and not dropout_calls.gradients[-1].is_contiguous()
+
+
 def _same(a, b):
     if a is None or b is None:
         return a is None and b is None

@@ -67,6 +67,8 @@ class dropout(torch.autograd.Function):
     def backward(ctx, d_out):
         if ctx.training:
             mask, ctx.mask = ctx.mask, None          # given back as saved tensors are; another backward draws the same bits
+            if mask is not None:
+                d_out = d_out.contiguous()           # an expanded gradient, say (the general way copies it too)
             grad = _native.host().dropout_bwd(d_out, ctx.p, ctx.seed, mask)
             if grad is not None:
                 return grad, None, None
