@@ -278,3 +278,34 @@ def test_backward_under_a_checkpoint_keeps_the_decisions_of_its_output(n):
     inner.register_hook(lambda gin, gout: seen.append(gin[0]))
     y.backward(torch.ones_like(y))
     assert len(seen) == 1 and torch.equal(seen[0] != 0, kept)
+
+
+def test_captured_backward_of_an_eager_forward():
+    """The backward alone in a graph, replayed after the forward's node has died and its memory has been written over: the
+    bits of the eager backward every time.  Both directions in a graph too."""
+    n, side = 1 << 22, torch.cuda.Stream()
+    x, dy = (torch.randn(n, device="cuda") for _ in range(2))
+    module = Dropout(0.5)
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        xg = x.clone().requires_grad_(True)
+
+        def forward():
+            random.seed(7)
+            return module(xg)
+
+        want = torch.autograd.grad(forward(), xg, dy)[0]
+        for both in (False, True):
+            y, graph = None if both else forward(), torch.cuda.CUDAGraph()
+            side.synchronize()
+            with torch.cuda.graph(graph, stream=side):
+                y = forward() if both else y
+                got = torch.autograd.grad(y, xg, dy)[0]
+            del y
+            for trial in range(3):
+                over = [torch.full((n // 16,), trial - 1, dtype=torch.int32, device="cuda") for _ in range(8)]
+                got.zero_()
+                graph.replay()
+                side.synchronize()
+                assert same_bits(got.cpu(), want.cpu()), f"both={both} replay {trial}"
+                del over

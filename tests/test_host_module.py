@@ -35,7 +35,7 @@ def test_host_tensors_and_wrong_argument_counts():
 def dropout_calls(monkeypatch):
     """Dropout over a host module that only notes what it is asked for, for tensors of four elements and more; the "mask" is
     the tensor 7."""
-    calls = types.SimpleNamespace(keep=[], masks=[], gradients=[])
+    calls = types.SimpleNamespace(keep=[], masks=[], gradients=[], capturing=False)
 
     class Host:
         def dropout_fwd(self, x, p, seed, keep):
@@ -49,6 +49,7 @@ def dropout_calls(monkeypatch):
 
     monkeypatch.setattr(_native, "host", lambda: Host())
     monkeypatch.setattr(dropout_layer, "KEEP_FROM", 4)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: calls.capturing)
     return calls
 
 
@@ -87,6 +88,18 @@ def test_dropout_reads_its_decisions_for_any_gradient(dropout_calls):
         assert dropout_calls.masks[-1] is not None and dropout_calls.gradients[-1].is_contiguous()
     Dropout(0.5)(torch.ones(3, requires_grad=True)).sum().backward()
     assert dropout_calls.masks[-1] is None and not dropout_calls.gradients[-1].is_contiguous()
+
+
+@pytest.mark.parametrize("forward_captured", [False, True])
+@pytest.mark.parametrize("backward_captured", [False, True])
+def test_dropout_decisions_do_not_cross_the_border_of_a_graph(dropout_calls, forward_captured, backward_captured):
+    """A backward captured after an eager forward draws: the decisions of that forward are gone when the graph is replayed.
+    Captured both, they live in the graph's memory."""
+    dropout_calls.capturing = forward_captured
+    y = Dropout(0.5)(torch.ones(4, requires_grad=True))
+    dropout_calls.capturing = backward_captured
+    y.backward(torch.ones(4))
+    assert (dropout_calls.masks[-1] is not None) == (forward_captured == backward_captured)
 
 
 def _same(a, b):

@@ -61,12 +61,16 @@ class dropout(torch.autograd.Function):
         if done is None:
             return _dropout_apply(input, p, seed, training, 'input')
         output, ctx.mask = done
+        if keep:
+            ctx.captured = torch.cuda.is_current_stream_capturing()
         return output
 
     @staticmethod
     def backward(ctx, d_out):
         if ctx.training:
             mask, ctx.mask = ctx.mask, None          # given back as saved tensors are; another backward draws the same bits
+            if mask is not None and ctx.captured != torch.cuda.is_current_stream_capturing():
+                mask = None          # a captured backward would read it on every replay, long after it has been freed
             if mask is not None:
                 d_out = d_out.contiguous()           # an expanded gradient, say (the general way copies it too)
             grad = _native.host().dropout_bwd(d_out, ctx.p, ctx.seed, mask)
