@@ -309,3 +309,22 @@ def test_captured_backward_of_an_eager_forward():
                 side.synchronize()
                 assert same_bits(got.cpu(), want.cpu()), f"both={both} replay {trial}"
                 del over
+
+
+def test_nothing_kept_where_saved_tensors_are_managed():
+    """Under saved-tensor hooks (offloading, a non-reentrant checkpoint) a program decides what stays on the device: a mask that
+    the hooks do not see is not made, and the backward draws the same bits."""
+    from torch.utils.checkpoint import checkpoint
+    n, module = 1 << 22, Dropout(0.5)
+    x = torch.randn(n, device="cuda", requires_grad=True)
+    dy = torch.randn(n, device="cuda")
+    random.seed(3)
+    kept = module(x)
+    want = torch.autograd.grad(kept, x, dy)[0]
+    random.seed(3)
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t.cpu(), lambda t: t.cuda()):
+        y = module(x)
+    assert y.grad_fn.mask is None and same_bits(y.detach().cpu(), kept.detach().cpu())
+    assert same_bits(torch.autograd.grad(y, x, dy)[0].cpu(), want.cpu())
+    assert checkpoint(module, x, use_reentrant=False).grad_fn.mask is None
+    assert module(x).grad_fn.mask is not None

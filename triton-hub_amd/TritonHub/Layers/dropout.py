@@ -41,11 +41,11 @@ KEEP_FROM = 1 << 22
 
 
 class dropout(torch.autograd.Function):
-    """forward(ctx, input, p, training) -> output; keeps (p, seed, training) on ctx.  The forward of a large input also
-    keeps there which elements were dropped (``mask``, one byte per 16 bytes of input) if a backward can follow, which reads them
-    and gives them back; every other backward, a second one among them, regenerates the mask from the seed.  The two give the same bits.  The mask is no saved tensor, as
-    the seed is none: a graph can be walked again without retain_graph, and a checkpoint that runs the forward once more,
-    with another seed, leaves the backward the decisions of the output it belongs to."""
+    """forward(ctx, input, p, training) -> output; keeps (p, seed, training) on ctx.  The forward of a large input also keeps
+    there which elements were dropped (``mask``, one byte per 16 bytes of input) if a backward can follow, which reads them and
+    gives them back; every other backward, a second one among them, regenerates the mask from the seed.  The two give the
+    same bits.  The mask is no saved tensor, as the seed is none, so a graph can be walked again without retain_graph; under
+    saved-tensor hooks, which would not see it, and so in a non-reentrant checkpoint, none is kept."""
 
     @staticmethod
     def forward(ctx, input, p, training):

@@ -14,6 +14,7 @@
 #include <Python.h>
 
 #include <ATen/ATen.h>
+#include <ATen/SavedTensorHooks.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
@@ -260,7 +261,8 @@ PyObject* act_bwd(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
 constexpr int64_t kMaskTo = int64_t{1} << 32;        // the masked kernels number up to 2^31 vectors
 
 // dropout_fwd(x, p, seed, keep) -> (out, mask or None), for 0 < p < 1 (in float32, as the kernels compare); keep: the decisions
-// are wanted for a backward (one byte per 16 bytes of input, in 32-bit words)
+// are wanted for a backward (one byte per 16 bytes of input, in 32-bit words).  Under saved-tensor hooks (offloading, a
+// non-reentrant checkpoint) none are kept: the hooks would not see the mask, and it would stay where they are to free memory.
 PyObject* dropout_fwd(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     HANDLE_TH_ERRORS
     if (wrong_count(nargs, 4)) return nullptr;
@@ -269,7 +271,7 @@ PyObject* dropout_fwd(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     long long seed;
     if (x == nullptr || !number(args[1], &p) || !(p > 0.0 && static_cast<float>(p) < 1.0f) || !whole(args[2], &seed)) Py_RETURN_NONE;
     const int64_t n = x->numel();
-    const bool keep = PyObject_IsTrue(args[3]) == 1 && n < kMaskTo;
+    const bool keep = PyObject_IsTrue(args[3]) == 1 && n < kMaskTo && at::SavedTensorDefaultHooks::get_tls_state().stack.empty();
     at::Tensor results[2] = {at::empty_like(*x), keep ? at::empty({thn::dropout_mask_words(n, static_cast<int>(x->element_size()))}, x->options().dtype(at::kInt)) : at::Tensor()};
     void *xp = x->data_ptr(), *yp = results[0].data_ptr(), *stream = stream_of(*x);
     uint32_t* mask = keep ? reinterpret_cast<uint32_t*>(results[1].data_ptr<int32_t>()) : nullptr;
