@@ -153,3 +153,16 @@ def test_same_bits_as_the_general_way(shape, dtype, monkeypatch):
     assert host.softmax_bwd(x, dy.reshape(-1, 1), 0) is None or n == 1
     with pytest.raises(RuntimeError, match="libthnorm"):
         host.softmax_fwd(x, 9)
+
+
+@pytest.mark.gpu
+def test_dropout_results_have_contiguous_strides(monkeypatch):
+    """Also where a dimension of one element of the input or the gradient has a stride of its own, as the general way does."""
+    def strides():
+        x, dy = (torch.randn(2, 1, 3, 8, device="cuda").as_strided((2, 1, 3, 8), (24, 7, 8, 1)) for _ in range(2))
+        y = Dropout(0.5)(x.requires_grad_(True))
+        return y.stride(), torch.autograd.grad(y, x, dy)[0].stride()
+
+    here = strides()
+    monkeypatch.setattr(_native, "host", lambda: _General())
+    assert here == strides() == ((24, 24, 8, 1),) * 2

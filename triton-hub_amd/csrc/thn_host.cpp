@@ -272,7 +272,9 @@ PyObject* dropout_fwd(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     if (x == nullptr || !number(args[1], &p) || !(p > 0.0 && static_cast<float>(p) < 1.0f) || !whole(args[2], &seed)) Py_RETURN_NONE;
     const int64_t n = x->numel();
     const bool keep = PyObject_IsTrue(args[3]) == 1 && n < kMaskTo && at::SavedTensorDefaultHooks::get_tls_state().stack.empty();
-    at::Tensor results[2] = {at::empty_like(*x), keep ? at::empty({thn::dropout_mask_words(n, static_cast<int>(x->element_size()))}, x->options().dtype(at::kInt)) : at::Tensor()};
+    // (contiguous strides also for dimensions of one element, whose strides empty_like would take over from x)
+    at::Tensor results[2] = {at::empty_like(*x, at::MemoryFormat::Contiguous),
+                             keep ? at::empty({thn::dropout_mask_words(n, static_cast<int>(x->element_size()))}, x->options().dtype(at::kInt)) : at::Tensor()};
     void *xp = x->data_ptr(), *yp = results[0].data_ptr(), *stream = stream_of(*x);
     uint32_t* mask = keep ? reinterpret_cast<uint32_t*>(results[1].data_ptr<int32_t>()) : nullptr;
     const int code = type_code(*x);
@@ -304,7 +306,7 @@ PyObject* dropout_bwd(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         }
         mask = reinterpret_cast<const uint32_t*>(t.data_ptr<int32_t>());
     }
-    const at::Tensor dx = at::empty_like(*g);
+    const at::Tensor dx = at::empty_like(*g, at::MemoryFormat::Contiguous);
     void *gp = g->data_ptr(), *dxp = dx.data_ptr(), *stream = stream_of(*g);
     const int code = type_code(*g);
     const int status = unlocked([&] {
