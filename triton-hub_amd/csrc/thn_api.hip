@@ -1724,7 +1724,7 @@ int dropout_launch(thn::DropoutMask mode, const void* x, void* out, uint32_t* ma
     a.key_hi = static_cast<uint32_t>(seed >> 32);
     a.threshold = thn::dropout_threshold(p);
     a.mask = mask;
-    if (mode != thn::DropoutMask::kNone && (a.threshold == thn::kDropAll || a.total_vecs > thn::kMaskedMost)) return THN_E_SHAPE;
+    if (mode != thn::DropoutMask::kNone && (a.threshold == thn::kDropAll || first_offset != 0 || n > thn::kMaskedMost)) return THN_E_SHAPE;
     // Bound by integer arithmetic: as many waves as a compute unit holds (8 workgroups of 256 threads).  From a mask, by
     // memory: 4 workgroups, as the element-wise kernels.
     const int64_t per_block = static_cast<int64_t>(thn::kDropoutBlock) * (mode == thn::DropoutMask::kNone ? 1 : thn::kMaskedVecs);

@@ -132,7 +132,7 @@ __device__ __forceinline__ double keep_div(double x, const KeepDivisor& d) { ret
 
 constexpr int kDropoutBlock = 256;
 constexpr int kMaskedVecs = 4;                   // vectors per thread and step of dropout_masked_kernel
-constexpr int64_t kMaskedMost = int64_t{1} << 31;  // vectors at most
+constexpr int64_t kMaskedMost = int64_t{1} << 32;  // elements at most
 constexpr uint32_t kDropAll = 0x80000000u;      // the threshold at which no element is kept (2 T does not fit a word there)
 
 // What a step of the kernels does with one element: the value it stores, `dropped` being the decision.  The float32 value is
@@ -183,11 +183,11 @@ __global__ void __launch_bounds__(kDropoutBlock) dropout_flat_kernel(const Dropo
 // piece's 256 words of mask holds their decisions, a byte per vector with the first in the highest byte, the first element of a
 // vector in the highest of the byte's VEC low bits.  (One byte per thread and vector cost the forward 14 us.)  The next
 // piece is requested before the present one is used, as in act_flat_kernel; slots past the end repeat the last vector, so
-// that no branch stands around a load or a store.  The threshold is below kDropAll (p < 1 in float32) and
-// the vectors have 32-bit numbers.
+// that no branch stands around a load or a store.  The threshold is below kDropAll (p < 1 in float32), the offsets of the
+// elements start at 0 and fit 32 bits.
 // bfloat16 16384 x 4096: forward 95 us (92 without a mask: two instructions per element and 8 MiB more), backward 46, which is
 // what two plain streams take (80 drawn again); both directions of a pass 174 -> 136.
-template <typename T, bool kWide, bool kRead>
+template <typename T, bool kRead>
 __global__ void __launch_bounds__(kDropoutBlock) dropout_masked_kernel(const DropoutArgs a) {
     using C = typename std::conditional<T::kBytes == 8, double, float>::type;
     constexpr int VEC = T::VEC, U = kMaskedVecs;
@@ -215,7 +215,7 @@ __global__ void __launch_bounds__(kDropoutBlock) dropout_masked_kernel(const Dro
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 const uint32_t v = place(piece, u);
-                const int64_t e0 = a.first_offset + static_cast<int64_t>(v) * VEC;
+                const int64_t e0 = static_cast<int64_t>(v) * VEC;
                 C xf[VEC], of[VEC];
                 unpack_as<T>(cur[u], xf);
                 if constexpr (!kRead && VEC < 8) word <<= 8 - VEC;
@@ -225,7 +225,7 @@ __global__ void __launch_bounds__(kDropoutBlock) dropout_masked_kernel(const Dro
                     if constexpr (kRead) {
                         dropped = (word >> (8 * (U - 1 - u) + VEC - 1 - e) & 1u) != 0u;
                     } else {
-                        dropped = is_dropped<kWide>(e0 + e, a);
+                        dropped = is_dropped<false>(e0 + e, a);
                         word = word << 1 | (dropped ? 1u : 0u);
                     }
                     of[e] = dropout_value(xf[e], dropped, keep);
@@ -238,7 +238,7 @@ __global__ void __launch_bounds__(kDropoutBlock) dropout_masked_kernel(const Dro
             word = next_word;
         }
     }
-    dropout_tail<T, kWide>(a, keep, false);
+    dropout_tail<T, false>(a, keep, false);
 }
 
 enum class DropoutMask { kNone, kWrite, kRead };

@@ -3,20 +3,19 @@
 
 namespace thn {
 
-template <typename T, bool kWide>
-static void launch_mode(DropoutMask mode, const DropoutArgs& a, int grid, hipStream_t st) {
-    switch (mode) {
-        case DropoutMask::kNone: hipLaunchKernelGGL((dropout_flat_kernel<T, kWide>), dim3(grid), dim3(kDropoutBlock), 0, st, a); break;
-        case DropoutMask::kWrite: hipLaunchKernelGGL((dropout_masked_kernel<T, kWide, false>), dim3(grid), dim3(kDropoutBlock), 0, st, a); break;
-        case DropoutMask::kRead: hipLaunchKernelGGL((dropout_masked_kernel<T, kWide, true>), dim3(grid), dim3(kDropoutBlock), 0, st, a); break;
-    }
-}
-
+// a masked call's offsets start at 0 and end below 2^32 (dropout_launch in thn_api.hip)
 template <typename T>
 static void launch_as(DropoutMask mode, const DropoutArgs& a, int grid, hipStream_t st) {
-    // offsets that all fit 32 bits: the second counter word is zero throughout
-    if (a.first_offset + a.total_elems <= (int64_t{1} << 32)) launch_mode<T, false>(mode, a, grid, st);
-    else launch_mode<T, true>(mode, a, grid, st);
+    const dim3 blocks(grid), threads(kDropoutBlock);
+    switch (mode) {
+        case DropoutMask::kNone:
+            // offsets that all fit 32 bits: the second counter word is zero throughout
+            if (a.first_offset + a.total_elems <= (int64_t{1} << 32)) hipLaunchKernelGGL((dropout_flat_kernel<T, false>), blocks, threads, 0, st, a);
+            else hipLaunchKernelGGL((dropout_flat_kernel<T, true>), blocks, threads, 0, st, a);
+            break;
+        case DropoutMask::kWrite: hipLaunchKernelGGL((dropout_masked_kernel<T, false>), blocks, threads, 0, st, a); break;
+        case DropoutMask::kRead: hipLaunchKernelGGL((dropout_masked_kernel<T, true>), blocks, threads, 0, st, a); break;
+    }
 }
 
 int launch_dropout(int dtype, DropoutMask mode, const DropoutArgs& a, int grid, hipStream_t st) {

@@ -258,7 +258,7 @@ PyObject* act_bwd(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     END_HANDLE_TH_ERRORS
 }
 
-constexpr int64_t kMaskTo = int64_t{1} << 32;        // the masked kernels number up to 2^31 vectors
+constexpr int64_t kMaskTo = int64_t{1} << 32;        // the masked kernels take offsets of 32 bits
 
 // dropout_fwd(x, p, seed, keep) -> (out, mask or None), for 0 < p < 1 (in float32, as the kernels compare); keep: the decisions
 // are wanted for a backward (one byte per 16 bytes of input, in 32-bit words).  Under saved-tensor hooks (offloading, a
