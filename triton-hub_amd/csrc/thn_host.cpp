@@ -57,13 +57,15 @@ bool plain_param(PyObject* o, int64_t n, const at::Tensor** out) {
 void* address(const at::Tensor* t) { return t == nullptr ? nullptr : t->data_ptr(); }
 void* stream_of(const at::Tensor& t) { return c10::hip::getCurrentHIPStream(t.get_device()).stream(); }
 
-// The C ABI runs without the interpreter's lock, as a ctypes call does.
+// The C ABI runs without the interpreter's lock, as a ctypes call does.  An exception on its way out (an allocation or a mutex
+// of the library's caches) finds the lock held again: HANDLE_TH_ERRORS turns it into a Python error.
+struct Unlocked {
+    PyThreadState* const state = PyEval_SaveThread();
+    ~Unlocked() { PyEval_RestoreThread(state); }
+};
 template <typename Fn> int unlocked(Fn&& fn) {
-    int status;
-    Py_BEGIN_ALLOW_THREADS
-    status = fn();
-    Py_END_ALLOW_THREADS
-    return status;
+    const Unlocked here;
+    return fn();
 }
 
 PyObject* failed(int status) {
