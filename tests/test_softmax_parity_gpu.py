@@ -197,6 +197,25 @@ def test_rows_held_by_a_compute_unit(kind, dtype):
     assert torch.allclose(dx0.double(), dx1.double(), rtol=2 * eps + 1e-5, atol=1e-6)
 
 
+def test_row_counts_that_leave_the_compute_units_idle():
+    """The edges of the row counts at which a row in registers costs more than two walks (softmax_wide_vecs in thn_api.hip)."""
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    bf16, f32 = torch.bfloat16, torch.float32
+    # family (2 forward, 3 backward), log-softmax, 16-byte vectors of a row, type, rows, whether the row stays in registers
+    for which, log, vecs, dtype, rows, wide in (
+            (2, 0, 7680, bf16, cus, True), (2, 0, 7680, bf16, cus + 1, False), (2, 0, 7680, bf16, cus + cus // 4, False),
+            (2, 0, 7680, bf16, cus + cus // 4 + 1, True), (2, 0, 7681, bf16, cus + 1, True), (2, 1, 7680, bf16, cus + 1, True),
+            (2, 0, 4097, f32, cus, True), (2, 0, 4097, f32, cus + 1, False), (2, 1, 4097, f32, 2 * cus, True),
+            (2, 1, 4097, f32, 2 * cus + 1, False), (2, 1, 4097, f32, 2 * cus + cus // 32 + 1, True), (2, 0, 8193, f32, cus + 1, True),
+            (2, 0, 22528, bf16, cus + 1, False), (2, 0, 22528, bf16, cus + cus // 32 + 1, True), (2, 0, 22527, bf16, cus + cus // 4, False),
+            (2, 0, 22527, bf16, cus + cus // 4 + 1, True), (2, 1, 24576, bf16, 2 * cus + 1, False), (2, 1, 24576, bf16, 3 * cus + 1, True),
+            (2, 0, 22527, bf16, cus // 2, False), (2, 0, 22528, bf16, cus // 2, True), (2, 0, 24576, f32, cus + 1, True),
+            (2, 1, 24576, f32, cus + 1, False), (2, 0, 20480, bf16, cus + 1, True), (3, 0, 5120, bf16, cus + cus // 2 - 1, False),
+            (3, 0, 5120, bf16, cus + cus // 2, True), (3, 0, 5121, bf16, cus + cus // 2 - 1, True), (3, 1, 5120, bf16, cus + 1, True)):
+        shape = query_launch(which, log, rows, vecs * (4 if dtype == f32 else 8), dtype)
+        assert (shape[0] >= 8) == wide, (which, log, vecs, dtype, rows, shape)
+
+
 @pytest.mark.parametrize("n", [32768 + 8, 400000])
 def test_a_nan_spoils_its_wide_row_and_no_other(n):
     """A NaN in a row wider than 64 KiB, in registers or walked twice: the row is NaN, as a narrow row is; -inf is not."""

@@ -408,16 +408,44 @@ int default_blocks_per_cu(int which, int flavour, int block) {
     return kDefaultBlocksPerCu;
 }
 
-// Vectors per thread of the register-resident softmax kernels (thn_softmax_wide.h) for M rows of N columns, 0 where the
-// looping kernels run: float64, rows of more than 24 x 1024 vectors, an overridden launch shape of those kernels, and where
-// the second walk costs nothing, because what it reads still lies in the eight 4-MiB L2s:
+// Row counts at which the forward loses by holding its rows in one workgroup per compute unit, where the looping kernels run
+// two: a last round of workgroups for a few rows, in rows that leave slots of their vectors per thread idle or that need all
+// 24, whose sums spill.  Looping / registers, of a forward alone and of a forward + backward:
+//   8 vectors per thread, at most 7.5 x 1024 vectors, softmax, a second round of up to a quarter: bfloat16 0.88-1.04 x and
+//     0.93-1.02 x (257 x 37600 0.88 and 0.93), float32 0.89-1.01 x and 0.95-1.01 x (257 x 18800 0.89 and 0.95); fuller rows
+//     0.95-1.08 x and 0.97-1.04 x, half of a second round 0.95-1.07 x and 0.99-1.05 x.  Log-softmax, whose backward holds its
+//     rows there as well, loses with a third round of up to a 32nd: bfloat16 0.92-0.98 x and 0.96-0.99 x, float32 0.86-0.93 x
+//     and 0.94-0.96 x (513 x 18800 0.86 and 0.94);
+//   24 vectors, 16-bit, a second or third round of up to a 32nd: 0.84-0.92 x and 0.92-0.98 x (257 x 164797 0.84 and 0.92 for
+//     log-softmax), 0.90-0.96 x and 0.95-0.99 x; with more than two of the 24 idle also up to a quarter of a second round
+//     (0.93-0.96 x and 0.97-0.99 x) and up to half of the compute units (128 x 164800 0.88-0.91 x and 0.96-0.97 x).  float32
+//     log-softmax, a second round of up to a 32nd: 0.88-1.00 x and 0.94-1.00 x; softmax gains 4-9 % of a pass there.
+// Left as it is: float32 with 8 vectors per thread loses up to 15 % of a forward alone at other counts too (513, 769, 3000), where
+// a softmax forward + backward gains 0-5 % and a log-softmax pass loses up to 6 % or gains as much, by the rounds.
+bool wide_fwd_loses(bool is_log, int64_t M, int64_t vecs, int k, int bytes, int cus) {
+    const auto few_rows_behind = [&](int rounds, int share) {
+        const int64_t over = M - static_cast<int64_t>(rounds) * cus;
+        return over > 0 && share * over <= cus;
+    };
+    if (k == 8) return vecs <= 7680 && (is_log ? few_rows_behind(2, 32) : few_rows_behind(1, 4));
+    if (k < 24) return false;
+    if (bytes != 2) return is_log && few_rows_behind(1, 32);
+    const bool idle = vecs < 22 * thn::kWideBlock;
+    return few_rows_behind(1, idle ? 4 : 32) || few_rows_behind(2, 32) || (idle && 2 * M <= cus);
+}
+
+// Vectors per thread of the register-resident softmax kernels (thn_softmax_wide.h) for M rows of N columns on `cus` compute
+// units, 0 where the looping kernels run: float64, rows of more than 24 x 1024 vectors, an overridden launch shape of those
+// kernels, and where the second walk costs nothing, because what it reads still lies in the eight 4-MiB L2s:
 //   forward, 16-bit: x of less than 24 MiB (bfloat16 looping -> registers, softmax: 64 x 40000 9.1 -> 9.9 us, 192 x 40000 10.0 ->
 //     10.6, 64 x 90001 16.2 -> 17.5, 192 x 90001 21.5 -> 18.7, 512 x 151936 75.5 -> 63.7).  float32 rows have half the
-//     elements per byte and gain at every row count (32 x 40000 10.1 -> 8.9, 256 x 40000 18.8 -> 15.4);
+//     elements per byte and gain below that too (32 x 40000 10.1 -> 8.9, 256 x 40000 18.8 -> 15.4; rows of little more than
+//     64 KiB, 16400 columns, lose 5-10 % of a forward alone between 16 and 128 rows and gain 0-4 % of a pass);
 //   softmax backward (which reads y twice either way): y and dy of less than 48 MiB together (bfloat16 64 x 40000 7.9 -> 8.3,
-//     300 x 40000 19.1 -> 19.8, 256 x 90001 37.2 -> 26.8), and float32 rows that need 24 vectors per thread (spills).
-//     The log-softmax backward gains everywhere (bfloat16 16 x 40000 8.5 -> 7.8, 300 x 90001 45.2 -> 39.7).
-int softmax_wide_vecs(int which, bool is_log, int64_t M, int64_t N, int dtype) {
+//     256 x 90001 37.2 -> 26.8), rows of at most 5 x 1024 vectors up to half of a second round of workgroups (bfloat16 383 x
+//     37600 0.95 x, float32 383 x 18800 0.93 x), and float32 rows that need 24 vectors per thread (spills).
+//     The log-softmax backward gains everywhere else (bfloat16 300 x 90001 45.2 -> 39.7; 16 x 32800 and 257 x 32800 0.92-0.96 x).
+int softmax_wide_vecs(int which, bool is_log, int64_t M, int64_t N, int dtype, int cus) {
     const int bytes = elem_bytes(dtype);
     const int64_t vecs = N / (16 / bytes);
     if (dtype == THN_F64 || vecs > thn::kWideMaxVecs) return 0;
@@ -427,8 +455,9 @@ int softmax_wide_vecs(int which, bool is_log, int64_t M, int64_t N, int dtype) {
     if (ov.k.load() >= 8 && ov.tpr.load() == thn::kWideBlock) return k;
     if (ov.block.load() > 0 || ov.bpc.load() > 0) return 0;
     const int64_t mib = M * N * bytes >> 20;
-    if (which == kSoftmaxFwd && bytes == 2 && mib < 24) return 0;
+    if (which == kSoftmaxFwd && ((bytes == 2 && mib < 24) || wide_fwd_loses(is_log, M, vecs, k, bytes, cus))) return 0;
     if (which == kSoftmaxBwd && !is_log && (mib < 24 || (bytes == 4 && k == 24))) return 0;
+    if (which == kSoftmaxBwd && !is_log && vecs <= 5 * thn::kWideBlock && M > cus && 2 * M < 3 * cus) return 0;
     return k;
 }
 
@@ -1877,7 +1906,7 @@ int thn_norm_query_launch(int which, int is_layernorm, int64_t M, int64_t N, int
             softmax_loop_launch(which, &block, &bpc);
             const int64_t cap = static_cast<int64_t>(cus) * bpc;
             grid = static_cast<int>(M < cap ? M : cap);
-            const int k = softmax_wide_vecs(which, flavour & 1, M, N, x_dtype);
+            const int k = softmax_wide_vecs(which, flavour & 1, M, N, x_dtype, cus);
             if (k > 0) {                            // rows in the registers of a compute unit (dense tensors)
                 shape[0] = k;
                 shape[1] = shape[2] = thn::kWideBlock;
@@ -2144,7 +2173,7 @@ int thn_softmax_fwd(const void* x, int64_t x_row_stride, void* y, int64_t y_row_
         a.sign = kind == THN_SOFTMIN ? -1.0f : 1.0f;
         int block, bpc, lrc;
         softmax_loop_launch(kSoftmaxFwd, &block, &bpc);
-        const int k = softmax_wide_vecs(kSoftmaxFwd, kind == THN_LOGSOFTMAX, M, N, dtype);
+        const int k = softmax_wide_vecs(kSoftmaxFwd, kind == THN_LOGSOFTMAX, M, N, dtype, cus);
         if (k > 0 && same_phase({{x, a.x_stride_bytes}, {y, a.y_stride_bytes}}, M, bytes)) {
             const int grid = static_cast<int>(M < cus ? M : cus);
             lrc = launch_softmax_fwd_wide(dtype, kind == THN_LOGSOFTMAX, k, a, grid, static_cast<hipStream_t>(stream));
@@ -2237,7 +2266,7 @@ int thn_softmax_bwd(const void* y, int64_t y_row_stride, const void* dy, int64_t
         a.sign = kind == THN_SOFTMIN ? -1.0f : 1.0f;
         int block, bpc, lrc;
         softmax_loop_launch(kSoftmaxBwd, &block, &bpc);
-        const int k = softmax_wide_vecs(kSoftmaxBwd, kind == THN_LOGSOFTMAX, M, N, dtype);
+        const int k = softmax_wide_vecs(kSoftmaxBwd, kind == THN_LOGSOFTMAX, M, N, dtype, cus);
         if (k > 0 && same_phase({{y, a.y_stride_bytes}, {dy, a.dy_stride_bytes}, {dx, a.dx_stride_bytes}}, M, bytes)) {
             const int grid = static_cast<int>(M < cus ? M : cus);
             lrc = launch_softmax_bwd_wide(dtype, kind == THN_LOGSOFTMAX, k, a, grid, static_cast<hipStream_t>(stream));
