@@ -15,7 +15,8 @@ import numpy as np
 import pytest
 import torch
 
-from conftest import ROOT, check_elementwise, f64
+from conftest import EPS32, FMT, ROOT, check_elementwise, f64
+from oracle import norm_oracle as no
 from oracle import softmax_oracle as so
 from TritonHub import _native
 from TritonHub.Activations import LogSoftmax, Softmax, Softmin, _launch
@@ -195,6 +196,62 @@ def test_rows_held_by_a_compute_unit(kind, dtype):
     eps = torch.finfo(dtype).eps                            # both are within an ulp and a few float32 roundings of the same value
     assert torch.allclose(y0.double(), y1.double(), rtol=2 * eps + 2e-6, atol=1e-6)
     assert torch.allclose(dx0.double(), dx1.double(), rtol=2 * eps + 1e-5, atol=1e-6)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("k", [8, 12, 16, 20, 24])
+@pytest.mark.parametrize("kind", KINDS)
+def test_a_compute_unit_carries_nothing_over_to_its_next_row(kind, k, dtype):
+    """Two and three rows per workgroup in every number of vectors per thread: a row is stored while the workgroup's next one is
+    requested and summed.  Dense rows of whole vectors and rows whose start moves against the 16-byte boundaries; every row
+    with a scale and an offset of its own, so that nothing of another row goes unseen.  Rows around the change of rounds
+    against the oracle, every row against a launch in which its workgroup has no other."""
+    vec = 16 // torch.empty((), dtype=dtype).element_size()
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    lib = _native.lib()
+    log, code = kind == "logsoftmax", CODE[kind]
+
+    def override(*shape):
+        for which in (2, 3):
+            assert lib.thn_norm_set_launch_override(which, *shape) == 0
+
+    for m in (cus + 3, 2 * cus + 1):
+        for n in ((k * 1024 - 100) * vec, (k * 1024 - 100) * vec - 3):
+            announce(f"rows carried by a compute unit {kind} {dtype} K={k} {m} x {n}")
+            g = torch.Generator(device="cuda").manual_seed(n + m)
+            r = torch.arange(m, device="cuda")[:, None]
+            x = torch.randn(m, n, device="cuda", generator=g).mul_(1 + r % 5).add_(r % 7).to(dtype)
+            # (row sums of up to 5 / 32 * 196608 = 30720: exp(y) times that stays below float16's 65504)
+            dy = torch.randn(m, n, device="cuda", generator=g).mul_(1 + r % 3).add_((r % 11 - 5) / 32).to(dtype)
+            try:
+                override(8, 1024, 0, 0)
+                assert query_launch(2, log, m, n, dtype)[0] == k and query_launch(3, log, m, n, dtype)[0] == k
+                y = _launch.softmax_fwd(x, code)
+                dx = _launch.softmax_bwd(y, dy, code)
+                for first in range(0, m, cus):          # each row the only one of its workgroup: the same bits
+                    part = slice(first, min(first + cus, m))
+                    assert torch.equal(_launch.softmax_fwd(x[part], code), y[part]), (m, n, first)
+                    assert torch.equal(_launch.softmax_bwd(y[part], dy[part], code), dx[part]), (m, n, first)
+            finally:
+                override(0, 0, 0, 0)
+            rows = torch.tensor([0, 1, cus - 1, cus, cus + 1, m - 1])
+            xc, gc, ys = (f64(t[rows.cuda()].cpu()) for t in (x, dy, y))
+            yo = so.FWD[kind](xc)
+            z = xc - xc.max(1, keepdims=True)
+            scale = np.abs(z) + np.abs(yo - z) + 1.0 if log else np.abs(yo)          # as in run_and_compare
+            check(y[rows.cuda()].cpu(), yo, scale, dtype, kind, f"{kind} K={k} {m} x {n} y")
+            scale = np.abs(gc) + np.exp(ys) * np.abs(gc).sum(1, keepdims=True) if log \
+                else np.abs(ys) * (np.abs(gc) + np.abs(ys * gc).sum(1, keepdims=True))
+            ref, got = so.BWD[kind](ys, gc), dx[rows.cuda()].cpu()
+            if log:
+                # check_elementwise's bound, and for rows whose sum is far from 0 the product exp(y) * sum: the exponential
+                # works on y log2(e) in float32, 2^-24 of which it is off by, and by 2 ulp of its own
+                bound = np.maximum(1e-5, 4 * no.ulp(ref, "fp32")) if dtype == torch.float32 else no.ulp(ref, FMT[dtype]) + 4 * EPS32 * scale
+                bound = bound + np.exp(ys) * np.abs(gc.sum(1, keepdims=True)) * EPS32 * (np.abs(ys) * 1.4427 + 4)
+                worst = (np.abs(f64(got) - ref) / bound).max()
+                assert worst <= 1, f"{kind} K={k} {m} x {n} dx: {worst} of the bound"
+            else:
+                check(got, ref, scale, dtype, kind, f"{kind} K={k} {m} x {n} dx")
 
 
 def test_row_counts_that_leave_the_compute_units_idle():
