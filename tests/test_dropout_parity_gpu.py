@@ -280,6 +280,27 @@ def test_backward_under_a_checkpoint_keeps_the_decisions_of_its_output(n):
     assert len(seen) == 1 and torch.equal(seen[0] != 0, kept)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16, torch.float64])
+@pytest.mark.parametrize("n", [1 << 22, (1 << 22) + 13])
+def test_kept_decisions_for_every_gradient(n, dtype):
+    """The first backward of a forward reads its decisions whatever the gradient's layout: off the 16-byte path, strided,
+    expanded."""
+    x = torch.randn(n, device="cuda").to(dtype).requires_grad_(True)
+    dy = torch.randn(n, device="cuda").to(dtype)
+    bits = {2: torch.int16, 4: torch.int32, 8: torch.int64}[x.element_size()]
+    for grad in (dy, torch.empty(n + 1, dtype=dtype, device="cuda")[1:].copy_(dy), torch.stack((dy, dy), 1)[:, 0], dy[:1].expand(n)):
+        random.seed(n)
+        seed = random.randint(0, 2 ** 16)
+        random.seed(n)
+        y = Dropout(0.3)(x)
+        assert y.grad_fn.mask is not None
+        got = torch.autograd.grad(y, x, grad, retain_graph=True)[0]
+        assert y.grad_fn.mask is None
+        flat, want = grad.contiguous(), torch.empty_like(dy)
+        assert _native.lib().thn_dropout(flat.data_ptr(), want.data_ptr(), n, 0, 0.3, seed, _native.dtype_code(dtype), 0) == 0
+        assert torch.equal(got.view(bits), want.view(bits))
+
+
 def test_captured_backward_of_an_eager_forward():
     """The backward alone in a graph, replayed after the forward's node has died and its memory has been written over: the
     bits of the eager backward every time.  Both directions in a graph too."""

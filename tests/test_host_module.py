@@ -31,6 +31,15 @@ def test_host_tensors_and_wrong_argument_counts():
             getattr(host, name)(*[x] * (count - 1))
 
 
+def test_dropout_refusals():
+    host, x = _native.host(), torch.randn(4, 8)
+    assert host.dropout_fwd(x, 0.5, 1, True) is None and host.dropout_bwd(x, 0.5, 1, None) is None
+    for count in (3, 5):
+        for name in ("dropout_fwd", "dropout_bwd"):
+            with pytest.raises(TypeError):
+                getattr(host, name)(*[x] * count)
+
+
 @pytest.fixture
 def dropout_calls(monkeypatch):
     """Dropout over a host module that only notes what it is asked for, for tensors of four elements and more; the "mask" is
@@ -166,3 +175,61 @@ def test_dropout_results_have_contiguous_strides(monkeypatch):
     here = strides()
     monkeypatch.setattr(_native, "host", lambda: _General())
     assert here == strides() == ((24, 24, 8, 1),) * 2
+
+
+@pytest.mark.gpu
+def test_dropout_forms_left_to_the_wrapper():
+    """A mask of another size, type or place, a probability or a seed that is no plain number, rows apart."""
+    host, n = _native.host(), 1 << 13          # two pieces of 1024 vectors in float32, one in 16 bits
+    x = torch.randn(n, device="cuda")
+    out, mask = host.dropout_fwd(x, 0.5, 1, True)
+    assert host.dropout_bwd(x, 0.5, 1, mask) is not None and host.dropout_bwd(x, 0.5, 1, None) is not None
+    for other in (mask[:-1], torch.cat((mask, mask)), mask.float(), mask.cpu(), mask.repeat(2)[::2], "mask"):
+        assert host.dropout_bwd(x, 0.5, 1, other) is None
+    assert host.dropout_bwd(x.bfloat16(), 0.5, 1, mask) is None          # half the pieces: half the mask
+    for p, seed in ((0.0, 1), (1.0, 1), (1.0 - 1e-12, 1), (float("nan"), 1), ("0.5", 1), (0.5, 1.0), (0.5, 1 << 70)):
+        assert host.dropout_fwd(x, p, seed, False) is None and host.dropout_bwd(x, p, seed, None) is None, (p, seed)
+    for t in (x[::2], x[:0], x.int()):
+        assert host.dropout_fwd(t, 0.5, 1, False) is None and host.dropout_bwd(t, 0.5, 1, None) is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("side_stream", [False, True])
+@pytest.mark.parametrize("dtype,param", [(torch.float16, torch.bfloat16), (torch.bfloat16, torch.float16), (torch.float32, torch.float64)])
+def test_other_parameter_types_streams_and_gradients(dtype, param, side_stream, monkeypatch):
+    """Parameters of another type than the input, the calls on a stream of their own with work in front of them, gradients
+    that are not contiguous (which the wrappers take): the same bits as the general way."""
+    rows, n = 300, 1000
+    g = torch.Generator(device="cuda").manual_seed(n)
+    x, dy = (torch.randn(rows, n, device="cuda", generator=g).to(dtype) for _ in range(2))
+    w, b = (torch.randn(n, device="cuda", generator=g).to(param) for _ in range(2))
+    gradients = (dy, dy.t().contiguous().t(), torch.stack((dy, dy), -1)[..., 0], dy[:1].expand(rows, n))
+    assert _native.host().norm_fwd(x, w, b, 1e-5, True, -1, 0) is not None
+
+    def everything():
+        for layernorm, bias in ((True, b), (False, None)):
+            y, mean, rstd = norm_launch.norm_fwd(x, w, bias, 1e-5, layernorm)
+            yield from (y, mean, rstd)
+            for grad in gradients:
+                yield from norm_launch.norm_bwd(x, grad, w, bias, mean, rstd, layernorm)
+        y = act_launch.softmax_fwd(x, _native.SOFTMAX)
+        yield y
+        for grad in gradients:
+            yield act_launch.softmax_bwd(y, grad, _native.SOFTMAX)
+            yield act_launch.act_bwd(x, grad, _native.ACT_GELU)
+
+    def on_a_stream():
+        stream = torch.cuda.Stream() if side_stream else torch.cuda.current_stream()
+        stream.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(stream):
+            busy = torch.ones(1 << 24, device="cuda")
+            for _ in range(4):
+                busy = busy * 1.5
+            results = list(everything())
+        stream.synchronize()
+        return results
+
+    here = on_a_stream()
+    monkeypatch.setattr(_native, "host", lambda: _General())
+    general = on_a_stream()
+    assert len(here) == len(general) and all(_same(a, c) for a, c in zip(here, general))
