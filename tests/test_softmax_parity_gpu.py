@@ -268,7 +268,10 @@ def test_row_counts_that_leave_the_compute_units_idle():
             (2, 0, 22527, bf16, cus + cus // 4 + 1, True), (2, 1, 24576, bf16, 2 * cus + 1, False), (2, 1, 24576, bf16, 3 * cus + 1, True),
             (2, 0, 22527, bf16, cus // 2, False), (2, 0, 22528, bf16, cus // 2, True), (2, 0, 24576, f32, cus + 1, True),
             (2, 1, 24576, f32, cus + 1, False), (2, 0, 20480, bf16, cus + 1, True), (3, 0, 5120, bf16, cus + cus // 2 - 1, False),
-            (3, 0, 5120, bf16, cus + cus // 2, True), (3, 0, 5121, bf16, cus + cus // 2 - 1, True), (3, 1, 5120, bf16, cus + 1, True)):
+            (3, 0, 5120, bf16, cus + cus // 2, True), (3, 0, 5121, bf16, cus + cus // 2 - 1, True), (3, 1, 5120, bf16, cus + 1, True),
+            # float32 tensors of 700 MiB (5734.4 rows of 8000 vectors) and 900 MiB (7372.8)
+            (2, 0, 8000, f32, 5734, True), (2, 0, 8000, f32, 5735, False), (2, 1, 8000, bf16, 5735, True), (2, 0, 8193, f32, 7373, True),
+            (3, 1, 8000, f32, 7372, True), (3, 1, 8000, f32, 7373, False), (3, 0, 8000, f32, 7373, True), (3, 1, 20481, f32, 7373, True)):
         shape = query_launch(which, log, rows, vecs * (4 if dtype == f32 else 8), dtype)
         assert (shape[0] >= 8) == wide, (which, log, vecs, dtype, rows, shape)
 

@@ -444,7 +444,10 @@ bool wide_fwd_loses(bool is_log, int64_t M, int64_t vecs, int k, int bytes, int 
 //   softmax backward (which reads y twice either way): y and dy of less than 48 MiB together (bfloat16 64 x 40000 7.9 -> 8.3,
 //     256 x 90001 37.2 -> 26.8), rows of at most 5 x 1024 vectors up to half of a second round of workgroups (bfloat16 383 x
 //     37600 0.95 x, float32 383 x 18800 0.93 x), and float32 rows that need 24 vectors per thread (spills).
-//     The log-softmax backward gains everywhere else (bfloat16 300 x 90001 45.2 -> 39.7; 16 x 32800 and 257 x 32800 0.92-0.96 x).
+//     The log-softmax backward gains at most sizes (bfloat16 300 x 90001 45.2 -> 39.7; 16 x 32800 and 257 x 32800 0.92-0.96 x);
+//   float32 tensors that dwarf the memory-side cache, in rows of more than 6 x 1024 vectors: forward with 8 vectors per thread
+//     from 700 MiB on 0.93-1.03 x (8192 x 31997 softmax 0.94), log-softmax backward from 900 MiB on 0.95-1.01 x (8192 x 32000 541 ->
+//     553; both directions 912 -> 928), up to 1.12 x and 1.18 x below that; 16-bit rows 0.97-1.17 x and 0.98-1.17 x at any size.
 int softmax_wide_vecs(int which, bool is_log, int64_t M, int64_t N, int dtype, int cus) {
     const int bytes = elem_bytes(dtype);
     const int64_t vecs = N / (16 / bytes);
@@ -457,6 +460,10 @@ int softmax_wide_vecs(int which, bool is_log, int64_t M, int64_t N, int dtype, i
     const int64_t mib = M * N * bytes >> 20;
     if (which == kSoftmaxFwd && ((bytes == 2 && mib < 24) || wide_fwd_loses(is_log, M, vecs, k, bytes, cus))) return 0;
     if (which == kSoftmaxBwd && !is_log && (mib < 24 || (bytes == 4 && k == 24))) return 0;
+    if (bytes == 4 && vecs > 6 * thn::kWideBlock) {
+        if (which == kSoftmaxFwd && k == 8 && mib >= 700) return 0;
+        if (which == kSoftmaxBwd && is_log && k < 24 && mib >= 900) return 0;
+    }
     if (which == kSoftmaxBwd && !is_log && vecs <= 5 * thn::kWideBlock && M > cus && 2 * M < 3 * cus) return 0;
     return k;
 }
