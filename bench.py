@@ -75,7 +75,7 @@ WORKLOADS = {
     "softmax_bf16_932067x72_narrow": ("softmax", 932067, 72, "bf16"),
     # off the 128-bit path: a ViT's attention row (197 columns, 25 unaligned windows: the flat kernels' other instances)
     "softmax_bf16_340654x197_ragged": ("softmax", 340654, 197, "bf16"),
-    # vocabulary-sized rows, wider than 64 KiB: the looping kernels (two walks per row)
+    # vocabulary-sized rows, wider than 64 KiB: the looping kernels (two walks per row) and the rows held in registers
     "logsoftmax_f32_8192x32000_vocab": ("logsoftmax", 8192, 32000, "f32"),
     "logsoftmax_bf16_4096x128256_vocab": ("logsoftmax", 4096, 128256, "bf16"),
     # row p-norm / normalize of a (1, rows, K) tensor (thn_normalize_fwd + thn_normalize_bwd, or thn_pnorm_*)
@@ -1117,8 +1117,8 @@ def dropout_main(args, lib, dev, m, n, dname, dtype):
         "roofline": {"bound": "hbm", "kernel": "dropout_flat_kernel", "achieved": round(achieved, 1),
                      "peak": HBM_PEAK_GBPS, "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBPS, 4),
                      "algorithmic_bytes_per_launch": launch_bytes, "avg_launch_us": round(fwd_us, 2), "traffic": None,
-                     "note": "limited by the 37 32x32-bit multiplications of one Philox-4x32-10 block per element "
-                             "(quarter-rate instructions), not by memory"},
+                     "note": "limited by the vector instructions of one Philox-4x32-10 block per element (17 32x32-bit "
+                             "multiplications among them), not by memory"},
     }
     if not args.no_cpu_baseline:
         from oracle import dropout_oracle as do

@@ -154,3 +154,44 @@ def test_looping_kernels_keep_to_their_rows(n, pad, dtype):
                                  n, p, code, st) == 0
         torch.cuda.synchronize()
         check_guards(dxbuf, m, n, pad, lead, f"p-norm backward p={p}")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("pad", PADS)
+@pytest.mark.parametrize("k,idle", [(8, 4 * 1024 - 1), (8, 0), (16, 77), (24, 3)])
+def test_rows_held_in_registers_keep_to_themselves(k, idle, pad, dtype):
+    """Softmax rows of 64 to 384 KiB in the registers of a compute unit: all streams with one pitch and one place against the
+    16-byte boundaries, which is what these kernels take; the padding of the inputs is NaN, so that reading it shows as well."""
+    vec = 16 // torch.empty((), dtype=dtype).element_size()
+    n, m = (k * 1024 - idle) * vec + (vec - 1 if idle else 0), 5
+    print(f"\n[case] output guards, rows in registers K={k} N={n} pad={pad} {dtype}", flush=True)
+    lib, st, code, pitch = _native.lib(), torch.cuda.current_stream().cuda_stream, _native.dtype_code(dtype), n + pad
+    g = torch.Generator(device="cuda").manual_seed(n + pad)
+
+    def source(values):
+        buf, ptr, lead = padded(m, n, pad, dtype)
+        buf.fill_(float("nan"))
+        buf[lead:lead + m * pitch].view(m, pitch)[:, :n] = values
+        return buf, ptr
+
+    x = (0.3 + torch.randn(m, n, device="cuda", generator=g)).to(dtype)
+    dy = torch.randn(m, n, device="cuda", generator=g).to(dtype)
+    try:
+        for which in (2, 3):
+            assert lib.thn_norm_set_launch_override(which, 8, 1024, 0, 0) == 0
+        for kind in (_native.SOFTMAX, _native.LOGSOFTMAX):
+            xbuf, xptr = source(x)
+            ybuf, yptr, lead = padded(m, n, pad, dtype)
+            assert lib.thn_softmax_fwd(xptr, pitch, yptr, pitch, m, n, kind, code, st) == 0
+            y = check_guards(ybuf, m, n, pad, lead, f"softmax forward kind {kind}")
+            ref = (torch.softmax if kind == _native.SOFTMAX else torch.log_softmax)(x.float(), -1)
+            assert torch.allclose(y, ref.cpu(), rtol=1e-2 if dtype == torch.bfloat16 else 1e-5, atol=1e-6)
+            ysaved, ysptr = source(ref.to(dtype))
+            dybuf, dyptr = source(dy)
+            dxbuf, dxptr, lead = padded(m, n, pad, dtype)
+            assert lib.thn_softmax_bwd(ysptr, pitch, dyptr, pitch, dxptr, pitch, m, n, kind, code, st) == 0
+            dx = check_guards(dxbuf, m, n, pad, lead, f"softmax backward kind {kind}")
+            assert not bool(torch.isnan(dx).any())
+    finally:
+        for which in (2, 3):
+            lib.thn_norm_set_launch_override(which, 0, 0, 0, 0)

@@ -127,7 +127,8 @@ def test_row_width_limit(kind, dtype, n_max):
     announce(f"row limit {kind} {dtype} N={n_max}")
     x, dy = make((6, n_max), dtype, seed=5, scale=2.0)
     run_and_compare(kind, x, dy, f"{kind} N={n_max}")
-    # one vector beyond what the row engine holds: the looping kernels, still one softmax of the whole row
+    # beyond what the row engine holds (the kernels for wider rows, the looping ones or those that hold a row in the registers
+    # of a compute unit): still one softmax of the whole row
     x, dy = make((6, n_max + 8), dtype, seed=6, scale=2.0)
     run_and_compare(kind, x, dy, f"{kind} N={n_max + 8}")
 

@@ -53,10 +53,10 @@ __device__ __forceinline__ float gelu_tanh_gate(float x) { return gelu_tanh_gate
 // factor 1/2 of Phi is folded into the coefficients.
 //
 // Backward form: erfc(z)/2 = t*Q(t)*exp(-z^2), Q of degree 8: a minimax fit of the relative error over z in [0, 9.3], behind
-// which the exponential underflows (4e-8; degree 7 gives 3e-7).  Its exponential is exp(-x^2/2), the one the normal
+// which the exponential underflows (5.1e-8 with the coefficients as stored; degree 7 gives 3e-7).  Its exponential is exp(-x^2/2), the one the normal
 // density needs: GeLU' = Phi(x) + x*phi(x) is 1 + r for x >= 0 and -r for x < 0 with r = exp(-x^2/2)*(|x|/sqrt(2 pi) - t*Q(t)).
 // Three instructions per element fewer than Q of degree 10 with Phi and phi put together afterwards, and closer to float64
-// (GeLU' in float32, x = 1.5 g + 0.25 with g normal, 2-norm: 4.5e-8 against 4.7e-8): LayerNorm + GeLU backward bfloat16
+// (GeLU' in float32, x = 1.5 g + 0.25 with g normal, relative 2-norm: 4.47e-8 against 4.75e-8): LayerNorm + GeLU backward bfloat16
 // 16384 x 4096, which is bound by arithmetic, 97.4 -> 92.9 us together with one instruction less for the corrected xhat.
 __device__ __forceinline__ float gelu_slope(float x) {
     const float a = __builtin_fabsf(x) * 0.84932180028801907f;

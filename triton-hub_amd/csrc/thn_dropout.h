@@ -15,9 +15,9 @@
 //    words that are dropped (dropout_threshold) and the test is one addition and one unsigned comparison: v lies in
 //    [-T, T - 1] exactly if uint32(v + T) < 2 T;
 //  * a dropped element is selected before it is scaled (0 scales to +0), which leaves no branch.
-// Issue costs measured for one wave (cycles): v_mad_u64_u32 / v_mul_hi_u32 4.2, v_bitop3_b32 and v_xor_b32 2.5, v_cmp_u32 4.2,
-// v_mul_f64 and the float64 conversions 4.2-4.5.  bfloat16 16384 x 4096 (134 MB in, 134 MB out),
-// launches of one direction after another: 123 -> 92 us.
+// bfloat16 16384 x 4096 (134 MB in, 134 MB out), launches of one direction after another: 123 -> 92 us.  43.3 vector
+// instructions per element at 4.1 cycles each: the vector units issue in 93 % of the cycles in which a compute unit is busy (97 % in
+// the forward that keeps its decisions), 78 us at the 2.38 GHz of these launches.
 #pragma once
 
 #include <hip/hip_runtime.h>

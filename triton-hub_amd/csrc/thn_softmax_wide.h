@@ -1,17 +1,18 @@
 // Softmax / Softmin / LogSoftmax over rows wider than 64 KiB that one compute unit can still hold in its registers
 // (up to 384 KiB: K vectors of 16 bytes in each of 1024 threads), in 16- and 32-bit storage: every tensor is read once.
 //
-// The looping kernels (thn_softmax.h) walk such a row twice.  The second walk comes from the memory-side cache, which
-// gives no more than memory itself: their forward moves 3 and their backward 5 tensors through a pipe that a
-// register-resident row loads with 2 and 3.  One workgroup fills a compute unit; while it writes vector k of a row it
+// The looping kernels (thn_softmax.h) walk such a row twice, the second time from the caches: their forward moves 3 and their
+// backward 5 tensors through the compute units where a register-resident row moves 2 and 3.  One workgroup fills a compute unit; while it writes vector k of a row it
 // requests vector k of its next row into the same registers, so that only the reductions between the passes leave
 // the unit without requests, and the units are in different phases.
 //
 // Measured (looping -> registers, us): log-softmax bfloat16 4096 x 128256 forward 439 -> 394, backward 587 -> 580, both
 // 1024 -> 975; softmax backward 721 -> 587, both 1160 -> 983; log-softmax both directions 512 x 151936 171 -> 149, 2000 x 50257
-// 216 -> 198, float32 512 x 96000 203 -> 183.  What bounds it is memory: tensors of 1 GiB stream at 5.3 (forward) and 5.4 TB/s
-// (backward), where a plain device-to-device copy of 1 GiB reaches 4.8; 2, 4 or 8 vectors of lag and 1, 2 or 4 of y
-// ahead stay within 2 % of each other.
+// 216 -> 198, float32 512 x 96000 203 -> 183.  Tensors of 1 GiB stream at 5.3 (forward) and 5.4 TB/s (backward), each byte fetched
+// and written once (FETCH_SIZE, WRITE_SIZE), where a bare copy loop reaches 6.15 and a loop with two reads 6.2: between the
+// last request of a row and the first of the next lie two reductions over the whole workgroup (backward: one), in which the
+// only workgroup of the compute unit asks for nothing.  2, 4 or 8 vectors of lag and 1, 2 or 4 of y ahead stay within 2 % of each
+// other.  Which rows and row counts run here: softmax_wide_vecs() in thn_api.hip.
 //
 // Rows may start at any element: the vectors are those on 16-byte boundaries, and the up to VEC - 1 elements in front of
 // and behind them go to one lane each ("edge" elements).  The launcher takes these kernels when all streams sit at the same

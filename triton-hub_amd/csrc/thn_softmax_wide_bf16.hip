@@ -1,4 +1,4 @@
-// Flat-mapped Softmax / Softmin / LogSoftmax kernels for narrow rows, BF16 storage.
+// Softmax / Softmin / LogSoftmax kernels for rows of 64 to 384 KiB that stay in registers, BF16 storage.
 #include "thn_softmax_wide.h"
 
 namespace thn {

@@ -1,4 +1,4 @@
-// Flat-mapped Softmax / Softmin / LogSoftmax kernels for narrow rows, F32 storage.
+// Softmax / Softmin / LogSoftmax kernels for rows of 64 to 384 KiB that stay in registers, F32 storage.
 #include "thn_softmax_wide.h"
 
 namespace thn {
