@@ -45,14 +45,14 @@ def _check_feature_dim(n: int, element_size: int) -> None:
 
 
 # How the forward reads x (include/thnorm.h, thn_cache_policy): 'keep' leaves x in the caches for the backward,
-# 'stream' does not; 'auto' keeps it exactly when autograd will run a backward for the call.
+# 'stream' does not; 'auto' keeps it when an input of the autograd Function requires a gradient (also under no_grad).
 _CACHE_POLICIES = ('auto', 'keep', 'stream')
 _cache_policy = 'auto'
 
 
 def set_cache_policy(policy: str) -> None:
-    """'auto' (default): the forward keeps x in the caches when a backward will follow (some input of the autograd
-    Function requires a gradient) and streams it otherwise (inference); 'keep' / 'stream': always.  Choose 'stream'
+    """'auto' (default): the forward keeps x in the caches when some input of the autograd Function requires a gradient
+    (parameters that do count under no_grad as well) and streams it otherwise; 'keep' / 'stream': always.  Choose 'stream'
     for training loops in which so much other work runs between a layer's forward and its backward that nothing of
     x would still be cached: the forward alone is 2-3 % faster that way.  Results are bit-identical under all three."""
     global _cache_policy
@@ -123,8 +123,8 @@ def _workspace(index: int, stream: int, nbytes: int, device) -> torch.Tensor:
 
 def norm_fwd(x: torch.Tensor, weight, bias, eps: float, layernorm: bool, act: int = -1, backward_follows: bool = True):
     """Returns (y like x, mean (M,) float32 or None, rstd (M,) float32).  `act` >= 0: the activation with that
-    code is applied in the same pass (thn_norm_act_fwd).  `backward_follows`: whether autograd will run a backward
-    for this call (it decides the cache policy of the read of x under set_cache_policy('auto'))."""
+    code is applied in the same pass (thn_norm_act_fwd).  `backward_follows`: whether a backward may follow
+    this call (it decides the cache policy of the read of x under set_cache_policy('auto'))."""
     done = _native.host().norm_fwd(x, weight, bias, eps, layernorm, act, _x_policy_flag(backward_follows))
     if done is not None:
         return done

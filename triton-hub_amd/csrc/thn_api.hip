@@ -419,7 +419,9 @@ int default_blocks_per_cu(int which, int flavour, int block) {
 //   24 vectors, 16-bit, a second or third round of up to a 32nd: 0.84-0.92 x and 0.92-0.98 x (257 x 164797 0.84 and 0.92 for
 //     log-softmax), 0.90-0.96 x and 0.95-0.99 x; with more than two of the 24 idle also up to a quarter of a second round
 //     (0.93-0.96 x and 0.97-0.99 x) and up to half of the compute units (128 x 164800 0.88-0.91 x and 0.96-0.97 x).  float32
-//     log-softmax, a second round of up to a 32nd: 0.88-1.00 x and 0.94-1.00 x; softmax gains 4-9 % of a pass there.
+//     log-softmax, a second round of up to a 32nd: 0.88-1.00 x and 0.94-1.00 x; softmax gains 4-9 % of a pass there.  At other
+//     counts the spills cost less than the second walk: log-softmax forward bfloat16 512 x 180000 95.9 -> 81.2 us, 1024 x 180000
+//     180 -> 167, float32 512 x 90000 89.4 -> 77.2, 3000 x 90000 497 -> 444.
 // Left as it is: float32 with 8 vectors per thread loses up to 15 % of a forward alone at other counts too (513, 769, 3000), where
 // a softmax forward + backward gains 0-5 % and a log-softmax pass loses up to 6 % or gains as much, by the rounds.
 bool wide_fwd_loses(bool is_log, int64_t M, int64_t vecs, int k, int bytes, int cus) {
