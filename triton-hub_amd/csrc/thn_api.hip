@@ -449,7 +449,7 @@ bool wide_fwd_loses(bool is_log, int64_t M, int64_t vecs, int k, int bytes, int 
 //     The log-softmax backward gains at most sizes (bfloat16 300 x 90001 45.2 -> 39.7; 16 x 32800 and 257 x 32800 0.92-0.96 x);
 //   float32 tensors that dwarf the memory-side cache, in rows of more than 6 x 1024 vectors: forward with 8 vectors per thread
 //     from 700 MiB on 0.93-1.03 x (8192 x 31997 softmax 0.94), log-softmax backward from 900 MiB on 0.95-1.01 x (8192 x 32000 541 ->
-//     553; both directions 912 -> 928), up to 1.12 x and 1.18 x below that; 16-bit rows 0.97-1.17 x and 0.98-1.17 x at any size.
+//     553; both directions 912 -> 928), up to 1.12 x and 1.18 x below that; 16-bit rows 0.97-1.17 x and 0.98-1.17 x from 2048 rows on.
 int softmax_wide_vecs(int which, bool is_log, int64_t M, int64_t N, int dtype, int cus) {
     const int bytes = elem_bytes(dtype);
     const int64_t vecs = N / (16 / bytes);
