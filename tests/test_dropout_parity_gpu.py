@@ -349,3 +349,25 @@ def test_nothing_kept_where_saved_tensors_are_managed():
     assert same_bits(torch.autograd.grad(y, x, dy)[0].cpu(), want.cpu())
     assert checkpoint(module, x, use_reentrant=False).grad_fn.mask is None
     assert module(x).grad_fn.mask is not None
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("p", [0.0123, 0.1, 0.4, 0.5, 0.7, 1 - 2.0 ** -20])
+def test_every_16_bit_value_is_divided_correctly(p, dtype):
+    """All values of the type -- subnormal numbers, infinities and NaN among them -- through the kernels with and without kept
+    decisions, for probabilities whose quotients a product gives and such that need the quotient itself (0.4 and 0.7)."""
+    announce(f"every value p={p} {dtype}")
+    values = torch.arange(1 << 16, dtype=torch.int32).to(torch.int16).view(dtype)
+    for copies in (3, 64):                              # 64: 2^22 elements, whose forward keeps its decisions
+        x = values.repeat(copies)
+        random.seed(7)
+        seed = random.randint(0, 2 ** 16)
+        random.seed(7)
+        xg = x.cuda().requires_grad_(True)
+        y = Dropout(p)(xg)
+        dx, = torch.autograd.grad(y, xg, x.cuda())
+        want = expected(x, p, seed)
+        for got in (y.detach().cpu(), dx.cpu()):
+            nan = torch.isnan(want)
+            assert torch.equal(torch.isnan(got), nan)
+            assert same_bits(got[~nan], want[~nan])

@@ -1739,6 +1739,25 @@ int act_blocks_per_cu(int act, bool bwd, int bytes) {
     return 2;
 }
 
+// thn::dropout_scale() takes 1-8 us, so each thread keeps the last few that it asked for (a function of its two arguments alone).
+float remembered_dropout_scale(float keep, int dtype) {
+    struct Entry {
+        float keep, scale;
+        int dtype;
+    };
+    constexpr unsigned kEntries = 8;
+    static thread_local Entry entries[kEntries] = {};       // keep = 0 gives 0, as the empty entries say
+    static thread_local unsigned oldest = 0;
+    if (dtype != THN_F16 && dtype != THN_BF16) return 0.0f;
+    for (const Entry& e : entries) {
+        if (e.keep == keep && (e.dtype == dtype || keep == 0.0f)) return e.scale;
+    }
+    entries[oldest] = Entry{keep, thn::dropout_scale(keep, dtype), dtype};
+    const float scale = entries[oldest].scale;
+    oldest = (oldest + 1) % kEntries;
+    return scale;
+}
+
 int dropout_launch(thn::DropoutMask mode, const void* x, void* out, uint32_t* mask, int64_t n, int64_t first_offset, float p,
                    uint64_t seed, int dtype, void* stream) {
     const int bytes = elem_bytes(dtype);
@@ -1761,6 +1780,7 @@ int dropout_launch(thn::DropoutMask mode, const void* x, void* out, uint32_t* ma
     a.key_lo = static_cast<uint32_t>(seed);
     a.key_hi = static_cast<uint32_t>(seed >> 32);
     a.threshold = thn::dropout_threshold(p);
+    a.scale = remembered_dropout_scale(1.0f - p, dtype);
     a.mask = mask;
     if (mode != thn::DropoutMask::kNone && (a.threshold == thn::kDropAll || first_offset != 0 || n > thn::kMaskedMost)) return THN_E_SHAPE;
     // Bound by integer arithmetic: as many waves as a compute unit holds (8 workgroups of 256 threads).  From a mask, by

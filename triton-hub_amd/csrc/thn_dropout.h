@@ -14,14 +14,20 @@
 //  * float32(fold(v)) * 4.6566127342e-10 < p is monotone in fold(v), so the host turns p into the number T of folded
 //    words that are dropped (dropout_threshold) and the test is one addition and one unsigned comparison: v lies in
 //    [-T, T - 1] exactly if uint32(v + T) < 2 T;
-//  * a dropped element is selected before it is scaled (0 scales to +0), which leaves no branch.
-// bfloat16 16384 x 4096 (134 MB in, 134 MB out), launches of one direction after another: 123 -> 92 us.  43.3 vector
-// instructions per element at 4.1 cycles each: the vector units issue in 93 % of the cycles in which a compute unit is busy (97 % in
-// the forward that keeps its decisions), 78 us at the 2.38 GHz of these launches.
+//  * a dropped element is selected before it is scaled (0 scales to +0), which leaves no branch;
+//  * 16-bit values are scaled by one multiplication where dropout_scale() finds a factor, instead of 3 instructions;
+//  * a forward that keeps its decisions shifts each into its word with the comparison's own mask as the carry of one
+//    addition, and takes the element's part of the first product as the addend of that multiplication.
+// bfloat16 16384 x 4096 (134 MB in, 134 MB out): a forward that keeps its decisions takes 88 us (41.5 vector instructions per
+// element, issuing in 96 % of the cycles in which a compute unit is busy; 45.1 instructions, 65 registers, which leave room for
+// 7 of the 8 workgroups per compute unit that are launched, and no decision before the first vectors had arrived: 95); with
+// its backward 132 -> 125.
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <math.h>
 #include <stdint.h>
+#include <string.h>
 #include <type_traits>
 
 #include "thn_device.h"
@@ -38,6 +44,7 @@ struct DropoutArgs {
     uint32_t key_lo, key_hi;
     uint32_t threshold;    // dropout_threshold(p)
     uint32_t* mask;        // dropout_masked_kernel: see there
+    float scale;           // dropout_scale(1 - p, type): 0 where the product would not round like the quotient
 };
 
 constexpr float kDropoutScale = 4.6566127342e-10f;
@@ -53,16 +60,55 @@ inline uint32_t dropout_threshold(float p) {
     return low;
 }
 
-// The first Philox word of counter (c0, c1, 0, 0); c1 = 0 is taken as given unless kWide.
+// A float32 r whose product x * r, rounded to float32 and then to a 16-bit type, is for every x of that type what the
+// quotient x / keep rounded the same way is; 0 if none of the three next to 1 / keep is one.  The roundings depend on
+// x's significand alone, so every one of them is tried: the normal numbers at one exponent (results only grow, keep being
+// at most 1: they stay normal, and infinity starts at the rounding boundary of the largest), the subnormal ones in units of
+// the smallest, where bfloat16 results below 128 units have been rounded to float32's subnormal grid of 2^-16 units first.
+// Found for 93 of the p = 0.01, 0.02 ... 0.99 with bfloat16, for 86 with float16.
+template <int kBits, bool kCoarse>      // significand bits with the hidden one; float32's own subnormal grid matters
+inline bool products_round_alike(float keep, float r) {
+    constexpr int kHidden = 1 << (kBits - 1), kDrop = 24 - kBits;
+    const auto narrow = [](float v) {
+        uint32_t u;
+        memcpy(&u, &v, 4);
+        return (u + (1u << (kDrop - 1)) - 1u + (u >> kDrop & 1u)) >> kDrop;
+    };
+    for (int m = kHidden; m < 2 * kHidden; ++m) {
+        const float x = static_cast<float>(m);
+        if (narrow(x / keep) != narrow(x * r)) return false;
+    }
+    const auto narrow_subnormal = [&](double exact) {
+        if (exact >= kHidden) return static_cast<double>(narrow(static_cast<float>(exact))) + 65536.0;
+        return nearbyint(kCoarse ? nearbyint(exact * 65536.0) / 65536.0 : static_cast<double>(static_cast<float>(exact)));
+    };
+    for (int m = 1; m < kHidden; ++m) {
+        if (narrow_subnormal(static_cast<double>(m) / keep) != narrow_subnormal(static_cast<double>(m) * r)) return false;
+    }
+    return true;
+}
+inline float dropout_scale(float keep, int dtype) {
+    if (!(keep > 0.0f) || (dtype != kF16 && dtype != kBF16)) return 0.0f;
+    const float r = 1.0f / keep;
+    const float candidates[3] = {r, nextafterf(r, 0.0f), nextafterf(r, 2.0f * r)};
+    for (const float c : candidates) {
+        if (dtype == kBF16 ? products_round_alike<8, true>(keep, c) : products_round_alike<11, false>(keep, c)) return c;
+    }
+    return 0.0f;
+}
+
+// The first Philox word of counter (c0, c1, 0, 0), the product of c0 and the first multiplier being given; c1 = 0 is taken
+// as given unless kWide.
+constexpr uint32_t kPhiloxM0 = 0xD2511F53u;
 template <bool kWide>
-__device__ __forceinline__ uint32_t philox_first_word(uint32_t i, uint32_t c1_in, uint32_t k0, uint32_t k1) {
-    constexpr uint32_t kM0 = 0xD2511F53u, kM1 = 0xCD9E8D57u, kW0 = 0x9E3779B9u, kW1 = 0xBB67AE85u;
+__device__ __forceinline__ uint32_t philox_first_word(uint64_t first_product, uint32_t c1_in, uint32_t k0, uint32_t k1) {
+    constexpr uint32_t kM0 = kPhiloxM0, kM1 = 0xCD9E8D57u, kW0 = 0x9E3779B9u, kW1 = 0xBB67AE85u;
     const auto product = [](uint32_t m, uint32_t c) { return static_cast<uint64_t>(m) * c; };
     const auto high = [](uint64_t p) { return static_cast<uint32_t>(p >> 32); };
     const auto low = [](uint64_t p) { return static_cast<uint32_t>(p); };
     const auto xor3 = [](uint32_t a, uint32_t b, uint32_t c) { return __builtin_amdgcn_bitop3_b32(a, b, c, 0x96); };
     // round 1: the third and fourth counter words are 0
-    uint64_t pa = product(kM0, i), pb;
+    uint64_t pa = first_product, pb;
     uint32_t c0 = kWide ? c1_in ^ k0 : k0, c1 = 0u, c2 = high(pa) ^ k1, c3 = low(pa);
     k0 += kW0;
     k1 += kW1;
@@ -107,7 +153,7 @@ __device__ __forceinline__ uint32_t philox_first_word(uint32_t i, uint32_t c1_in
 template <bool kWide>
 __device__ __forceinline__ bool is_dropped(int64_t offset, const DropoutArgs& a) {
     const uint64_t o = static_cast<uint64_t>(offset);
-    const uint32_t w = philox_first_word<kWide>(static_cast<uint32_t>(o), static_cast<uint32_t>(o >> 32), a.key_lo, a.key_hi);
+    const uint32_t w = philox_first_word<kWide>(static_cast<uint64_t>(kPhiloxM0) * static_cast<uint32_t>(o), static_cast<uint32_t>(o >> 32), a.key_lo, a.key_hi);
     return w + a.threshold < 2u * a.threshold;
 }
 
@@ -143,6 +189,22 @@ __device__ __forceinline__ float dropout_value(float x, bool dropped, const Keep
     return keep_div(kept, keep);
 }
 __device__ __forceinline__ double dropout_value(double x, bool dropped, const KeepDivisor& keep) { return keep_div(dropped ? 0.0 : x, keep); }
+template <bool kProduct, typename C> __device__ __forceinline__ C dropout_value(C x, bool dropped, const KeepDivisor& keep, float scale) {
+    if constexpr (kProduct) return (dropped ? 0.0f : x) * scale;
+    else return dropout_value(x, dropped, keep);
+}
+
+// The same with the decisions of the wave's lanes in a scalar mask.  The selection is written out: from `dropped ? 0 : x` the compiler makes
+// a second comparison, with the result inverted, beside the one that the mask comes from.
+template <bool kProduct> __device__ __forceinline__ float dropout_selected(float x, uint64_t drop, const KeepDivisor& keep, float scale) {
+    float kept;
+    asm("v_cndmask_b32_e64 %0, %1, 0, %2" : "=v"(kept) : "v"(x), "s"(drop));
+    if constexpr (kProduct) return kept * scale;
+    else return keep_div(kept, keep);
+}
+template <bool kProduct> __device__ __forceinline__ double dropout_selected(double x, uint64_t drop, const KeepDivisor& keep, float) {
+    return keep_div((drop >> __lane_id() & 1u) != 0u ? 0.0 : x, keep);
+}
 
 // the tail that does not fill a vector
 template <typename T, bool kWide>
@@ -155,7 +217,7 @@ __device__ __forceinline__ void dropout_tail(const DropoutArgs& a, const KeepDiv
     }
 }
 
-template <typename T, bool kWide>
+template <typename T, bool kWide, bool kProduct>
 __global__ void __launch_bounds__(kDropoutBlock) dropout_flat_kernel(const DropoutArgs a) {
     using C = typename std::conditional<T::kBytes == 8, double, float>::type;
     constexpr int VEC = T::VEC;
@@ -172,7 +234,7 @@ __global__ void __launch_bounds__(kDropoutBlock) dropout_flat_kernel(const Dropo
         unpack_as<T>(raw, xf);
         const int64_t e0 = a.first_offset + v * VEC;
 #pragma unroll
-        for (int e = 0; e < VEC; ++e) of[e] = dropout_value(xf[e], is_dropped<kWide>(e0 + e, a), keep);
+        for (int e = 0; e < VEC; ++e) of[e] = dropout_value<kProduct>(xf[e], is_dropped<kWide>(e0 + e, a), keep, a.scale);
         st128u(a.out + v * 16, pack_as<T, C>(of));
     }
     dropout_tail<T, kWide>(a, keep, all);
@@ -181,14 +243,14 @@ __global__ void __launch_bounds__(kDropoutBlock) dropout_flat_kernel(const Dropo
 // A forward that keeps its decisions (kRead = false) and the backward that reads them instead of drawing them again.  A
 // workgroup takes pieces of 256 x 4 vectors, thread t of it vectors t, t + 256, t + 512 and t + 768 of a piece; word t of the
 // piece's 256 words of mask holds their decisions, a byte per vector with the first in the highest byte, the first element of a
-// vector in the highest of the byte's VEC low bits.  (One byte per thread and vector cost the forward 14 us.)  The next
-// piece is requested before the present one is used, as in act_flat_kernel; slots past the end repeat the last vector, so
+// vector in the highest of the byte's VEC low bits.  (One byte per thread and vector cost the forward 14 us.)  The backward
+// requests the next piece before it uses the present one, as act_flat_kernel does, the forward, which has arithmetic to wait on, each vector
+// of it when that of the present one is stored (16 registers fewer: 8 workgroups per compute unit); slots past the end repeat the last vector, so
 // that no branch stands around a load or a store.  The threshold is below kDropAll (p < 1 in float32), the offsets of the
 // elements start at 0 and fit 32 bits.
-// bfloat16 16384 x 4096: forward 95 us (92 without a mask: two instructions per element and 8 MiB more), backward 46, which is
-// what two plain streams take (80 drawn again); both directions of a pass 174 -> 136.
-template <typename T, bool kRead>
-__global__ void __launch_bounds__(kDropoutBlock) dropout_masked_kernel(const DropoutArgs a) {
+// bfloat16 16384 x 4096: forward 88 us, backward 45, which is what two plain streams take (80 drawn again).
+template <typename T, bool kRead, bool kProduct>
+__global__ void __launch_bounds__(kDropoutBlock, kRead || T::kBytes > 2 ? 1 : 8) dropout_masked_kernel(const DropoutArgs a) {
     using C = typename std::conditional<T::kBytes == 8, double, float>::type;
     constexpr int VEC = T::VEC, U = kMaskedVecs;
     const KeepDivisor keep = make_keep_divisor(1.0f - a.p);
@@ -199,43 +261,69 @@ __global__ void __launch_bounds__(kDropoutBlock) dropout_masked_kernel(const Dro
         return v < last ? v : last;
     };
     const auto load = [&](uint32_t v) { return ld128u(a.x + static_cast<uint64_t>(v) * 16); };
+    // The first product of element e of a vector: the part of e is the addend of the multiplication.  (Kept from the compiler,
+    // which would add e to the offset first, one instruction more per element; an instruction reads one scalar operand.)
+    uint32_t m0 = kPhiloxM0;
+    uint64_t of_element[VEC];
+    asm("" : "+v"(m0));
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) {
+        of_element[e] = static_cast<uint64_t>(kPhiloxM0) * e;
+        asm("" : "+s"(of_element[e]));
+    }
     if (blockIdx.x < pieces) {
-        u32x4 cur[U], nxt[U];
+        u32x4 cur[U], nxt[kRead ? U : 1];
         uint32_t word = 0u, next_word = 0u;
 #pragma unroll
         for (int u = 0; u < U; ++u) cur[u] = load(place(blockIdx.x, u));
         if constexpr (kRead) word = a.mask[static_cast<uint64_t>(blockIdx.x * kDropoutBlock + threadIdx.x)];
-        drain_vector_memory(cur);
+        if constexpr (kRead) drain_vector_memory(cur);
         for (uint32_t piece = blockIdx.x; piece < pieces; piece += gridDim.x) {
             const uint32_t next = piece + gridDim.x < pieces ? piece + gridDim.x : piece;
+            if constexpr (kRead) {
 #pragma unroll
-            for (int u = 0; u < U; ++u) nxt[u] = load(place(next, u));
-            if constexpr (kRead) next_word = a.mask[static_cast<uint64_t>(next * kDropoutBlock + threadIdx.x)];
-            else word = 0u;
+                for (int u = 0; u < U; ++u) nxt[u] = load(place(next, u));
+                next_word = a.mask[static_cast<uint64_t>(next * kDropoutBlock + threadIdx.x)];
+            } else {
+                word = 0u;
+            }
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 const uint32_t v = place(piece, u);
-                const int64_t e0 = static_cast<int64_t>(v) * VEC;
                 C xf[VEC], of[VEC];
-                unpack_as<T>(cur[u], xf);
-                if constexpr (!kRead && VEC < 8) word <<= 8 - VEC;
+                if constexpr (kRead) {
+                    unpack_as<T>(cur[u], xf);
 #pragma unroll
-                for (int e = 0; e < VEC; ++e) {
-                    bool dropped;
-                    if constexpr (kRead) {
-                        dropped = (word >> (8 * (U - 1 - u) + VEC - 1 - e) & 1u) != 0u;
-                    } else {
-                        dropped = is_dropped<false>(e0 + e, a);
-                        word = word << 1 | (dropped ? 1u : 0u);
+                    for (int e = 0; e < VEC; ++e) {
+                        const bool dropped = (word >> (8 * (U - 1 - u) + VEC - 1 - e) & 1u) != 0u;
+                        of[e] = dropout_value<kProduct>(xf[e], dropped, keep, a.scale);
                     }
-                    of[e] = dropout_value(xf[e], dropped, keep);
+                } else {
+                    // the decisions first: nothing waits for the vector before they are made
+                    uint64_t drop[VEC];
+                    if constexpr (VEC < 8) word <<= 8 - VEC;
+#pragma unroll
+                    for (int e = 0; e < VEC; ++e) {
+                        const uint64_t first = static_cast<uint64_t>(m0) * (v * VEC) + of_element[e];
+                        const uint32_t w = philox_first_word<false>(first, 0u, a.key_lo, a.key_hi);
+                        drop[e] = __builtin_amdgcn_uicmp(w + a.threshold, 2u * a.threshold, 36);
+                        // word = 2 * word + dropped, in one instruction
+                        asm volatile("v_addc_co_u32_e64 %0, vcc, %0, %0, %1" : "+v"(word) : "s"(drop[e]) : "vcc");
+                    }
+                    pin_loaded(cur[u]);
+                    unpack_as<T>(cur[u], xf);
+#pragma unroll
+                    for (int e = 0; e < VEC; ++e) of[e] = dropout_selected<kProduct>(xf[e], drop[e], keep, a.scale);
                 }
                 st128u(a.out + static_cast<uint64_t>(v) * 16, pack_as<T, C>(of));
+                if constexpr (!kRead) cur[u] = load(place(next, u));
             }
             if constexpr (!kRead) a.mask[static_cast<uint64_t>(piece * kDropoutBlock + threadIdx.x)] = word;
+            if constexpr (kRead) {
 #pragma unroll
-            for (int u = 0; u < U; ++u) cur[u] = nxt[u];
-            word = next_word;
+                for (int u = 0; u < U; ++u) cur[u] = nxt[u];
+                word = next_word;
+            }
         }
     }
     dropout_tail<T, false>(a, keep, false);
