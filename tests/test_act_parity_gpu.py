@@ -7,6 +7,8 @@ rounding the 16-bit result inherits; float64 storage: bit-exact for the selectio
 Threshold), 1e-13 for Softplus (all computed in float64, as the reference does), the float32 bound for the
 kernels the reference widens to float32.  The backward is compared at the tensor the Function saved.
 """
+import math
+
 import numpy as np
 import pytest
 import torch
@@ -251,3 +253,27 @@ def test_c_abi_direct_calls_and_errors():
             assert torch.equal(out, ref)
     finally:
         lib.thn_norm_set_launch_override(7, 0, 0, 0, 0)
+
+
+def test_gelu_formula_in_float32():
+    """Both directions against float64 over the range where the exponential is a float32 number, and the special values.
+    exp(-x^2/2) carries the relative errors of x^2 (a product, its square: 3 roundings) times its exponent x^2/2, everything else --
+    the reciprocal, seven multiply-adds, the fit -- below 16 roundings: (16 + 2 x^2) 2^-24 of Phi (and of x*phi in the derivative)."""
+    x = torch.linspace(-13.0, 13.0, 40001, device="cuda")[1:]
+    x = torch.cat([x, torch.logspace(-20, 0, 500, device="cuda"), -torch.logspace(-20, 0, 500, device="cuda")]).requires_grad_()
+    y = A.GeLU()(x)
+    (dx,) = torch.autograd.grad(y, x, torch.ones_like(x))
+    w = x.detach().double()
+    cdf, tail = 0.5 * torch.erfc(-w * math.sqrt(0.5)), w * torch.exp(-0.5 * w * w) / math.sqrt(2.0 * math.pi)
+    bound = (16.0 + 2.0 * w * w) * 2.0 ** -24
+    # (Phi and the exponential are rounded to the spacing of denormal numbers below 2^-126, or flushed, before they meet x)
+    least = 2.0 ** -126 * (1.0 + w.abs())
+    assert bool(((y.detach().double() - w * cdf).abs() <= bound * (w * cdf).abs() + least).all())
+    assert bool(((dx.double() - (cdf + tail)).abs() <= bound * (cdf + tail.abs()) + least).all())
+
+    special = torch.tensor([0.0, -0.0, 3e38, -3e38, math.inf, -math.inf, math.nan], device="cuda", requires_grad=True)
+    y = A.GeLU()(special)
+    (dx,) = torch.autograd.grad(y, special, torch.ones_like(special))
+    assert y[:5].tolist() == [0.0, 0.0, special[2].item(), 0.0, math.inf] and bool(y[5:].isnan().all())
+    # (at zero the bound above, of Phi = 0.5)
+    assert bool(((dx[:2] - 0.5).abs() <= 8.0 * 2.0 ** -24).all()) and dx[2:4].tolist() == [1.0, 0.0] and bool(dx[4:].isnan().all())

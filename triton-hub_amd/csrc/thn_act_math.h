@@ -46,53 +46,44 @@ __device__ __forceinline__ GateParts gelu_tanh_gate_parts(float x) {
 }
 __device__ __forceinline__ float gelu_tanh_gate(float x) { return gelu_tanh_gate_parts(x).gate; }
 
-// Phi(x) = 0.5*(1 + erf(x/sqrt 2)), the normal distribution function of GeLU, from the complementary error function
-// of z = |x|/sqrt 2, in two forms that work with t = 1/(1 + z/2) in (0, 1].  Both are branch free, accurate in the
-// negative tail (where 1 + erf(..) cancels) and a third of the instructions of the library erff.  Their
-// exponentials are base 2 (the hardware's v_exp_f32), so they work on a = z*sqrt(log2 e), a^2 = z^2*log2(e), and the
-// factor 1/2 of Phi is folded into the coefficients.
-//
-// Backward form: erfc(z)/2 = t*Q(t)*exp(-z^2), Q of degree 8: a minimax fit of the relative error over z in [0, 9.3], behind
-// which the exponential underflows (5.1e-8 with the coefficients as stored; degree 7 gives 3e-7).  Its exponential is exp(-x^2/2), the one the normal
-// density needs: GeLU' = Phi(x) + x*phi(x) is 1 + r for x >= 0 and -r for x < 0 with r = exp(-x^2/2)*(|x|/sqrt(2 pi) - t*Q(t)).
-// Three instructions per element fewer than Q of degree 10 with Phi and phi put together afterwards, and closer to float64
-// (GeLU' in float32, x = 1.5 g + 0.25 with g normal, relative 2-norm: 4.47e-8 against 4.75e-8): LayerNorm + GeLU backward bfloat16
-// 16384 x 4096, which is bound by arithmetic, 97.4 -> 92.9 us together with one instruction less for the corrected xhat.
-__device__ __forceinline__ float gelu_slope(float x) {
-    const float a = __builtin_fabsf(x) * 0.84932180028801907f;
-    const float t = rcp_fast(__builtin_fmaf(0.35355339059327379f, __builtin_fabsf(x), 1.0f));
-    float q = -0.02940019778907299f;
-    q = __builtin_fmaf(q, t, 0.1416291743516922f);
-    q = __builtin_fmaf(q, t, -0.2422293722629547f);
-    q = __builtin_fmaf(q, t, 0.13745570182800293f);
-    q = __builtin_fmaf(q, t, -0.012217934243381023f);
-    q = __builtin_fmaf(q, t, 0.10087623447179794f);
-    q = __builtin_fmaf(q, t, 0.12167113274335861f);
-    q = __builtin_fmaf(q, t, 0.14117106795310974f);
-    q = __builtin_fmaf(q, t, 0.14104416966438293f);
-    const float r = __builtin_amdgcn_exp2f(-a * a) * __builtin_fmaf(0.39894228040143267794f, __builtin_fabsf(x), -(t * q));
-    return x < 0.0f ? -r : 1.0f + r;
+// GeLU from the normal distribution function Phi(x) = 0.5*(1 + erf(x/sqrt 2)).  With t = 1/(1 + c|x|) in (0, 1] both directions
+// take Phi(-|x|) = t*Q(t)*exp(-x^2/2), Q a polynomial of degree 7: branch free, accurate in the negative tail (where
+// 1 + erf(..) cancels), a third of the instructions of the library erff.  c is free and sets how fast such a fit converges: at
+// the c below degree 7 reaches what took degree 9 and 8 at c = 0.35.  The sign of x rides on t, t_s = 1/(sgn + c*x) (|t| is a
+// modifier of the polynomial's instructions, no instruction), and step = max(sgn, 0), so that one multiply-add takes the place
+// of a comparison, a subtraction and a selection:
+//   Phi(x) = step - t_s*Q*exp(-x^2/2),   GeLU'(x) = Phi(x) + x*phi(x) = step + exp(-x^2/2)*(x/sqrt(2 pi) - t_s*Q).
+// The exponential is base 2 (the hardware's v_exp_f32), of a^2 with a = x*sqrt(log2(e)/2).  19 instruction slots per element
+// forward and 20 backward (a transcendental counts as 2) instead of 21 and 22; against float64 (2-norm, x = 1.5 g + 0.25 with g normal)
+// 3.29e-8 and 4.26e-8 instead of 3.32e-8 and 4.46e-8, and no larger for g alone, for the negative tail and for |x| < 6.
+// Forward + backward bfloat16 16384 x 4096: GeLU 110.0 -> 108.8 us, LayerNorm + GeLU 146.5 -> 140.8.
+struct NormalParts {
+    float tq, e, step;      // t_s*Q(t), exp(-x^2/2), x < 0 ? 0 : 1
+};
+template <int DEGREE>
+__device__ __forceinline__ NormalParts normal_parts(float x, float c, const float (&coefficients)[DEGREE + 1]) {
+    const float sgn = __builtin_copysignf(1.0f, x);
+    const float t = rcp_fast(__builtin_fmaf(c, x, sgn));
+    const float a = x * 0.84932180028801907f;
+    float q = coefficients[DEGREE];
+#pragma unroll
+    for (int i = DEGREE - 1; i >= 0; --i) q = __builtin_fmaf(q, __builtin_fabsf(t), coefficients[i]);
+    return NormalParts{t * q, __builtin_amdgcn_exp2f(-a * a), sgn > 0.0f ? sgn : 0.0f};
 }
 
-// Forward form: erfc(z)/2 = t*exp(-z^2 + P(t) - ln 2) (the Chebyshev fit of Numerical Recipes 6.2, relative error
-// below 1.5e-7 for every z with the coefficients scaled to base 2): one multiplication fewer than the product form,
-// which measured 1-6 % slower in the forward kernels (again with a degree-8 polynomial R(t) for t*Q(t), one instruction
-// fewer than this: LayerNorm + GeLU forward bfloat16 16384 x 4096 66.4 -> 68.5 us).
+// Minimax fit of the relative error of Phi(-|x|) (x in [0, 13.3], behind which the exponential underflows): 8.3e-8.
 __device__ __forceinline__ float normal_cdf(float x) {
-    const float a = __builtin_fabsf(x) * 0.84932180028801907f;
-    const float t = rcp_fast(__builtin_fmaf(0.41627730557884884f, a, 1.0f));
-    float p = 0.2465173f;
-    p = __builtin_fmaf(p, t, -1.1861149f);
-    p = __builtin_fmaf(p, t, 2.1474745f);
-    p = __builtin_fmaf(p, t, -1.6377531f);
-    p = __builtin_fmaf(p, t, 0.40232158f);
-    p = __builtin_fmaf(p, t, -0.26875687f);
-    p = __builtin_fmaf(p, t, 0.13963005f);
-    p = __builtin_fmaf(p, t, 0.5397006f);
-    p = __builtin_fmaf(p, t, 1.4427292f);
-    p = __builtin_fmaf(p, t, -2.8257482f);
-    const float half_erfc = t * __builtin_amdgcn_exp2f(__builtin_fmaf(-a, a, p));
-    return x < 0.0f ? half_erfc : 1.0f - half_erfc;
+    const NormalParts p = normal_parts<7>(x, 0.3036f, {0.12107304f, 0.12204604f, 0.1020654f, 0.12441437f, -0.044881325f,
+                                                       0.19440602f, -0.15598506f, 0.036861554f});
+    return __builtin_fmaf(-p.tq, p.e, p.step);
+}
+
+// Minimax fit of the error relative to |x|/sqrt(2 pi) + t*Q, which is what GeLU' is made of: 2.3e-8.  (c = 0.385 to 0.41 measure
+// alike; beyond 0.415 the fit is worse than degree 8 at 0.354 was.)
+__device__ __forceinline__ float gelu_slope(float x) {
+    const NormalParts p = normal_parts<7>(x, 0.401f, {0.16005206f, 0.15829173f, 0.14927879f, 0.011608556f, 0.21302079f,
+                                                      -0.34127876f, 0.18568613f, -0.036659308f});
+    return __builtin_fmaf(p.e, __builtin_fmaf(0.39894228040143267794f, x, -p.tq), p.step);
 }
 
 // Mish needs t = tanh(softplus(x)) with softplus(x) = x > 20 ? x : log(1 + e^x) (mish.py:19-22).  With w = e^x and

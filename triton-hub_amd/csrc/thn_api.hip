@@ -404,7 +404,7 @@ int default_blocks_per_cu(int which, int flavour, int block) {
     if (which >= kPnormFwd && which <= kNormalizeBwd && block <= 256) return 2;
     // A GeLU epilogue makes the norm kernels arithmetic-bound (about 30 instruction slots per element): they take
     // as many workgroups per compute unit as their registers allow, up to four.
-    if ((which == kFusedFwd || which == kFusedBwd) && ((flavour >> 1) == thn::kGelu || (flavour >> 1) == thn::kGeluTanh)) return 4;
+    if ((which == kFusedFwd || which == kFusedBwd) && thn::arithmetic_bound(flavour >> 1)) return 4;
     return kDefaultBlocksPerCu;
 }
 
