@@ -3,10 +3,13 @@ and 4 vectors and rows of up to 32 vectors whose vector count is not a power of 
 4 rows per lane forced through the launch override (and once by the library's own choice), against the CPU oracle; row
 counts that end in the middle of a wave, a workgroup and a grid step; masked (-inf) logits; rows that are column blocks
 of a wider buffer; run-to-run identical results."""
+import math
+
 import pytest
 import torch
 
 import test_softmax_parity_gpu as sm
+from TritonHub import Activations as A
 from TritonHub import _native
 
 pytestmark = pytest.mark.gpu
@@ -115,3 +118,39 @@ def test_default_choice_masked_logits_strided_rows_and_determinism():
     gb = torch.randn(777, 128, generator=g).half()
     sm.run_and_compare("softmin", xb[:, :88].contiguous(), gb[:, :88].contiguous(), "flat strided f16 777 x 88",
                        x_gpu=xb.cuda()[:, :88].detach(), dy_gpu=gb.cuda()[:, :88])
+
+
+@pytest.mark.parametrize("vecs,ragged", [(17, 0), (17, -3), (21, 0), (25, -3), (31, -1), (31, 0), (32, -1), (32, -3)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_rows_of_17_to_32_vectors_do_not_meet(dtype, vecs, ragged):
+    """Rows of one wave share its lanes: a row's bits do not depend on its neighbours, whatever they hold (32 vectors leave no idle
+    lane for the sums to read), on the row count (a single row, partial steps, several steps of a workgroup) or on the distance
+    between rows."""
+    vec = 16 // torch.empty(0, dtype=dtype).element_size()
+    n = vecs * vec + ragged
+    rows = 40000
+    g = torch.Generator(device="cuda").manual_seed(n)
+    x = torch.randn(rows, n, device="cuda", generator=g).mul_(3).to(dtype)
+    want = {fn: fn()(x) for fn in (A.Softmax, A.Softmin, A.LogSoftmax)}
+    exact = torch.softmax(x.double(), -1)
+    # exp of a difference of up to 30: 30 roundings of 2^-24 for the argument and as many for the sum, and the storage type's own
+    step = torch.finfo(dtype).eps
+    assert bool(((want[A.Softmax].double() - exact).abs() <= exact * (step + 64 * 2.0 ** -24) + 1e-38).all())
+    wild = x.clone()
+    for first, value in ((1, math.nan), (3, math.inf), (5, -math.inf), (7, torch.finfo(dtype).min), (9, torch.finfo(dtype).max)):
+        wild[first::16] = value
+    calm = torch.ones(rows, dtype=torch.bool, device="cuda")
+    for first in (1, 3, 5, 7, 9):
+        calm[first::16] = False
+    padded = torch.zeros(rows, n + 5 * vec, device="cuda", dtype=dtype)
+    padded[:, :n] = x
+    for fn, y in want.items():
+        out = fn()(wild)
+        assert torch.equal(out[calm], y[calm])
+        assert bool(out[1::16].isnan().all()) and bool(out[5::16].isnan().all())
+        flat = 1.0 / n if fn is not A.LogSoftmax else -math.log(n)
+        for first in (7, 9):
+            assert bool(((out[first::16].double() - flat).abs() <= abs(flat) * (step + 64 * 2.0 ** -24)).all())
+        assert torch.equal(fn()(padded[:, :n]), y)
+        for m in (1, 2, 3, 8, 9, 1025):
+            assert torch.equal(fn()(x[:m].contiguous()), y[:m])

@@ -118,6 +118,143 @@ __global__ void __launch_bounds__(kFlatBlock) softmax_flat_fwd_kernel(const Soft
     }
 }
 
+// The tree of segment_allreduce_op for values that are ready to be read by any lane: where that one selects after the read,
+// the lane to read from is chosen once, in front of the row loop.  A lane with nothing to take reads itself for a maximum and, for
+// a sum, the wave's last lane, which is outside every segment and holds 0 when L does not divide 64; for L that do, the
+// sum selects.
+template <int LOG> struct FlatTree {
+    int max_from[LOG > 0 ? LOG : 1], sum_from[LOG > 0 ? LOG : 1];       // byte addresses of ds_bpermute
+    bool idle;
+    __device__ __forceinline__ FlatTree(int lane, int pos, int L) : idle(64 % L != 0) {
+#pragma unroll
+        for (int s = 0; s < LOG; ++s) {
+            const bool take = pos + (1 << s) < L;
+            max_from[s] = (take ? lane + (1 << s) : lane) * 4;
+            sum_from[s] = (take ? lane + (1 << s) : 63) * 4;
+        }
+    }
+    template <typename Op, int NV>
+    __device__ __forceinline__ static void reduce(float (&v)[NV], const int (&from)[LOG > 0 ? LOG : 1], int first) {
+#pragma unroll
+        for (int s = 0; s < LOG; ++s) {
+#pragma unroll
+            for (int i = 0; i < NV; ++i) v[i] = Op::apply(v[i], as_f32(static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(from[s], static_cast<int>(as_u32(v[i]))))));
+        }
+#pragma unroll
+        for (int i = 0; i < NV; ++i) v[i] = lane_read(v[i], first);
+    }
+    template <int NV> __device__ __forceinline__ void max(float (&v)[NV], int first) const { reduce<OpMax>(v, max_from, first); }
+    template <int NV> __device__ __forceinline__ void sum(float (&v)[NV], int lane, int pos, int L, int first) const {
+        if (idle) reduce<OpSum>(v, sum_from, first);
+        else segment_allreduce_op<LOG, NV, OpSum>(v, lane, pos, L, first);
+    }
+};
+
+// Where a lane's vector of its row is, from one step to the next.  An address moves by the same distance every step and stops at
+// the last row's: an addition, a comparison and two selections, where row * stride took three products, which run at a quarter
+// of the rate.  (Strides are at least a row and M rows lie in memory, so the sum cannot wrap; a single row's stride, which
+// nothing bounds, does not count.)
+template <typename P> struct FlatWalk {
+    P at, last;
+    int64_t step;
+    FlatWalk() = default;
+    __device__ __forceinline__ FlatWalk(P base, int64_t stride, int64_t row, int64_t last_row, int64_t rows_per_iter, int voff)
+        : at(base + (row < last_row ? row : last_row) * stride + voff), last(base + last_row * stride + voff),
+          step(last_row > 0 ? rows_per_iter * stride : 0) {}
+    __device__ __forceinline__ void advance() {
+        const P next = at + step;
+        at = next < last ? next : last;
+    }
+};
+
+// The forward over rows of 17 to 32 vectors: 206 instruction slots per wave and step of two rows per lane (bfloat16, off the
+// 128-bit path) instead of 310, of which 52 went into addresses, 20 into selections around the reductions and 16 into the
+// columns that two windows share.  The vector units had been busy for 19 us of a forward of 24.5 (768 x 197 x 197), with as much memory
+// time: 24.3 -> 23.0 us, rows of 250 columns 46.8 -> 45.9 and of 100 in float32 44.2 -> 43.8 (2^26 and 2^25 elements).  Same bits.  Rows
+// of up to 16 vectors stay with the kernel above: there memory bounds it, and this one, which requests its vectors closer together, is
+// slower at most widths (bfloat16 N = 32 41.8 -> 44.0, 72 43.6 -> 44.3, 127 44.6 -> 46.0; with two or four workgroups per compute
+// unit instead of its best, three, up to 57.4).  So is the backward (197 columns 67.7 -> 68.2, 127 72.3 -> 75.1).
+template <typename T, bool LOGSM, int J, bool ALIGNED>
+__global__ void __launch_bounds__(kFlatBlock) softmax_flat_fwd_kernel_17_to_32(const SoftmaxFwdArgs a) {
+    constexpr int VEC = T::VEC;
+    constexpr int W = kFlatBlock / 64;
+    const int L = a.n_vecs;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int rpw = 64 / L;
+    const FlatLane f = flat_lane(lane, L);
+    int voff, lead;
+    flat_slot<T, ALIGNED>(f.t, L, a.n_cols, voff, lead);
+    const float neg_inf = OpMax::identity<float>();
+    // softmin: the sign bits are flipped on the packed vectors
+    const uint32_t flip = a.sign < 0.0f ? (T::kBytes == 2 ? 0x80008000u : 0x80000000u) : 0u;
+    const FlatTree<5> tree(lane, f.pos, L);
+    float counts[VEC];          // an overlapping window's leading columns count in the slot before
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) counts[e] = e >= lead ? 1.0f : 0.0f;
+
+    const int64_t rows_per_block = static_cast<int64_t>(W) * rpw * J;
+    const int64_t rows_per_iter = static_cast<int64_t>(gridDim.x) * rows_per_block;
+    const int64_t last_row = a.M - 1;
+    const int64_t row0 = static_cast<int64_t>(blockIdx.x) * rows_per_block + static_cast<int64_t>(wave) * rpw + f.r;
+    FlatWalk<const char*> x[J];
+    FlatWalk<char*> y[J];
+    u32x4 cur[J];
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+        x[j] = FlatWalk<const char*>(a.x, a.x_stride_bytes, row0 + static_cast<int64_t>(j * W) * rpw, last_row, rows_per_iter, voff);
+        y[j] = FlatWalk<char*>(a.y, a.y_stride_bytes, row0 + static_cast<int64_t>(j * W) * rpw, last_row, rows_per_iter, voff);
+        cur[j] = slot_load<T, ALIGNED>(x[j].at, 0, a.n_cols);
+    }
+    drain_vector_memory(cur);
+
+    for (int64_t base = static_cast<int64_t>(blockIdx.x) * rows_per_block; base < a.M; base += rows_per_iter) {
+        u32x4 nxt[J];
+#pragma unroll
+        for (int j = 0; j < J; ++j) {
+            x[j].advance();
+            nxt[j] = slot_load<T, ALIGNED>(x[j].at, 0, a.n_cols);
+        }
+        float xf[J][VEC];
+        float m[J];
+#pragma unroll
+        for (int j = 0; j < J; ++j) {
+            cur[j] ^= flip;
+            T::unpack(cur[j], xf[j]);
+            float mj = neg_inf;
+#pragma unroll
+            for (int e = 0; e < VEC; ++e) mj = fmaxf(mj, xf[j][e]);          // mirror lanes and overlapping windows repeat real columns: harmless for a maximum
+            m[j] = mj;
+        }
+        tree.max(m, f.first);
+        float s[J];
+#pragma unroll
+        for (int j = 0; j < J; ++j) {
+            float sk = 0.0f;
+#pragma unroll
+            for (int e = 0; e < VEC; ++e) {
+                const float z = xf[j][e] - m[j];
+                const float ez = exp_c(z);
+                xf[j][e] = LOGSM ? z : ez;
+                // (ez is at most 1, or a NaN that the whole row gets)
+                sk = ALIGNED ? sk + ez : fmaf(ez, counts[e], sk);
+            }
+            s[j] = f.own ? sk : 0.0f;
+        }
+        tree.sum(s, lane, f.pos, L, f.first);
+#pragma unroll
+        for (int j = 0; j < J; ++j) {
+            const float scale = LOGSM ? logf(s[j]) : 1.0f / s[j];
+            float yf[VEC];
+#pragma unroll
+            for (int e = 0; e < VEC; ++e) yf[e] = LOGSM ? xf[j][e] - scale : xf[j][e] * scale;
+            slot_store<T, ALIGNED, true>(y[j].at, 0, a.n_cols, yf);   // the backward works from the saved y
+            y[j].advance();
+        }
+#pragma unroll
+        for (int j = 0; j < J; ++j) cur[j] = nxt[j];
+    }
+}
+
 template <typename T, bool LOGSM, int J, int LOG, bool ALIGNED>
 __global__ void __launch_bounds__(kFlatBlock) softmax_flat_bwd_kernel(const SoftmaxBwdArgs a) {
     constexpr int VEC = T::VEC;
@@ -191,6 +328,12 @@ __global__ void __launch_bounds__(kFlatBlock) softmax_flat_bwd_kernel(const Soft
     }
 }
 
+// log_steps = 5 is what rows of 17 to 32 vectors have.
+template <typename T, bool LOGSM, int J, int LOG, bool ALIGNED> constexpr auto softmax_flat_fwd() {
+    if constexpr (LOG == 5) return &softmax_flat_fwd_kernel_17_to_32<T, LOGSM, J, ALIGNED>;
+    else return &softmax_flat_fwd_kernel<T, LOGSM, J, LOG, ALIGNED>;
+}
+
 // Launchers: 0 launched, 1 no such instance, <0 HIP error.  `log_steps`: tree steps of the segmented reductions (0 for
 // rows of one vector, 2 up to 4 vectors, 4 up to 16, 5 up to 32); `rows_each` = J.
 #define THN_DECLARE_SOFTMAX_FLAT_LAUNCHERS(NAME)                                                                \
@@ -208,9 +351,14 @@ THN_DECLARE_SOFTMAX_FLAT_LAUNCHERS(bf16)
         return is_log ? run_kernel<ARGS_T>(KERNEL<T, true, J_, LOG_, AL>, a, grid, kFlatBlock, st, nullptr)      \
                       : run_kernel<ARGS_T>(KERNEL<T, false, J_, LOG_, AL>, a, grid, kFlatBlock, st, nullptr);    \
     }
-#define THN_SOFTMAX_FLAT_FWD_AL(J_, LOG_) THN_SOFTMAX_FLAT_CASE(softmax_flat_fwd_kernel, SoftmaxFwdArgs, true, J_, LOG_)
+#define THN_SOFTMAX_FLAT_FWD_CASE(AL, J_, LOG_)                                                                 \
+    if (rows_each == J_ && log_steps == LOG_) {                                                                 \
+        return is_log ? run_kernel<SoftmaxFwdArgs>(softmax_flat_fwd<T, true, J_, LOG_, AL>(), a, grid, kFlatBlock, st, nullptr)      \
+                      : run_kernel<SoftmaxFwdArgs>(softmax_flat_fwd<T, false, J_, LOG_, AL>(), a, grid, kFlatBlock, st, nullptr);    \
+    }
+#define THN_SOFTMAX_FLAT_FWD_AL(J_, LOG_) THN_SOFTMAX_FLAT_FWD_CASE(true, J_, LOG_)
 #define THN_SOFTMAX_FLAT_BWD_AL(J_, LOG_) THN_SOFTMAX_FLAT_CASE(softmax_flat_bwd_kernel, SoftmaxBwdArgs, true, J_, LOG_)
-#define THN_SOFTMAX_FLAT_FWD_SC(J_, LOG_) THN_SOFTMAX_FLAT_CASE(softmax_flat_fwd_kernel, SoftmaxFwdArgs, false, J_, LOG_)
+#define THN_SOFTMAX_FLAT_FWD_SC(J_, LOG_) THN_SOFTMAX_FLAT_FWD_CASE(false, J_, LOG_)
 #define THN_SOFTMAX_FLAT_BWD_SC(J_, LOG_) THN_SOFTMAX_FLAT_CASE(softmax_flat_bwd_kernel, SoftmaxBwdArgs, false, J_, LOG_)
 // X(J, LOG): rows per lane and step x tree steps
 #define THN_SOFTMAX_FLAT_SHAPES(X) X(2, 0) X(4, 0) X(2, 2) X(4, 2) X(2, 4) X(4, 4) X(2, 5) X(4, 5)
