@@ -199,11 +199,11 @@ constexpr RowForm bwd_form() {
     return RowForm{true, !LN, true};     // K = 3, 4: rows of more than 32 KiB
 }
 
-// Epilogues that make the norm kernels arithmetic-bound: vector instructions issue in 85 % of a LayerNorm + GeLU forward's time and
-// 81 % of its backward's (950 and 630 slots of 4 cycles per wave and row).  Two attempts to fill the rest measured slower, forward + backward bfloat16
-// 16384 x 4096 against 139.8 us: requesting the next row into the registers of the present one, once that is unpacked (no copies,
-// 16 and 8 instructions per row fewer) 141.3 to 143.1; w and b in LDS, which makes room for four waves per SIMD instead of three and two
-// 143.2 -- under a profiler, with pauses between the launches, the latter's backward is 7 % faster: back to back the clock falls.
+// Epilogues that make the norm kernels arithmetic-bound: vector instructions issue in 98 % of the busy cycles of a LayerNorm + GeLU
+// forward and in 91 % of its backward's (bfloat16 16384 x 4096, 28.1 and 37.6 per element).  Two attempts to fill the rest measured slower, forward + backward
+// against 139.8 us: requesting the next row into the registers of the present one, once that is unpacked (no copies,
+// 16 and 8 instructions per row fewer) 141.3 to 143.1; w and b in LDS, which makes room for four waves per SIMD instead of three and two,
+// 143.2.  Under a profiler, with pauses between the launches, the latter's backward is 7 % faster: back to back the clock falls.
 constexpr bool arithmetic_bound(int act) { return act == kGelu || act == kGeluTanh; }
 
 // Makes the compiler forget what it has derived from the packed vectors, so that the next pass really
