@@ -194,16 +194,23 @@ template <bool kProduct, typename C> __device__ __forceinline__ C dropout_value(
     else return dropout_value(x, dropped, keep);
 }
 
-// The same with the decisions of the wave's lanes in a scalar mask.  The selection is written out: from `dropped ? 0 : x` the compiler makes
-// a second comparison, with the result inverted, beside the one that the mask comes from.
-template <bool kProduct> __device__ __forceinline__ float dropout_selected(float x, uint64_t drop, const KeepDivisor& keep, float scale) {
-    float kept;
-    asm("v_cndmask_b32_e64 %0, %1, 0, %2" : "=v"(kept) : "v"(x), "s"(drop));
-    if constexpr (kProduct) return kept * scale;
-    else return keep_div(kept, keep);
-}
-template <bool kProduct> __device__ __forceinline__ double dropout_selected(double x, uint64_t drop, const KeepDivisor& keep, float) {
-    return keep_div((drop >> __lane_id() & 1u) != 0u ? 0.0 : x, keep);
+// word = 2^VEC * word + the decisions of a vector, whose lanes' bits the scalar masks hold: an addition with carry each.  A vector
+// instruction needs two wait states behind the comparison that writes the scalar mask it reads; the compiler, which
+// sees to that for its own instructions, does not look into an asm block, so the block begins with them.  The masks go
+// through it: what reads them afterwards reads them behind those wait states too.
+template <int VEC> __device__ __forceinline__ void shift_in_decisions(uint32_t& word, uint64_t (&drop)[VEC]) {
+    static_assert(VEC == 2 || VEC == 4 || VEC == 8);
+#define THN_SHIFT_IN(MASK) "\n\tv_addc_co_u32_e64 %0, vcc, %0, %0, %" #MASK
+    if constexpr (VEC == 2) {
+        asm("s_nop 1" THN_SHIFT_IN(1) THN_SHIFT_IN(2) : "+v"(word), "+s"(drop[0]), "+s"(drop[1]) : : "vcc");
+    } else if constexpr (VEC == 4) {
+        asm("s_nop 1" THN_SHIFT_IN(1) THN_SHIFT_IN(2) THN_SHIFT_IN(3) THN_SHIFT_IN(4)
+            : "+v"(word), "+s"(drop[0]), "+s"(drop[1]), "+s"(drop[2]), "+s"(drop[3]) : : "vcc");
+    } else {
+        asm("s_nop 1" THN_SHIFT_IN(1) THN_SHIFT_IN(2) THN_SHIFT_IN(3) THN_SHIFT_IN(4) THN_SHIFT_IN(5) THN_SHIFT_IN(6) THN_SHIFT_IN(7) THN_SHIFT_IN(8)
+            : "+v"(word), "+s"(drop[0]), "+s"(drop[1]), "+s"(drop[2]), "+s"(drop[3]), "+s"(drop[4]), "+s"(drop[5]), "+s"(drop[6]), "+s"(drop[7]) : : "vcc");
+    }
+#undef THN_SHIFT_IN
 }
 
 // the tail that does not fill a vector
@@ -307,13 +314,13 @@ __global__ void __launch_bounds__(kDropoutBlock, kRead || T::kBytes > 2 ? 1 : 8)
                         const uint64_t first = static_cast<uint64_t>(m0) * (v * VEC) + of_element[e];
                         const uint32_t w = philox_first_word<false>(first, 0u, a.key_lo, a.key_hi);
                         drop[e] = __builtin_amdgcn_uicmp(w + a.threshold, 2u * a.threshold, 36);
-                        // word = 2 * word + dropped, in one instruction
-                        asm volatile("v_addc_co_u32_e64 %0, vcc, %0, %0, %1" : "+v"(word) : "s"(drop[e]) : "vcc");
                     }
+                    shift_in_decisions(word, drop);
                     pin_loaded(cur[u]);
                     unpack_as<T>(cur[u], xf);
+                    // (the mask as the condition: from the comparison itself the compiler would make a second one, inverted)
 #pragma unroll
-                    for (int e = 0; e < VEC; ++e) of[e] = dropout_selected<kProduct>(xf[e], drop[e], keep, a.scale);
+                    for (int e = 0; e < VEC; ++e) of[e] = dropout_value<kProduct>(xf[e], __builtin_amdgcn_inverse_ballot_w64(drop[e]), keep, a.scale);
                 }
                 st128u(a.out + static_cast<uint64_t>(v) * 16, pack_as<T, C>(of));
                 if constexpr (!kRead) cur[u] = load(place(next, u));
