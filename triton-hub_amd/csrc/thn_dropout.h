@@ -250,9 +250,11 @@ __global__ void __launch_bounds__(kDropoutBlock) dropout_flat_kernel(const Dropo
 // A forward that keeps its decisions (kRead = false) and the backward that reads them instead of drawing them again.  A
 // workgroup takes pieces of 256 x 4 vectors, thread t of it vectors t, t + 256, t + 512 and t + 768 of a piece; word t of the
 // piece's 256 words of mask holds their decisions, a byte per vector with the first in the highest byte, the first element of a
-// vector in the highest of the byte's VEC low bits.  (One byte per thread and vector cost the forward 14 us.)  The backward
-// requests the next piece before it uses the present one, as act_flat_kernel does, the forward, which has arithmetic to wait on, each vector
-// of it when that of the present one is stored (16 registers fewer: 8 workgroups per compute unit); slots past the end repeat the last vector, so
+// vector in the highest of the byte's VEC low bits.  (One byte per thread and vector cost the forward 14 us.)  The next piece is
+// requested before the present one is used, as act_flat_kernel does (kAhead), except by the forward over 16-bit values, whose 8 Philox
+// blocks per vector are arithmetic enough to wait on: it requests each vector of the next piece when that of the present one is
+// stored (16 registers fewer: 8 workgroups per compute unit).  float32 and float64, with 4 and 2 blocks per vector, lose by that
+// (forward of 2^24 float64 49.5 us against 48.4, 2^23 float32 15.3 against 14.7).  Slots past the end repeat the last vector, so
 // that no branch stands around a load or a store.  The threshold is below kDropAll (p < 1 in float32), the offsets of the
 // elements start at 0 and fit 32 bits.
 // bfloat16 16384 x 4096: forward 88 us, backward 45, which is what two plain streams take (80 drawn again).
@@ -260,6 +262,7 @@ template <typename T, bool kRead, bool kProduct>
 __global__ void __launch_bounds__(kDropoutBlock, kRead || T::kBytes > 2 ? 1 : 8) dropout_masked_kernel(const DropoutArgs a) {
     using C = typename std::conditional<T::kBytes == 8, double, float>::type;
     constexpr int VEC = T::VEC, U = kMaskedVecs;
+    constexpr bool kAhead = kRead || T::kBytes > 2;
     const KeepDivisor keep = make_keep_divisor(1.0f - a.p);
     const uint32_t pieces = static_cast<uint32_t>((a.total_vecs + kDropoutBlock * U - 1) / (kDropoutBlock * U));
     const uint32_t last = static_cast<uint32_t>(a.total_vecs - 1);
@@ -279,21 +282,20 @@ __global__ void __launch_bounds__(kDropoutBlock, kRead || T::kBytes > 2 ? 1 : 8)
         asm("" : "+s"(of_element[e]));
     }
     if (blockIdx.x < pieces) {
-        u32x4 cur[U], nxt[kRead ? U : 1];
+        u32x4 cur[U], nxt[kAhead ? U : 1];
         uint32_t word = 0u, next_word = 0u;
 #pragma unroll
         for (int u = 0; u < U; ++u) cur[u] = load(place(blockIdx.x, u));
         if constexpr (kRead) word = a.mask[static_cast<uint64_t>(blockIdx.x * kDropoutBlock + threadIdx.x)];
-        if constexpr (kRead) drain_vector_memory(cur);
+        if constexpr (kAhead) drain_vector_memory(cur);
         for (uint32_t piece = blockIdx.x; piece < pieces; piece += gridDim.x) {
             const uint32_t next = piece + gridDim.x < pieces ? piece + gridDim.x : piece;
-            if constexpr (kRead) {
+            if constexpr (kAhead) {
 #pragma unroll
                 for (int u = 0; u < U; ++u) nxt[u] = load(place(next, u));
-                next_word = a.mask[static_cast<uint64_t>(next * kDropoutBlock + threadIdx.x)];
-            } else {
-                word = 0u;
             }
+            if constexpr (kRead) next_word = a.mask[static_cast<uint64_t>(next * kDropoutBlock + threadIdx.x)];
+            else word = 0u;
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 const uint32_t v = place(piece, u);
@@ -323,14 +325,14 @@ __global__ void __launch_bounds__(kDropoutBlock, kRead || T::kBytes > 2 ? 1 : 8)
                     for (int e = 0; e < VEC; ++e) of[e] = dropout_value<kProduct>(xf[e], __builtin_amdgcn_inverse_ballot_w64(drop[e]), keep, a.scale);
                 }
                 st128u(a.out + static_cast<uint64_t>(v) * 16, pack_as<T, C>(of));
-                if constexpr (!kRead) cur[u] = load(place(next, u));
+                if constexpr (!kAhead) cur[u] = load(place(next, u));
             }
             if constexpr (!kRead) a.mask[static_cast<uint64_t>(piece * kDropoutBlock + threadIdx.x)] = word;
-            if constexpr (kRead) {
+            if constexpr (kAhead) {
 #pragma unroll
                 for (int u = 0; u < U; ++u) cur[u] = nxt[u];
-                word = next_word;
             }
+            if constexpr (kRead) word = next_word;
         }
     }
     dropout_tail<T, false>(a, keep, false);
