@@ -268,3 +268,12 @@ def test_frozen_bias_of_another_dtype_without_weight():
     x64 = f64(x); z, mean, rstd = no.layernorm_fwd(x64, None, f64(bias), 1e-5)
     dx_ref, _, _ = no.layernorm_bwd(x64, ao.bwd("gelu", z, f64(dy)), None, mean, rstd, has_bias=False)
     assert np.abs(f64(outs[1][1]) - dx_ref).max() < 0.02                    # bf16 dx of O(1) values: 2-3 ulp at most
+
+
+@pytest.mark.parametrize("n", [4098, 6001])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_rmsnorm_gelu_tanh_backward_off_the_128_bit_path_fits_twice(dtype, n):
+    """Two workgroups of 256 threads share a compute unit: registers for one only cost this kernel a quarter of its speed."""
+    _, _, block, grid, aligned = query_launch(10, 2 * _native.ACT_GELU_TANH, 16384, n, dtype)
+    assert (block, aligned) == (256, 0)
+    assert grid == 2 * torch.cuda.get_device_properties(0).multi_processor_count

@@ -96,16 +96,6 @@ __device__ __forceinline__ float rsqrt_refined(float v) {
     return (v > 0.0f && v < __builtin_inff()) ? refined : r;
 }
 
-// Which of a workgroup's rows thread `tid` works on.  A row of 64 threads or more takes whole waves, so the number is the
-// same in every lane of one.  Said so (SCALAR), the row's number and the addresses of its data stay in scalar registers and the
-// loop spends no vector instructions on them: 16 and 19 fewer per thread and row, nine of them quarter-rate products, in the
-// LayerNorm + GeLU kernels, which vector instructions bound (forward + backward bfloat16 16384 x 4096 148.5 -> 146.5 us, with the shorter GeLU of thn_act_math.h 140.8).  The
-// kernels that memory bounds lost by it (normalize float16 65536 x 1024 102.8 -> 104.7 us, LayerNorm 8192 x 6000 87.2 -> 87.9).
-template <int TPR, bool SCALAR> __device__ __forceinline__ int row_group(int tid) {
-    if constexpr (SCALAR && TPR >= 64) return __builtin_amdgcn_readfirstlane(tid / TPR);
-    else return tid / TPR;
-}
-
 // ---------------------------------------------------------------------------------------------------
 // Storage traits.  A "vector" is 16 bytes of a row: VEC elements.  unpack() widens a vector to float32,
 // pack() narrows with round-to-nearest-even (v_cvt_pk_bf16_f32 / v_cvt_f16_f32 / v_cvt_f64_f32).

@@ -206,6 +206,23 @@ constexpr RowForm bwd_form() {
 // 143.2.  Under a profiler, with pauses between the launches, the latter's backward is 7 % faster: back to back the clock falls.
 constexpr bool arithmetic_bound(int act) { return act == kGelu || act == kGeluTanh; }
 
+// A row of 64 threads or more takes whole waves, so its place g in the workgroup is the same in every lane of one.  Said so
+// (readfirstlane), the row's number and the addresses of its data stay in scalar registers and the loop spends no vector instructions on
+// them: 16 and 19 fewer per thread and row, nine of them quarter-rate products.  Where vector instructions bound a kernel that is worth
+// it, us of 2^26 16-bit elements without -> with it: LayerNorm + GeLU, both directions on the 128-bit path and the backward off it
+// (bfloat16 1536 columns backward 89.4 -> 80.7, float16 8195 columns 411 -> 381), and the RMSNorm + GeLU backward over rows of one wave (65 to 192 vectors:
+// bfloat16 640 columns 3.5 %, float16 1536 81.4 -> 78.8).  Elsewhere it changed the registers for the worse and stays off (float32: 2^25 elements):
+//  * other RMSNorm kernels, whose loops need fewer registers: backward + GeLU in its tanh form bfloat16 4098 columns 136 -> 178, 6001
+//    121 -> 142 (one workgroup of 256 threads per compute unit instead of two, or spills), float32 + GeLU 3000 71.8 -> 77.9; on the
+//    128-bit path within 2 % either way;
+//  * the LayerNorm forward off the 128-bit path: + GeLU bfloat16 4098 columns 112.6 -> 118.9, float16 12291 81.1 -> 88.1;
+//  * float32, whose kernels wait for memory: within 1 %;
+//  * the kernels without such an epilogue: normalize float16 65536 x 1024 102.8 -> 104.7, LayerNorm 8192 x 6000 87.2 -> 87.9.
+template <typename T, bool LN, int ACT, bool ALIGNED, bool BWD> constexpr bool scalar_rows(int threads_per_row) {
+    if (T::kBytes != 2 || !arithmetic_bound(ACT) || threads_per_row < 64) return false;
+    return LN ? ALIGNED || BWD : ALIGNED && BWD && ACT == kGelu && threads_per_row == 64;
+}
+
 // Makes the compiler forget what it has derived from the packed vectors, so that the next pass really
 // unpacks them again instead of keeping the float32 values of the previous pass in registers.  No instruction.
 template <int K>
@@ -234,7 +251,8 @@ __global__ void __launch_bounds__(BLOCK) norm_fwd_kernel(const FwdArgs a) {
     __shared__ float red[RedSmem<TPR, G, 2>::kFloats];
 
     const int tid = threadIdx.x;
-    const int g = row_group<TPR, arithmetic_bound(ACT)>(tid);
+    int g = tid / TPR;
+    if constexpr (scalar_rows<T, LN, ACT, ALIGNED, false>(TPR)) g = __builtin_amdgcn_readfirstlane(g);
     const int t = tid % TPR;
     int phase = 0;
 
@@ -523,7 +541,8 @@ __global__ void __launch_bounds__(BLOCK) norm_bwd_kernel(const BwdArgs a) {
     __shared__ Acc comb[G > 1 ? VEC * (BLOCK / 2) : 1];
 
     const int tid = threadIdx.x;
-    const int g = row_group<TPR, arithmetic_bound(ACT)>(tid);
+    int g = tid / TPR;
+    if constexpr (scalar_rows<T, LN, ACT, ALIGNED, true>(TPR)) g = __builtin_amdgcn_readfirstlane(g);
     const int t = tid % TPR;
     int phase = 0;
 
