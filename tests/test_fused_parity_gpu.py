@@ -277,3 +277,12 @@ def test_rmsnorm_gelu_tanh_backward_off_the_128_bit_path_fits_twice(dtype, n):
     _, _, block, grid, aligned = query_launch(10, 2 * _native.ACT_GELU_TANH, 16384, n, dtype)
     assert (block, aligned) == (256, 0)
     assert grid == 2 * torch.cuda.get_device_properties(0).multi_processor_count
+
+
+@pytest.mark.parametrize("act", [_native.ACT_GELU, _native.ACT_GELU_TANH])
+@pytest.mark.parametrize("n", [1536, 3000, 5120, 6000])
+def test_float32_rmsnorm_gelu_backward_runs_one_workgroup_per_compute_unit(n, act):
+    """Memory bounds it: a second 512-thread workgroup, where the registers leave room for one, made it 8 % slower."""
+    k, _, block, grid, aligned = query_launch(10, 2 * act, 16384, n, torch.float32)
+    assert (k, block, aligned) == (3, 512, 1)
+    assert grid == torch.cuda.get_device_properties(0).multi_processor_count

@@ -403,7 +403,7 @@ int default_blocks_per_cu(int which, int flavour, int block) {
     // per compute unit.
     if (which >= kPnormFwd && which <= kNormalizeBwd && block <= 256) return 2;
     // A GeLU epilogue makes the norm kernels arithmetic-bound (about 30 instruction slots per element): they take
-    // as many workgroups per compute unit as their registers allow, up to four.
+    // as many workgroups per compute unit as their registers allow, up to four (one exception in plan_launch()).
     if ((which == kFusedFwd || which == kFusedBwd) && thn::arithmetic_bound(flavour >> 1)) return 4;
     return kDefaultBlocksPerCu;
 }
@@ -871,6 +871,11 @@ int plan_launch(int which, int flavour, bool aligned, int64_t M, int64_t N, int 
             cap < 2) {
             cap = 2;
         }
+        // The float32 RMSNorm backward with a GeLU epilogue in 512-thread workgroups of 3 vectors per thread waits for memory, not
+        // for arithmetic (half the elements per byte of a 16-bit row): one workgroup, although the registers leave room for two
+        // (2^25 elements, two -> one: N = 5120 77.1 -> 71.4 us, 6000 80.2 -> 74.3; 3000 and 1536 within half a percent when one
+        // fits anyway.  LayerNorm's registers leave room for one; with 2 vectors two are as good).
+        if (which == kFusedBwd && aligned && bytes == 4 && (flavour & 1) == 0 && s.k == 3 && s.block == 512) cap = 1;
         if ((narrow_forward_pair || narrow_backward_pair) && cap < 2) cap = 2;
         if (which == kPnormFwd && s.k == 5) cap = 1;       // 1280 vectors per workgroup step: see THN_PN_SHAPES_FIVE above
     }
