@@ -97,7 +97,7 @@ __global__ void __launch_bounds__(kActBlock) act_flat_kernel(const ActArgs a) {
 #pragma unroll
                 for (int e = 0; e < VEC; ++e) {
                     if constexpr (BWD) of[e] = act_bwd<ACT, C>(xf[e], gf[e], p0, p1);
-                    else of[e] = act_fwd<ACT, C>(xf[e], p0, p1);
+                    else of[e] = act_fwd<ACT, C, true>(xf[e], p0, p1);
                 }
                 const int64_t v = v0 + u * kActBlock;
                 if constexpr (kKeepOut) st128_keep(a.out + (v < last ? v : last) * 16, pack_as<T, C>(of));
@@ -117,7 +117,7 @@ __global__ void __launch_bounds__(kActBlock) act_flat_kernel(const ActArgs a) {
     if (blockIdx.x == 0 && i < a.total_elems) {
         const C x = load_elem<T, C>(a.x, i);
         if constexpr (BWD) store_elem<T, C>(a.out, i, act_bwd<ACT, C>(x, load_elem<T, C>(a.g, i), p0, p1));
-        else store_elem<T, C>(a.out, i, act_fwd<ACT, C>(x, p0, p1));
+        else store_elem<T, C>(a.out, i, act_fwd<ACT, C, true>(x, p0, p1));
     }
 }
 
@@ -167,7 +167,7 @@ __global__ void __launch_bounds__(kActBlock) act_rows_kernel(const ActArgs a) {
 #pragma unroll
                     for (int e = 0; e < VEC; ++e) {
                         if constexpr (BWD) of[e] = act_bwd<ACT, C>(xf[e], gf[e], p0, p1);
-                        else of[e] = act_fwd<ACT, C>(xf[e], p0, p1);
+                        else of[e] = act_fwd<ACT, C, true>(xf[e], p0, p1);
                     }
                     st128u(outr + v * 16, pack_as<T, C>(of));
                 } else {
@@ -176,7 +176,7 @@ __global__ void __launch_bounds__(kActBlock) act_rows_kernel(const ActArgs a) {
                     for (int64_t c = v * VEC; c < a.N; ++c) {
                         const C x = load_elem<T, C>(xr, c);
                         if constexpr (BWD) store_elem<T, C>(outr, c, act_bwd<ACT, C>(x, load_elem<T, C>(gr, c), p0, p1));
-                        else store_elem<T, C>(outr, c, act_fwd<ACT, C>(x, p0, p1));
+                        else store_elem<T, C>(outr, c, act_fwd<ACT, C, true>(x, p0, p1));
                     }
                 }
             }

@@ -49,40 +49,50 @@ __device__ __forceinline__ float gelu_tanh_gate(float x) { return gelu_tanh_gate
 // GeLU from the normal distribution function Phi(x) = 0.5*(1 + erf(x/sqrt 2)).  With t = 1/(1 + c|x|) in (0, 1] both directions
 // take Phi(-|x|) = t*Q(t)*exp(-x^2/2), Q a polynomial of degree 7: branch free, accurate in the negative tail (where
 // 1 + erf(..) cancels), a third of the instructions of the library erff.  c is free and sets how fast such a fit converges: at
-// the c below degree 7 reaches what took degree 9 and 8 at c = 0.35.  The sign of x rides on t, t_s = 1/(sgn + c*x) (|t| is a
-// modifier of the polynomial's instructions, no instruction), and step = max(sgn, 0), so that one multiply-add takes the place
-// of a comparison, a subtraction and a selection:
+// the c below degree 7 reaches what took degree 9 and 8 at c = 0.35.  The sign of x rides on t, t_s = 1/(sgn + c*x), and
+// step = max(sgn, 0), so that one multiply-add takes the place of a comparison, a subtraction and a selection:
 //   Phi(x) = step - t_s*Q*exp(-x^2/2),   GeLU'(x) = Phi(x) + x*phi(x) = step + exp(-x^2/2)*(x/sqrt(2 pi) - t_s*Q).
 // The exponential is base 2 (the hardware's v_exp_f32), of a^2 with a = x*sqrt(log2(e)/2).  19 instruction slots per element
-// forward and 20 backward (a transcendental counts as 2) instead of 21 and 22; against float64 (2-norm, x = 1.5 g + 0.25 with g normal)
-// 3.29e-8 and 4.26e-8 instead of 3.32e-8 and 4.46e-8, and no larger for g alone, for the negative tail and for |x| < 6.
-// Forward + backward bfloat16 16384 x 4096: GeLU 110.0 -> 108.8 us, LayerNorm + GeLU 146.5 -> 140.8.
+// forward and 20 backward (a transcendental counts as 2) instead of 21 and 22.  Float32 against float64, 2-norm: x = 1.5 g + 0.25 with g
+// normal 3.29e-8 and 4.26e-8 instead of 3.32e-8 and 4.46e-8, g alone 3.88e-8 and 4.83e-8 instead of 3.98e-8 and 5.14e-8; in bands of
+// x the roundings fall differently, up to 0.7 and up to 1.23 times as large ([-4, -3] 4.4e-7 -> 3.1e-7 forward, [-2, -1.5] 1.43e-7 -> 1.62e-7).
+//
+// |t| is a modifier of the polynomial's multiply-adds, which then have no room for a coefficient and read it from a scalar register.
+// LITERALS: |t| in a register of its own, an instruction more, and the coefficients in the instructions.  That is the faster
+// one where little else is in flight, without -> with, us: the element-wise forward of 2^23 and 2^24 bfloat16 elements 6.8-7.1 -> 6.3-6.7
+// and 12.0 -> 11.3 (2^26 42.6 -> 42.3; before degree 7 6.6, 11.5 and 43.7; float16 9.5 -> 9.5 and 12.4 -> 12.3, before 9.2 and 12.0), 2^22 float64
+// elements 10.1 -> 9.8, and the RMSNorm forward off the 128-bit path (2^26 bfloat16 elements, 4098 columns 94.9 -> 92.1).  The
+// forwards on that path lose 2-4 % by it (RMSNorm + GeLU bfloat16 1536 columns 47.0 -> 49.0), and the backwards spill.
 struct NormalParts {
     float tq, e, step;      // t_s*Q(t), exp(-x^2/2), x < 0 ? 0 : 1
 };
-template <int DEGREE>
+template <int DEGREE, bool LITERALS>
 __device__ __forceinline__ NormalParts normal_parts(float x, float c, const float (&coefficients)[DEGREE + 1]) {
     const float sgn = __builtin_copysignf(1.0f, x);
     const float t = rcp_fast(__builtin_fmaf(c, x, sgn));
     const float a = x * 0.84932180028801907f;
+    float size = __builtin_fabsf(t);
+    if constexpr (LITERALS) asm("" : "+v"(size));
     float q = coefficients[DEGREE];
 #pragma unroll
-    for (int i = DEGREE - 1; i >= 0; --i) q = __builtin_fmaf(q, __builtin_fabsf(t), coefficients[i]);
+    for (int i = DEGREE - 1; i >= 0; --i) q = __builtin_fmaf(q, size, coefficients[i]);
     return NormalParts{t * q, __builtin_amdgcn_exp2f(-a * a), sgn > 0.0f ? sgn : 0.0f};
 }
 
-// Minimax fit of the relative error of Phi(-|x|) (x in [0, 13.3], behind which the exponential underflows): 8.3e-8.
+// Minimax fit of the relative error of Phi(-|x|) (x in [0, 13.3], behind which the exponential underflows): 1.24e-7 with c and the
+// coefficients as stored.
+template <bool LITERALS>
 __device__ __forceinline__ float normal_cdf(float x) {
-    const NormalParts p = normal_parts<7>(x, 0.3036f, {0.12107304f, 0.12204604f, 0.1020654f, 0.12441437f, -0.044881325f,
-                                                       0.19440602f, -0.15598506f, 0.036861554f});
+    const NormalParts p = normal_parts<7, LITERALS>(x, 0.3036f, {0.12107304f, 0.12204604f, 0.1020654f, 0.12441437f, -0.044881325f,
+                                                                 0.19440602f, -0.15598506f, 0.036861554f});
     return __builtin_fmaf(-p.tq, p.e, p.step);
 }
 
-// Minimax fit of the error relative to |x|/sqrt(2 pi) + t*Q, which is what GeLU' is made of: 2.3e-8.  (c = 0.385 to 0.41 measure
-// alike; beyond 0.415 the fit is worse than degree 8 at 0.354 was.)
+// Minimax fit of the error relative to |x|/sqrt(2 pi) + t*Q, which is what GeLU' is made of: 4.5e-8 as stored.  (c = 0.385 to 0.41
+// measure alike; beyond 0.415 the fit is worse than degree 8 at 0.354 was.)
 __device__ __forceinline__ float gelu_slope(float x) {
-    const NormalParts p = normal_parts<7>(x, 0.401f, {0.16005206f, 0.15829173f, 0.14927879f, 0.011608556f, 0.21302079f,
-                                                      -0.34127876f, 0.18568613f, -0.036659308f});
+    const NormalParts p = normal_parts<7, false>(x, 0.401f, {0.16005206f, 0.15829173f, 0.14927879f, 0.011608556f, 0.21302079f,
+                                                             -0.34127876f, 0.18568613f, -0.036659308f});
     return __builtin_fmaf(p.e, __builtin_fmaf(0.39894228040143267794f, x, -p.tq), p.step);
 }
 
@@ -103,10 +113,10 @@ __device__ __forceinline__ MishParts mish_parts(float x) {
     return m;
 }
 
-template <int ACT, typename C>
+template <int ACT, typename C, bool LITERALS = false>
 __device__ __forceinline__ C act_fwd(C x, C p0, C p1) {
     if constexpr (ACT == kGelu) {
-        return x * normal_cdf(x);                                                          // gelu.py:28
+        return x * normal_cdf<LITERALS>(x);                                                  // gelu.py:28
     } else if constexpr (ACT == kGeluTanh) {
         return x * gelu_tanh_gate(x);                                                      // gelu.py:23-26
     } else if constexpr (ACT == kSilu) {

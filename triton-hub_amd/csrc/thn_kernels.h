@@ -358,7 +358,7 @@ __global__ void __launch_bounds__(BLOCK) norm_fwd_kernel(const FwdArgs a) {
                     } else {
                         yf[e] = xf[e] * rstd * wr[k][e];
                     }
-                    if constexpr (ACT != kNoAct) yf[e] = act_fwd<ACT, float>(yf[e], 0.0f, 0.0f);
+                    if constexpr (ACT != kNoAct) yf[e] = act_fwd<ACT, float, !ALIGNED>(yf[e], 0.0f, 0.0f);
                 }
                 slot_store<T, ALIGNED>(yrow, voff[k], a.n_cols, yf);
                 if constexpr (kForm.ahead) cur[k] = nxt[k];
@@ -446,7 +446,7 @@ __global__ void __launch_bounds__(BLOCK) norm_fwd_kernel(const FwdArgs a) {
                 if constexpr (LN && arithmetic_bound(ACT)) yf[e] = fmaf(fmaf(xf[k][e], rstd, shift_y), wr[k][e], br[k][e]);
                 else if constexpr (LN) yf[e] = fmaf((xf[k][e] - delta) * rstd, wr[k][e], br[k][e]);
                 else yf[e] = xf[k][e] * rstd * wr[k][e];
-                if constexpr (ACT != kNoAct) yf[e] = act_fwd<ACT, float>(yf[e], 0.0f, 0.0f);
+                if constexpr (ACT != kNoAct) yf[e] = act_fwd<ACT, float, !ALIGNED>(yf[e], 0.0f, 0.0f);
             }
             slot_store<T, ALIGNED>(yrow, voff[k], a.n_cols, yf);
         }
