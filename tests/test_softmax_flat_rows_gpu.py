@@ -122,7 +122,7 @@ def test_default_choice_masked_logits_strided_rows_and_determinism():
 
 @pytest.mark.parametrize("vecs,ragged", [(17, 0), (17, -3), (21, 0), (25, -3), (31, -1), (31, 0), (32, -1), (32, -3)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
-def test_rows_of_17_to_32_vectors_do_not_meet(dtype, vecs, ragged):
+def test_rows_of_17_to_31_vectors_do_not_meet(dtype, vecs, ragged):
     """Rows of one wave share its lanes: a row's bits do not depend on its neighbours, whatever they hold (32 vectors leave no idle
     lane for the sums to read), on the row count (a single row, partial steps, several steps of a workgroup) or on the distance
     between rows."""

@@ -118,25 +118,24 @@ __global__ void __launch_bounds__(kFlatBlock) softmax_flat_fwd_kernel(const Soft
     }
 }
 
-// The tree of segment_allreduce_op for values that are ready to be read by any lane: where that one selects after the read,
-// the lane to read from is chosen once, in front of the row loop.  A lane with nothing to take reads itself for a maximum and, for
-// a sum, the wave's last lane, which is outside every segment and holds 0 when L does not divide 64; for L that do, the
-// sum selects.
-template <int LOG> struct FlatTree {
-    int max_from[LOG > 0 ? LOG : 1], sum_from[LOG > 0 ? LOG : 1];       // byte addresses of ds_bpermute
-    bool idle;
-    __device__ __forceinline__ FlatTree(int lane, int pos, int L) : idle(64 % L != 0) {
+// The tree of segment_allreduce_op over segments of 17 to 31 lanes for values that are ready to be read by any lane: where that
+// one selects after the read, the lane to read from is chosen once, in front of the row loop.  A lane with nothing to take reads
+// itself for a maximum and, for a sum, the wave's last lane, which is outside every segment (none of these lengths divides 64) and holds 0.
+struct FlatTree {
+    static constexpr int kSteps = 5;
+    int max_from[kSteps], sum_from[kSteps];       // byte addresses of ds_bpermute
+    __device__ __forceinline__ FlatTree(int lane, int pos, int L) {
 #pragma unroll
-        for (int s = 0; s < LOG; ++s) {
+        for (int s = 0; s < kSteps; ++s) {
             const bool take = pos + (1 << s) < L;
             max_from[s] = (take ? lane + (1 << s) : lane) * 4;
             sum_from[s] = (take ? lane + (1 << s) : 63) * 4;
         }
     }
     template <typename Op, int NV>
-    __device__ __forceinline__ static void reduce(float (&v)[NV], const int (&from)[LOG > 0 ? LOG : 1], int first) {
+    __device__ __forceinline__ static void reduce(float (&v)[NV], const int (&from)[kSteps], int first) {
 #pragma unroll
-        for (int s = 0; s < LOG; ++s) {
+        for (int s = 0; s < kSteps; ++s) {
 #pragma unroll
             for (int i = 0; i < NV; ++i) v[i] = Op::apply(v[i], as_f32(static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(from[s], static_cast<int>(as_u32(v[i]))))));
         }
@@ -144,10 +143,7 @@ template <int LOG> struct FlatTree {
         for (int i = 0; i < NV; ++i) v[i] = lane_read(v[i], first);
     }
     template <int NV> __device__ __forceinline__ void max(float (&v)[NV], int first) const { reduce<OpMax>(v, max_from, first); }
-    template <int NV> __device__ __forceinline__ void sum(float (&v)[NV], int lane, int pos, int L, int first) const {
-        if (idle) reduce<OpSum>(v, sum_from, first);
-        else segment_allreduce_op<LOG, NV, OpSum>(v, lane, pos, L, first);
-    }
+    template <int NV> __device__ __forceinline__ void sum(float (&v)[NV], int first) const { reduce<OpSum>(v, sum_from, first); }
 };
 
 // Where a lane's vector of its row is, from one step to the next.  An address moves by the same distance every step and stops at
@@ -167,15 +163,20 @@ template <typename P> struct FlatWalk {
     }
 };
 
-// The forward over rows of 17 to 32 vectors: 206 instruction slots per wave and step of two rows per lane (bfloat16, off the
-// 128-bit path) instead of 310, of which 52 went into addresses, 20 into selections around the reductions and 16 into the
-// columns that two windows share.  The vector units had been busy for 19 us of a forward of 24.5 (768 x 197 x 197), with as much memory
-// time: 24.3 -> 23.0 us, rows of 250 columns 46.8 -> 45.9 and of 100 in float32 44.2 -> 43.8 (2^26 and 2^25 elements).  Same bits.  Rows
-// of up to 16 vectors stay with the kernel above: there memory bounds it, and this one, which requests its vectors closer together, is
-// slower at most widths (bfloat16 N = 32 41.8 -> 44.0, 72 43.6 -> 44.3, 127 44.6 -> 46.0; with two or four workgroups per compute
-// unit instead of its best, three, up to 57.4).  So is the backward (197 columns 67.7 -> 68.2, 127 72.3 -> 75.1).
-template <typename T, bool LOGSM, int J, bool ALIGNED>
-__global__ void __launch_bounds__(kFlatBlock) softmax_flat_fwd_kernel_17_to_32(const SoftmaxFwdArgs a) {
+// The forward over 16-bit rows of 17 to 31 vectors, two rows per lane and step: 206 instruction slots per wave and step (bfloat16, off
+// the 128-bit path) instead of 310, of which 52 went into addresses, 20 into selections around the reductions and 16 into the
+// columns that two windows share.  With 8 exponentials per 16 bytes the vector units had been as busy as the memory: 19 us of a
+// forward of 24.5 (768 x 197 x 197), 24.3 -> 23.0.  2^26 elements, softmax / log-softmax, means over nine numbers of vectors: bfloat16 on
+// the 128-bit path -4.8 / -3.8 %, off it -5.9 / -4.6 %, float16 -4.8 / -5.1 % and -8.0 / -4.7 % (191 columns bfloat16 53.7 -> 49.4 us; every
+// one of them faster); 2^23 elements -3 to -9 %. Same bits.
+// The kernel above, which requests its vectors further apart, keeps what memory bounds: float32 rows (2^25 elements up to 3 % slower
+// with this one: 96 columns 44.6 -> 45.5 us, 127 45.1 -> 46.4, 0.9 % faster in the mean), rows of 32 vectors off the path (255 columns
+// bfloat16 49.4 -> 49.0 and, log-softmax, 48.5 -> 49.1), rows of up to 16 vectors (bfloat16 N = 32 41.8 -> 44.0, 72 43.6 -> 44.3, 127
+// 44.6 -> 46.0; with two or four workgroups per compute unit instead of its best, three, up to 57.4).  So does the backward (197 columns
+// 67.7 -> 68.2, 127 72.3 -> 75.1).
+template <typename T, bool LOGSM, bool ALIGNED>
+__global__ void __launch_bounds__(kFlatBlock) softmax_flat_fwd_kernel_17_to_31(const SoftmaxFwdArgs a) {
+    constexpr int J = 2;
     constexpr int VEC = T::VEC;
     constexpr int W = kFlatBlock / 64;
     const int L = a.n_vecs;
@@ -186,8 +187,8 @@ __global__ void __launch_bounds__(kFlatBlock) softmax_flat_fwd_kernel_17_to_32(c
     flat_slot<T, ALIGNED>(f.t, L, a.n_cols, voff, lead);
     const float neg_inf = OpMax::identity<float>();
     // softmin: the sign bits are flipped on the packed vectors
-    const uint32_t flip = a.sign < 0.0f ? (T::kBytes == 2 ? 0x80008000u : 0x80000000u) : 0u;
-    const FlatTree<5> tree(lane, f.pos, L);
+    const uint32_t flip = a.sign < 0.0f ? 0x80008000u : 0u;
+    const FlatTree tree(lane, f.pos, L);
     float counts[VEC];          // an overlapping window's leading columns count in the slot before
 #pragma unroll
     for (int e = 0; e < VEC; ++e) counts[e] = e >= lead ? 1.0f : 0.0f;
@@ -240,7 +241,7 @@ __global__ void __launch_bounds__(kFlatBlock) softmax_flat_fwd_kernel_17_to_32(c
             }
             s[j] = f.own ? sk : 0.0f;
         }
-        tree.sum(s, lane, f.pos, L, f.first);
+        tree.sum(s, f.first);
 #pragma unroll
         for (int j = 0; j < J; ++j) {
             const float scale = LOGSM ? logf(s[j]) : 1.0f / s[j];
@@ -328,10 +329,12 @@ __global__ void __launch_bounds__(kFlatBlock) softmax_flat_bwd_kernel(const Soft
     }
 }
 
-// log_steps = 5 is what rows of 17 to 32 vectors have.
-template <typename T, bool LOGSM, int J, int LOG, bool ALIGNED> constexpr auto softmax_flat_fwd() {
-    if constexpr (LOG == 5) return &softmax_flat_fwd_kernel_17_to_32<T, LOGSM, J, ALIGNED>;
-    else return &softmax_flat_fwd_kernel<T, LOGSM, J, LOG, ALIGNED>;
+// (log_steps = 5: rows of 17 to 32 vectors)
+template <typename T, bool LOGSM, int J, int LOG, bool ALIGNED> auto softmax_flat_fwd(int n_vecs) {
+    if constexpr (T::kBytes == 2 && J == 2 && LOG == 5) {
+        if (n_vecs < 32) return &softmax_flat_fwd_kernel_17_to_31<T, LOGSM, ALIGNED>;
+    }
+    return &softmax_flat_fwd_kernel<T, LOGSM, J, LOG, ALIGNED>;
 }
 
 // Launchers: 0 launched, 1 no such instance, <0 HIP error.  `log_steps`: tree steps of the segmented reductions (0 for
@@ -353,8 +356,8 @@ THN_DECLARE_SOFTMAX_FLAT_LAUNCHERS(bf16)
     }
 #define THN_SOFTMAX_FLAT_FWD_CASE(AL, J_, LOG_)                                                                 \
     if (rows_each == J_ && log_steps == LOG_) {                                                                 \
-        return is_log ? run_kernel<SoftmaxFwdArgs>(softmax_flat_fwd<T, true, J_, LOG_, AL>(), a, grid, kFlatBlock, st, nullptr)      \
-                      : run_kernel<SoftmaxFwdArgs>(softmax_flat_fwd<T, false, J_, LOG_, AL>(), a, grid, kFlatBlock, st, nullptr);    \
+        return is_log ? run_kernel<SoftmaxFwdArgs>(softmax_flat_fwd<T, true, J_, LOG_, AL>(a.n_vecs), a, grid, kFlatBlock, st, nullptr)      \
+                      : run_kernel<SoftmaxFwdArgs>(softmax_flat_fwd<T, false, J_, LOG_, AL>(a.n_vecs), a, grid, kFlatBlock, st, nullptr);    \
     }
 #define THN_SOFTMAX_FLAT_FWD_AL(J_, LOG_) THN_SOFTMAX_FLAT_FWD_CASE(true, J_, LOG_)
 #define THN_SOFTMAX_FLAT_BWD_AL(J_, LOG_) THN_SOFTMAX_FLAT_CASE(softmax_flat_bwd_kernel, SoftmaxBwdArgs, true, J_, LOG_)
