@@ -1744,7 +1744,8 @@ int act_blocks_per_cu(int act, bool bwd, int bytes) {
     return 2;
 }
 
-// thn::dropout_scale() takes 1-8 us, so each thread keeps the last few that it asked for (a function of its two arguments alone).
+// thn::dropout_scale() takes 1.6 us for float16 and 0.4 for bfloat16, so each thread keeps the last few that it asked for (a function
+// of its two arguments alone).
 float remembered_dropout_scale(float keep, int dtype) {
     struct Entry {
         float keep, scale;
@@ -1762,6 +1763,8 @@ float remembered_dropout_scale(float keep, int dtype) {
     oldest = (oldest + 1) % kEntries;
     return scale;
 }
+
+constexpr int64_t kDropoutScaleFrom = int64_t{1} << 22;
 
 int dropout_launch(thn::DropoutMask mode, const void* x, void* out, uint32_t* mask, int64_t n, int64_t first_offset, float p,
                    uint64_t seed, int dtype, void* stream) {
@@ -1785,7 +1788,9 @@ int dropout_launch(thn::DropoutMask mode, const void* x, void* out, uint32_t* ma
     a.key_lo = static_cast<uint32_t>(seed);
     a.key_hi = static_cast<uint32_t>(seed >> 32);
     a.threshold = thn::dropout_threshold(p);
-    a.scale = remembered_dropout_scale(1.0f - p, dtype);
+    // Smaller calls take less time than the host needs for them, with the quotient too: a program with more probabilities than are
+    // remembered, or a new one on each call, must not pay for the search there.
+    if (n >= kDropoutScaleFrom) a.scale = remembered_dropout_scale(1.0f - p, dtype);
     a.mask = mask;
     if (mode != thn::DropoutMask::kNone && (a.threshold == thn::kDropAll || first_offset != 0 || n > thn::kMaskedMost)) return THN_E_SHAPE;
     // Bound by integer arithmetic: as many waves as a compute unit holds (8 workgroups of 256 threads).  From a mask, by

@@ -65,27 +65,34 @@ inline uint32_t dropout_threshold(float p) {
 // x's significand alone, so every one of them is tried: the normal numbers at one exponent (results only grow, keep being
 // at most 1: they stay normal, and infinity starts at the rounding boundary of the largest), the subnormal ones in units of
 // the smallest, where bfloat16 results below 128 units have been rounded to float32's subnormal grid of 2^-16 units first.
-// Found for 93 of the p = 0.01, 0.02 ... 0.99 with bfloat16, for 86 with float16.
+// Found for 92 of the p = 0.01, 0.02 ... 0.99 with bfloat16, for 86 with float16.
+// (Loops without an exit, which the compiler makes vector loops of: 1.6 us for float16 and 0.4 for bfloat16 on the host, in the mean
+// over those p; one value at a time took 6.1 and 1.4.)
 template <int kBits, bool kCoarse>      // significand bits with the hidden one; float32's own subnormal grid matters
 inline bool products_round_alike(float keep, float r) {
     constexpr int kHidden = 1 << (kBits - 1), kDrop = 24 - kBits;
     const auto narrow = [](float v) {
         uint32_t u;
         memcpy(&u, &v, 4);
-        return (u + (1u << (kDrop - 1)) - 1u + (u >> kDrop & 1u)) >> kDrop;
+        return static_cast<int32_t>((u + (1u << (kDrop - 1)) - 1u + (u >> kDrop & 1u)) >> kDrop);
     };
+    int32_t differ = 0;
     for (int m = kHidden; m < 2 * kHidden; ++m) {
         const float x = static_cast<float>(m);
-        if (narrow(x / keep) != narrow(x * r)) return false;
+        differ |= narrow(x / keep) ^ narrow(x * r);
     }
-    const auto narrow_subnormal = [&](double exact) {
-        if (exact >= kHidden) return static_cast<double>(narrow(static_cast<float>(exact))) + 65536.0;
-        return nearbyint(kCoarse ? nearbyint(exact * 65536.0) / 65536.0 : static_cast<double>(static_cast<float>(exact)));
-    };
+    if (differ != 0) return false;
+    // (a float32 result from kHidden units on is a normal number; below it goes to whole units, to even)
+    const auto narrow_subnormal = [&](float v) { return narrow(v >= static_cast<float>(kHidden) ? v : (v + 0x1p23f) - 0x1p23f); };
+    const auto coarse = [](double exact) { return static_cast<float>(((exact * 65536.0 + 0x1p52) - 0x1p52) / 65536.0); };     // (1 / keep is at most 2^24)
     for (int m = 1; m < kHidden; ++m) {
-        if (narrow_subnormal(static_cast<double>(m) / keep) != narrow_subnormal(static_cast<double>(m) * r)) return false;
+        const float x = static_cast<float>(m);
+        float quotient = x / keep, product = x * r;
+        if (kCoarse && quotient < static_cast<float>(kHidden)) quotient = coarse(static_cast<double>(m) / keep);
+        if (kCoarse && product < static_cast<float>(kHidden)) product = coarse(static_cast<double>(m) * r);
+        differ |= narrow_subnormal(quotient) ^ narrow_subnormal(product);
     }
-    return true;
+    return differ == 0;
 }
 inline float dropout_scale(float keep, int dtype) {
     if (!(keep > 0.0f) || (dtype != kF16 && dtype != kBF16)) return 0.0f;
