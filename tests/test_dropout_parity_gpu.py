@@ -352,22 +352,30 @@ def test_nothing_kept_where_saved_tensors_are_managed():
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("p", [0.0123, 0.1, 0.4, 0.5, 0.7, 1 - 2.0 ** -20])
+@pytest.mark.parametrize("p", [0.0123, 0.1, 0.4, 0.5, 0.7, 0.98, 1 - 2.0 ** -20])
 def test_every_16_bit_value_is_divided_correctly(p, dtype):
     """All values of the type -- subnormal numbers, infinities and NaN among them -- through the kernels with and without kept
-    decisions, for probabilities whose quotients a product gives and such that need the quotient itself (0.4 and 0.7)."""
+    decisions and, from 2^22 elements on, a factor, for probabilities whose quotients a product gives and such that need the
+    quotient itself (0.4 and 0.7).  Kept elements hold every value (of the four that p = 1 - 2^-20 keeps, four of them)."""
     announce(f"every value p={p} {dtype}")
     values = torch.arange(1 << 16, dtype=torch.int32).to(torch.int16).view(dtype)
-    for copies in (3, 64):                              # 64: 2^22 elements, whose forward keeps its decisions
-        x = values.repeat(copies)
-        random.seed(7)
-        seed = random.randint(0, 2 ** 16)
-        random.seed(7)
+    random.seed(7)
+    seed = random.randint(0, 2 ** 16)
+    for n in ((1 << 22) - 8, 1 << 22):                  # 2^22 elements: the forward keeps its decisions
+        kept = expected(torch.ones(n), p, seed) != 0
+        x = torch.empty(n, dtype=dtype)
+        for part in (kept, ~kept):
+            x[part] = values.repeat(n // values.numel() + 1)[:int(part.sum())]
+        assert x[kept].view(torch.int16).unique().numel() == min(1 << 16, int(kept.sum()))
+        want = expected(x, p, seed)
         xg = x.cuda().requires_grad_(True)
+        random.seed(7)
         y = Dropout(p)(xg)
         dx, = torch.autograd.grad(y, xg, x.cuda())
-        want = expected(x, p, seed)
-        for got in (y.detach().cpu(), dx.cpu()):
+        random.seed(7)
+        with torch.no_grad():
+            alone = Dropout(p)(xg)
+        for got in (y.detach().cpu(), dx.cpu(), alone.cpu()):
             nan = torch.isnan(want)
             assert torch.equal(torch.isnan(got), nan)
             assert same_bits(got[~nan], want[~nan])

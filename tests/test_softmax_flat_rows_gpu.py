@@ -147,10 +147,37 @@ def test_rows_of_17_to_31_vectors_do_not_meet(dtype, vecs, ragged):
     for fn, y in want.items():
         out = fn()(wild)
         assert torch.equal(out[calm], y[calm])
-        assert bool(out[1::16].isnan().all()) and bool(out[5::16].isnan().all())
+        assert bool(out[1::16].isnan().all()) and bool(out[3::16].isnan().all()) and bool(out[5::16].isnan().all())
         flat = 1.0 / n if fn is not A.LogSoftmax else -math.log(n)
         for first in (7, 9):
             assert bool(((out[first::16].double() - flat).abs() <= abs(flat) * (step + 64 * 2.0 ** -24)).all())
         assert torch.equal(fn()(padded[:, :n]), y)
         for m in (1, 2, 3, 8, 9, 1025):
             assert torch.equal(fn()(x[:m].contiguous()), y[:m])
+
+
+@pytest.mark.parametrize("vecs,ragged", [(2, -3), (17, -1), (17, -3), (25, -3), (31, -2), (32, -3)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_single_values_in_the_columns_that_two_windows_share(dtype, vecs, ragged):
+    """Off the 128-bit path the last vector of a row overlaps the one before it: its first columns must count once in the sum, and
+    a NaN or an infinity there must reach the whole row as it does from any other column, and no other row."""
+    vec = 16 // torch.empty(0, dtype=dtype).element_size()
+    n = vecs * vec + ragged
+    shared = range(n - vec, (vecs - 1) * vec)
+    assert len(shared) == -ragged
+    g = torch.Generator(device="cuda").manual_seed(n)
+    x = torch.randn(4000, n, device="cuda", generator=g).mul_(3).to(dtype)
+    values = [math.nan, math.inf, -math.inf, torch.finfo(dtype).min, 12.0]
+    for i, column in enumerate(c for c in shared for _ in values):
+        x[16 * i + 1, column] = values[i % len(values)]
+    step = torch.finfo(dtype).eps
+    for fn, sign in ((A.Softmax, 1.0), (A.Softmin, -1.0), (A.LogSoftmax, 1.0)):
+        out = fn()(x).double()
+        log = torch.log_softmax(sign * x.double(), -1)
+        exact = log if fn is A.LogSoftmax else log.exp()
+        # the storage type's rounding and 64 of float32 (arguments of up to 30, the sum); a 16-bit result below its smallest normal number is rounded to its grid
+        allowed = (step + 64 * 2.0 ** -24) * exact.abs() + (30 * 2.0 ** -24 if fn is A.LogSoftmax else torch.finfo(dtype).tiny)
+        finite = exact.isfinite()
+        assert torch.equal(out.isnan(), exact.isnan())
+        assert torch.equal(out[exact.isinf()], exact[exact.isinf()])
+        assert bool(((out - exact).abs() <= allowed)[finite].all())
