@@ -18,10 +18,10 @@
 //  * 16-bit values are scaled by one multiplication where dropout_scale() finds a factor, instead of 3 instructions;
 //  * a forward that keeps its decisions shifts each into its word with the comparison's own mask as the carry of one
 //    addition, and takes the element's part of the first product as the addend of that multiplication.
-// bfloat16 16384 x 4096 (134 MB in, 134 MB out): a forward that keeps its decisions takes 88 us (41.5 vector instructions per
-// element, issuing in 96 % of the cycles in which a compute unit is busy; 45.1 instructions, 65 registers, which leave room for
-// 7 of the 8 workgroups per compute unit that are launched, and no decision before the first vectors had arrived: 95); with
-// its backward 132 -> 125.
+// bfloat16 16384 x 4096 (134 MB in, 134 MB out): a forward that keeps its decisions takes 88.6 us under the profiler (41.8 vector
+// instructions per element, issuing in 96 % of the cycles in which a compute unit is busy; with 45.4 instructions, registers for
+// 7 of the 8 workgroups per compute unit that are launched and no decision before the first vectors had arrived 97.7); with
+// its backward 134.0 -> 127.3 among others.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -264,7 +264,7 @@ __global__ void __launch_bounds__(kDropoutBlock) dropout_flat_kernel(const Dropo
 // (forward of 2^24 float64 49.5 us against 48.4, 2^23 float32 15.3 against 14.7).  Slots past the end repeat the last vector, so
 // that no branch stands around a load or a store.  The threshold is below kDropAll (p < 1 in float32), the offsets of the
 // elements start at 0 and fit 32 bits.
-// bfloat16 16384 x 4096: forward 88 us, backward 45, which is what two plain streams take (80 drawn again).
+// bfloat16 16384 x 4096 under the profiler: forward 88.6 us, backward 45.2, which is what two plain streams take (80 drawn again).
 template <typename T, bool kRead, bool kProduct>
 __global__ void __launch_bounds__(kDropoutBlock, kRead || T::kBytes > 2 ? 1 : 8) dropout_masked_kernel(const DropoutArgs a) {
     using C = typename std::conditional<T::kBytes == 8, double, float>::type;

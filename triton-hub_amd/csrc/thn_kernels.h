@@ -436,7 +436,10 @@ __global__ void __launch_bounds__(BLOCK) norm_fwd_kernel(const FwdArgs a) {
             rstd = rsqrt_refined(fmaf(q[0], a.inv_n, a.eps));
         }
 
-        const float shift_y = -delta * rstd;       // (d - delta)*rstd in one multiply-add, where arithmetic is what counts
+        // (d - delta)*rstd in one multiply-add, where arithmetic is what counts.  As accurate, delta being the rounding residue of
+        // mean0; the forms above that unpack a row again, bound by other things, keep the subtraction, so the last bit of an
+        // element may depend on which form its row's width gets.
+        const float shift_y = -delta * rstd;
         char* yrow = a.y + row * a.y_stride_bytes;
 #pragma unroll
         for (int k = 0; k < K; ++k) {
@@ -517,8 +520,8 @@ __device__ __forceinline__ void store_partial(float* dst, const float (&f)[VEC])
 
 // ACT != kNoAct: the forward was y = act(z), z = xhat*w + b.  The pre-activation is not stored: the kernel
 // recomputes z from the saved statistics and replaces the upstream gradient by dy * act'(z) before anything else
-// uses it.  z needs the corrected xhat, so LayerNorm takes one more reduction round (sum(u) first); the loop is
-// still bound by memory.
+// uses it.  z needs the corrected xhat, so LayerNorm takes one more reduction round (sum(u) first).  With a GeLU
+// epilogue over 16-bit rows vector instructions bound the loop (arithmetic_bound), with the others, and over wider types, memory.
 template <typename T, bool LN, int K, int TPR, int BLOCK, bool ALIGNED, int ACT = kNoAct>
 __global__ void __launch_bounds__(BLOCK) norm_bwd_kernel(const BwdArgs a) {
     constexpr int VEC = T::VEC;
