@@ -388,7 +388,8 @@ int thn_norm_set_launch_override(int which, int vecs_per_thread, int threads_per
  * thn_act code.  For the p-norm / normalize forward (4) a non-zero `is_layernorm` asks for thn_normalize_fwd's launch
  * (0: thn_pnorm_fwd's; they differ for 16-bit rows of 769 to 1024 vectors off the 128-bit path).  Rows wider than 64 KiB of the softmax and p-norm families report their looping kernels:
  * {vectors per thread and step, block_threads, block_threads, grid_blocks, 0}, or, softmax rows of up to 384 KiB that stay in
- * the registers of a compute unit (dense tensors), {vectors per thread, 1024, 1024, grid_blocks, 1}.  Norm problems that take the flat
+ * the registers of a compute unit (dense tensors), {vectors per thread, 1024, 1024, grid_blocks, 1}, or, few rows that are cut into
+ * slices (dense tensors; the override {4, 512, 0, 0} selects them), {4, 512, 512, grid_blocks, 1}.  Norm problems that take the flat
  * kernels (narrow 16-bit rows whose vector count is not a power of two; off the 128-bit path narrow rows of any
  * vector count and type) report {rows per lane and step, vectors per row, 256, grid_blocks, 1}: a threads_per_row that
  * is not a power of two identifies them (off the path a flat launch over 8, 16 or 32 vectors with one row per lane

@@ -20,6 +20,7 @@
 #include "thn_softmax_dispatch.h"
 #include "thn_softmax_flat.h"
 #include "thn_softmax_wide.h"
+#include "thn_softmax_sliced.h"
 #include "thn_pnorm_flat.h"
 #include "thn_tiny.h"
 
@@ -437,7 +438,7 @@ bool wide_fwd_loses(bool is_log, int64_t M, int64_t vecs, int k, int bytes, int 
 }
 
 // Vectors per thread of the register-resident softmax kernels (thn_softmax_wide.h) for M rows of N columns on `cus` compute
-// units, 0 where the looping kernels run: float64, rows of more than 24 x 1024 vectors, an overridden launch shape of those
+// units, 0 where the looping kernels run (few rows are cut into slices before it comes to that, softmax_slicing()): float64, rows of more than 24 x 1024 vectors, an overridden launch shape of those
 // kernels, and where the second walk costs nothing, because what it reads still lies in the eight 4-MiB L2s:
 //   forward, 16-bit: x of less than 24 MiB (bfloat16 looping -> registers, softmax: 64 x 40000 9.1 -> 9.9 us, 192 x 40000 10.0 ->
 //     10.6, 64 x 90001 16.2 -> 17.5, 192 x 90001 21.5 -> 18.7, 512 x 151936 75.5 -> 63.7).  float32 rows have half the
@@ -470,6 +471,34 @@ int softmax_wide_vecs(int which, bool is_log, int64_t M, int64_t N, int dtype, i
     return k;
 }
 
+// Whether M rows of N columns are cut into slices (thn_softmax_sliced.h), and how:
+//   rows of more than 384 KiB, which would be walked twice by a workgroup each: up to 1.5 times as many as compute units.
+//   narrower ones, from 128 KiB on: fewer than half as many as compute units, a softmax backward, which reads y and dy twice here, up
+//     to a quarter (below 128 KiB two launches cost what the slices gain);
+//   narrower ones that would be walked twice: also up to a fifth more than compute units, but for a softmax backward.
+// A launch override keeps the slices off, except {4 vectors per thread, 512 threads per row, 0, 0}, which selects them.
+bool softmax_slicing(int which, bool is_log, int64_t M, int64_t N, int dtype, int cus, thn::Slicing* out) {
+    const int bytes = elem_bytes(dtype);
+    const int64_t vecs = N / (16 / bytes);
+    if (dtype == THN_F64 || N * bytes <= kMaxRowBytes || vecs > static_cast<int64_t>(thn::kSlicedMost) * thn::kSlicedBlock * thn::kSlicedVecs) return false;
+    const Override& ov = g_override[which];
+    const int k = ov.k.load(), tpr = ov.tpr.load(), block = ov.block.load(), bpc = ov.bpc.load();
+    if (k == thn::kSlicedVecs && tpr == thn::kSlicedBlock && block == 0 && bpc == 0) {
+        if (M > INT32_MAX / thn::kSlicedMost) return false;
+    } else if (k > 0 || tpr > 0 || block > 0 || bpc > 0) {
+        return false;
+    } else {
+        const bool reads_twice = which == kSoftmaxBwd && !is_log;
+        bool gains;
+        if (vecs > thn::kWideMaxVecs) gains = 2 * M <= 3 * cus;
+        else if (N * bytes >= 131072 && 2 * M < cus) gains = !reads_twice || 4 * M <= cus;
+        else gains = M > cus && 5 * M <= 6 * cus && !reads_twice && softmax_wide_vecs(which, is_log, M, N, dtype, cus) == 0;
+        if (!gains) return false;
+    }
+    *out = thn::even_slices(static_cast<int>(vecs));
+    return true;
+}
+
 // Every row of every stream starts at the same offset from a 16-byte boundary, on an element.
 bool same_phase(std::initializer_list<std::pair<const void*, int64_t>> streams, int64_t M, int bytes) {
     const uintptr_t base = reinterpret_cast<uintptr_t>(streams.begin()->first);
@@ -492,6 +521,21 @@ int launch_softmax_fwd_wide(int dtype, bool is_log, int k, const SoftmaxFwdArgs&
 }
 int launch_softmax_bwd_wide(int dtype, bool is_log, int k, const SoftmaxBwdArgs& a, int grid, hipStream_t st) {
     THN_WIDE_SWITCH(launch_softmax_bwd_wide)
+}
+
+int launch_softmax_fwd_sliced(int dtype, bool is_log, const SoftmaxFwdArgs& a, const thn::Slicing& s, hipStream_t st) {
+    switch (dtype) {
+        case THN_F32: return thn::launch_softmax_fwd_sliced_f32(is_log, a, s, st);
+        case THN_F16: return thn::launch_softmax_fwd_sliced_f16(is_log, a, s, st);
+        default: return thn::launch_softmax_fwd_sliced_bf16(is_log, a, s, st);
+    }
+}
+int launch_softmax_bwd_sliced(int dtype, bool is_log, const SoftmaxBwdArgs& a, const thn::Slicing& s, hipStream_t st) {
+    switch (dtype) {
+        case THN_F32: return thn::launch_softmax_bwd_sliced_f32(is_log, a, s, st);
+        case THN_F16: return thn::launch_softmax_bwd_sliced_f16(is_log, a, s, st);
+        default: return thn::launch_softmax_bwd_sliced_bf16(is_log, a, s, st);
+    }
 }
 
 void softmax_loop_launch(int which, int* block, int* bpc) {
@@ -1945,6 +1989,14 @@ int thn_norm_query_launch(int which, int is_layernorm, int64_t M, int64_t N, int
             softmax_loop_launch(which, &block, &bpc);
             const int64_t cap = static_cast<int64_t>(cus) * bpc;
             grid = static_cast<int>(M < cap ? M : cap);
+            thn::Slicing slicing;
+            if (softmax_slicing(which, flavour & 1, M, N, x_dtype, cus, &slicing)) {      // rows cut into slices (dense tensors)
+                shape[0] = thn::kSlicedVecs;
+                shape[1] = shape[2] = thn::kSlicedBlock;
+                shape[3] = static_cast<int>(M) * slicing.slices;
+                shape[4] = 1;
+                return THN_OK;
+            }
             const int k = softmax_wide_vecs(which, flavour & 1, M, N, x_dtype, cus);
             if (k > 0) {                            // rows in the registers of a compute unit (dense tensors)
                 shape[0] = k;
@@ -2213,7 +2265,11 @@ int thn_softmax_fwd(const void* x, int64_t x_row_stride, void* y, int64_t y_row_
         int block, bpc, lrc;
         softmax_loop_launch(kSoftmaxFwd, &block, &bpc);
         const int k = softmax_wide_vecs(kSoftmaxFwd, kind == THN_LOGSOFTMAX, M, N, dtype, cus);
-        if (k > 0 && same_phase({{x, a.x_stride_bytes}, {y, a.y_stride_bytes}}, M, bytes)) {
+        const bool in_step = same_phase({{x, a.x_stride_bytes}, {y, a.y_stride_bytes}}, M, bytes);
+        thn::Slicing slicing;
+        if (in_step && softmax_slicing(kSoftmaxFwd, kind == THN_LOGSOFTMAX, M, N, dtype, cus, &slicing)) {
+            lrc = launch_softmax_fwd_sliced(dtype, kind == THN_LOGSOFTMAX, a, slicing, static_cast<hipStream_t>(stream));
+        } else if (k > 0 && in_step) {
             const int grid = static_cast<int>(M < cus ? M : cus);
             lrc = launch_softmax_fwd_wide(dtype, kind == THN_LOGSOFTMAX, k, a, grid, static_cast<hipStream_t>(stream));
         } else {
@@ -2306,7 +2362,11 @@ int thn_softmax_bwd(const void* y, int64_t y_row_stride, const void* dy, int64_t
         int block, bpc, lrc;
         softmax_loop_launch(kSoftmaxBwd, &block, &bpc);
         const int k = softmax_wide_vecs(kSoftmaxBwd, kind == THN_LOGSOFTMAX, M, N, dtype, cus);
-        if (k > 0 && same_phase({{y, a.y_stride_bytes}, {dy, a.dy_stride_bytes}, {dx, a.dx_stride_bytes}}, M, bytes)) {
+        const bool in_step = same_phase({{y, a.y_stride_bytes}, {dy, a.dy_stride_bytes}, {dx, a.dx_stride_bytes}}, M, bytes);
+        thn::Slicing slicing;
+        if (in_step && softmax_slicing(kSoftmaxBwd, kind == THN_LOGSOFTMAX, M, N, dtype, cus, &slicing)) {
+            lrc = launch_softmax_bwd_sliced(dtype, kind == THN_LOGSOFTMAX, a, slicing, static_cast<hipStream_t>(stream));
+        } else if (k > 0 && in_step) {
             const int grid = static_cast<int>(M < cus ? M : cus);
             lrc = launch_softmax_bwd_wide(dtype, kind == THN_LOGSOFTMAX, k, a, grid, static_cast<hipStream_t>(stream));
         } else {

@@ -260,7 +260,8 @@ __global__ void __launch_bounds__(BLOCK) softmax_bwd_kernel(const SoftmaxBwdArgs
 // Rows wider than 64 KiB (the reference cuts such a row into 64 KiB chunks and normalises each chunk by itself,
 // softmax.py:34-40 -- which is not a softmax of the row; here the row is one softmax).  One 1024-thread workgroup
 // per row, grid-stride over rows, two walks per row (thn_walk.h); the second comes from the L2 / Infinity Cache.  Rows that
-// a compute unit can hold in its registers run thn_softmax_wide.h instead where that is faster (softmax_wide_vecs()).
+// a compute unit can hold in its registers run thn_softmax_wide.h instead where that is faster (softmax_wide_vecs()), few rows
+// thn_softmax_sliced.h (softmax_slicing()).
 //   forward:  walk 1 keeps a running maximum m and sum(exp(x - m)) per thread (the sum is rescaled whenever the
 //             maximum moves: a few times per thread), combined over the workgroup; walk 2 writes y;
 //   backward: walk 1 sum(y*g) (log-softmax: sum(g)); walk 2 writes dx.

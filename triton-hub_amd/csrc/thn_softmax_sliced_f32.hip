@@ -1,0 +1,6 @@
+// Softmax / Softmin / LogSoftmax kernels for few rows of more than 64 KiB, cut into slices, F32 storage.
+#include "thn_softmax_sliced.h"
+
+namespace thn {
+THN_DEFINE_SOFTMAX_SLICED_LAUNCHERS(f32, F32)
+}  // namespace thn
