@@ -88,9 +88,7 @@ constexpr int kPolicyFlags = THN_X_KEEP | THN_X_STREAM;
 // `ln16`: LayerNorm over 16-bit rows (the two norm backwards have instances of their own for that).
 bool shape_compiled(int which, bool aligned, bool ln16, Shape s) {
 #define THN_MATCH(K_, TPR_, BLOCK_) if (s.k == K_ && s.tpr == TPR_ && s.block == BLOCK_) return true;
-    if (!aligned && (which == kFusedFwd || which == kFusedBwd)) {
-        THN_SCALAR_SHAPES(THN_MATCH)
-    } else if (!aligned && which == kNormBwd) {
+    if (!aligned && which == kNormBwd) {
         THN_BWD_SHAPES(THN_MATCH)
         THN_BWD_SHAPES_THREE(THN_MATCH)
     } else if (which == kNormBwd) {
@@ -103,7 +101,9 @@ bool shape_compiled(int which, bool aligned, bool ln16, Shape s) {
         THN_FUSED_FWD_SHAPES(THN_MATCH)
     } else if (which == kFusedBwd) {
         THN_FUSED_BWD_SHAPES(THN_MATCH)
-        if (ln16) {
+        if (!aligned) {
+            THN_FUSED_BWD_SHAPES_OFF_PATH(THN_MATCH)
+        } else if (ln16) {
             THN_FUSED_BWD_SHAPES_LN16(THN_MATCH)
         }
     } else if (which >= kPnormFwd) {
@@ -339,6 +339,7 @@ constexpr int kTprList[] = {8, 16, 32, 64, 128, 256, 512, 1024};
 // Workgroups per compute unit: one (kDefaultBlocksPerCu), except where default_blocks_per_cu(),
 // narrow_row_blocks_per_cu() or the row-count dependent rules in plan_launch() say otherwise.
 constexpr int kDefaultBlocksPerCu = 1;
+constexpr int kFusedBwdSharedVecs = 256;      // rows whose backward with an epilogue may share a compute unit between 256-thread workgroups
 
 int ceil_div(int a, int b) { return (a + b - 1) / b; }
 
@@ -350,8 +351,6 @@ Shape heuristic_shape(int which, bool aligned, bool ln16, int n_vecs) {
     if ((which == kNormBwd || which == kFusedBwd) && aligned && ln16 && n_vecs > 2048) {
         return Shape{ceil_div(n_vecs, 512), 512, 512};
     }
-    // (every family but the norm kernels with an activation epilogue takes the same shapes off the 128-bit path as on it)
-    const bool same_shapes = which != kFusedFwd && which != kFusedBwd;
     int kmax = (which == kNormBwd && n_vecs > 128) ? 3 : 4;
     // Softmax backward: the forward's shape up to 8 KiB rows -- as many rows per workgroup in both directions, so a row
     // meets the same XCD and its L2 (forward + backward of 2^26 elements: bfloat16 N = 512 / 2048 / 4096 101.2 / 102.7 /
@@ -360,18 +359,13 @@ Shape heuristic_shape(int which, bool aligned, bool ln16, int n_vecs) {
     // wider rows 2 vectors per thread per stream (bfloat16 N = 8192 98.5 us against 98.9, float32 N = 8192 198.7 / 200.8).
     if (which == kSoftmaxBwd && n_vecs > 512 && n_vecs <= 2048) kmax = 2;
     if (which == kNormalizeBwd && n_vecs <= 2048) kmax = 2;    // two or three input streams
-    if (aligned && which == kFusedBwd && n_vecs <= 2048) kmax = n_vecs > 128 ? 3 : 2;   // bias and pre-activation are live too
+    if (which == kFusedBwd && n_vecs <= 2048) kmax = n_vecs > 128 ? 3 : 2;   // bias and pre-activation are live too
     Shape s{4, 1024, 1024};
     for (int tpr : kTprList) {
         if (static_cast<int64_t>(tpr) * kmax >= n_vecs) {
             s.tpr = tpr;
             break;
         }
-    }
-    if (!aligned && !same_shapes) {
-        s.k = 4;
-        s.block = s.tpr > 256 ? s.tpr : 256;
-        return s;
     }
     if (which == kNormBwd && n_vecs > 8 && n_vecs <= 16) s.tpr = 16;      // 256-byte rows: one vector per thread
     s.k = ceil_div(n_vecs, s.tpr);
@@ -386,7 +380,7 @@ Shape heuristic_shape(int which, bool aligned, bool ln16, int n_vecs) {
             s.k = 3;
         }
     }
-    if (s.k == 3 && s.tpr < 64) s.k = 4;     // K = 3 is only compiled for TPR >= 64
+    if (s.k == 3 && s.tpr < (which == kFusedFwd ? 16 : 64)) s.k = 4;     // K = 3 is only compiled for TPR >= 64 (16)
     if (which != kNormBwd && which != kFusedBwd) s.block = s.tpr > 256 ? s.tpr : 256;
     else s.block = s.tpr >= 128 ? (s.tpr > 512 ? s.tpr : 512) : 256;
     if (which == kNormFwd && s.k == 3 && s.tpr == 256) s.block = 512;     // THN_FWD_SHAPES_TWO_ROWS
@@ -404,7 +398,7 @@ int default_blocks_per_cu(int which, int flavour, int block) {
     // per compute unit.
     if (which >= kPnormFwd && which <= kNormalizeBwd && block <= 256) return 2;
     // A GeLU epilogue makes the norm kernels arithmetic-bound (about 30 instruction slots per element): they take
-    // as many workgroups per compute unit as their registers allow, up to four (one exception in plan_launch()).
+    // as many workgroups per compute unit as their registers allow, up to four (exceptions in plan_launch()).
     if ((which == kFusedFwd || which == kFusedBwd) && thn::arithmetic_bound(flavour >> 1)) return 4;
     return kDefaultBlocksPerCu;
 }
@@ -846,6 +840,36 @@ int plan_launch(int which, int flavour, bool aligned, int64_t M, int64_t N, int 
         one_row.block = s.tpr;
         if (!too_empty && shape_compiled(which, aligned, ln16, one_row)) s = one_row;
     }
+    // The norm kernels with an activation epilogue in shapes of their own (THN_FUSED_FWD_SHAPES, THN_FUSED_BWD_SHAPES): 5 x t vectors for rows of 4t + 1
+    // to 5t, t = 8 ... 128, and 3 x 16 and 3 x 32 for rows of 33 to 48 and 65 to 96 vectors.  Fewer threads per row make fewer workgroups of the
+    // same rows: a forward takes them from 1.5 workgroup steps per compute unit on, a backward from 4 (one step less and a
+    // forward of 1859 x 640 takes 5.1 us instead of 4.6, a backward of 6469 x 640 19.0 instead of 17.4).  float32 rows on the 128-bit path wait
+    // for memory with any of them (640 columns 23.1 and 23.2 us); an RMSNorm without GeLU does from t = 16 down (640: 22.1 us with either).
+    if (which == kFusedFwd && N >= vec_elems) {
+        const bool many = 2 * M * s.tpr >= 3 * static_cast<int64_t>(cus) * 256;
+        int t = 8;
+        while (5 * t < n_vecs) t *= 2;
+        const Shape five{5, t, 256};
+        const bool arithmetic = thn::arithmetic_bound(flavour >> 1) || (flavour & 1) != 0;
+        if (s.tpr <= 256 && (!many || (aligned && bytes >= 4 && s.tpr < 64))) {
+            if (!aligned || s.tpr < 64) s.k = n_vecs > 2 * s.tpr ? 4 : s.k;
+        }
+        if (n_vecs > 4 * t && 2 * M * t >= 3 * static_cast<int64_t>(cus) * 256 && (t > 16 || arithmetic) && (bytes == 2 || (!aligned && t > 16)) &&
+            shape_compiled(which, aligned, ln16, five)) {
+            s = five;
+        }
+    }
+    if (which == kFusedBwd && N >= vec_elems && (fills_three_16 || fills_three_32)) {
+        const int t = fills_three_16 ? 16 : 32;
+        if (!aligned || M * t >= 4 * static_cast<int64_t>(cus) * 256) s = Shape{3, t, 256};
+    }
+    if (which == kFusedBwd && N >= vec_elems && !aligned) {
+        const bool ln = (flavour & 1) != 0;
+        const int act = flavour >> 1;
+        if (ln && bytes == 2 && !thn::arithmetic_bound(act) && n_vecs > 192 && n_vecs <= 256) s = Shape{4, 64, 256};
+        if (n_vecs > 1536 && n_vecs <= 2048 && !(ln && bytes == 2)) s = Shape{4, 512, 512};
+        if (!ln && bytes == 2 && act == thn::kGeluTanh && n_vecs > 512 && n_vecs <= 1024) s = Shape{4, 256, 256};
+    }
     const Override& ov = g_override[which];
     Shape cand = s;
     if (ov.k.load() > 0) cand.k = ov.k.load();
@@ -877,10 +901,9 @@ int plan_launch(int which, int flavour, bool aligned, int64_t M, int64_t N, int 
         // with two; softmax and normalize the same way).
         const bool one_stream = which == kNormFwd || which == kSoftmaxFwd || which == kPnormFwd || which == kFusedFwd;
         const bool shifted_one_row = pitch_bytes % 128 != 0 && s.block == s.tpr;
-        // (rows off the 128-bit path alike, except under an activation epilogue, whose one shape there has four vectors
-        // per thread: bfloat16 N = 1025 RMSNorm / LayerNorm forward 56.2 / 59.5 -> 49.9 / 53.5 us per 2^26 elements, 2049:
+        // (rows off the 128-bit path alike: bfloat16 N = 1025 RMSNorm / LayerNorm forward 56.2 / 59.5 -> 49.9 / 53.5 us per 2^26 elements, 2049:
         // 56.8 / 69.2 -> 50.8 / 55.0; float32 N = 513 106.1 / 109.4 -> 96.8 / 97.3)
-        if (one_stream && (aligned || which != kFusedFwd) && s.block * s.k < 1024 && n_vecs > 16 && cap < 2 &&
+        if (one_stream && s.block * s.k < 1024 && n_vecs > 16 && cap < 2 &&
             (!shifted_one_row || M <= 32 * static_cast<int64_t>(cus))) {
             cap = 2;
         }
@@ -915,11 +938,28 @@ int plan_launch(int which, int flavour, bool aligned, int64_t M, int64_t N, int 
             cap < 2) {
             cap = 2;
         }
-        // The float32 RMSNorm backward with a GeLU epilogue in 512-thread workgroups of 3 vectors per thread waits for memory, not
-        // for arithmetic (half the elements per byte of a 16-bit row): one workgroup, although the registers leave room for two
-        // (2^25 elements, two -> one: N = 5120 77.1 -> 71.4 us, 6000 80.2 -> 74.3; 3000 and 1536 within half a percent when one
-        // fits anyway.  LayerNorm's registers leave room for one; with 2 vectors two are as good).
-        if (which == kFusedBwd && aligned && bytes == 4 && (flavour & 1) == 0 && s.k == 3 && s.block == 512) cap = 1;
+        // Epilogues other than GeLU: more than one workgroup of 256 threads, which is one wave per SIMD, for the backward (rows of up to 192
+        // vectors) -- two from 4 workgroup steps per compute unit on, four from 16 on with 16-bit rows of up to 128 slots.  2^25 bfloat16
+        // elements, one -> four: RMSNorm + SiLU N = 256 53.7 -> 41.3 us, 512 52.0 -> 41.2, 1024 53.1 -> 41.8; LayerNorm + SiLU 256 56.1 -> 43.0, 512 55.1 -> 43.4
+        // (two 45.5), 1024 56.2 -> 44.8; one -> two: 1152 48.5 -> 42.3 and 61.4 -> 52.2, 1536 LayerNorm 51.5 -> 46.1; 2^24 float32 elements, RMSNorm + SiLU 160
+        // 49.5 -> 39.5, 320 51.0 -> 39.5.  With fewer steps (3541 x 512 9.4 -> 10.0 us) they only make more partial rows.
+        // Two, or four with more than 3 x 64 vectors per row, for the 16-bit LayerNorm forward (2048 23.3 -> 22.3, 4096 27.8 -> 23.2, 6144 24.9 -> 22.8, 896
+        // 26.0 -> 23.2, 384 two 22.2, four 23.1).
+        if ((which == kFusedBwd || which == kFusedFwd) && s.block == 256 && !thn::arithmetic_bound(flavour >> 1)) {
+            const int64_t steps = M * s.tpr / (256 * static_cast<int64_t>(cus));
+            int most = 1;
+            const bool idle = 8 * n_vecs < 7 * s.k * s.tpr;      // an eighth of the slots: full rows of 32 bits, or of 3 x 64 vectors without LayerNorm, gain nothing
+            const bool gains = bytes == 2 ? (flavour & 1) != 0 || s.k < 3 || s.tpr < 64 || idle : idle;
+            if (which == kFusedBwd && n_vecs <= kFusedBwdSharedVecs && steps >= 4 && gains) most = bytes == 2 && steps >= 16 && s.k * s.tpr <= 128 ? 4 : 2;
+            if (which == kFusedFwd && bytes == 2 && (flavour & 1) != 0 && steps >= 4) most = s.k == 4 || s.tpr >= 128 ? 4 : 2;
+            if (cap < most) cap = most;
+        }
+        // 5 vectors per thread: two, with any epilogue (LayerNorm + GeLU N = 640 30.5 us, one 32.5; RMSNorm + GeLU 1280 25.9, four 27.8).
+        if (which == kFusedFwd && s.k == 5) cap = 2;
+        // A GeLU backward in 512-thread workgroups: one, also where the registers leave room for two (2^24 float32 elements, two -> one: LayerNorm
+        // N = 1024 41.3 -> 39.5 us, 2048 43.2 -> 39.8, 4096 45.7 -> 40.3, RMSNorm 38.1 -> 36.2, 39.7 -> 38.1, 42.4 -> 38.4; 2^25 of them, RMSNorm 5120
+        // 77.1 -> 71.4, 6000 80.2 -> 74.3; 2^25 bfloat16 elements, RMSNorm 2048 43.0 -> 40.0).
+        if (which == kFusedBwd && s.block == 512 && thn::arithmetic_bound(flavour >> 1)) cap = 1;
         if ((narrow_forward_pair || narrow_backward_pair) && cap < 2) cap = 2;
         if (which == kPnormFwd && s.k == 5) cap = 1;       // 1280 vectors per workgroup step: see THN_PN_SHAPES_FIVE above
     }
@@ -1442,6 +1482,7 @@ int64_t bwd_workspace_bytes(int which, int flavour, int64_t M, int64_t N, int wa
     if (narrow > bpc) bpc = narrow;
     if (bytes == 2 && n_vecs <= 96 && bpc < 2) bpc = 2;      // the LayerNorm backward over narrow 16-bit rows (plan_launch)
     if (which == kNormBwd && n_vecs <= thn::kStagedMaxVecs && bpc < kStagedBlocksPerCu) bpc = kStagedBlocksPerCu;   // the staged kernels
+    if (which == kFusedBwd && n_vecs <= kFusedBwdSharedVecs && bpc < 4) bpc = 4;      // 256-thread workgroups (plan_launch)
     const int forced = g_override[which].bpc.load();
     if (forced > bpc) bpc = forced;
     if (bpc > kMaxBlocksPerCu) bpc = kMaxBlocksPerCu;

@@ -70,13 +70,8 @@ struct Shape {
 // live in LDS).  A 1024-thread workgroup has half as many and spills at 4 vectors per thread.
 #define THN_BWD_SHAPES_LN16(X) X(5, 512, 512) X(6, 512, 512) X(7, 512, 512) X(8, 512, 512)
 
-// Rows off the 128-bit path (N not a whole number of 16-byte vectors, or a pointer or stride off 16 bytes) run the
-// plain norm kernels in the same shapes as rows on it (their slots are 16-byte windows at element-aligned
-// addresses, the ragged last one overlapping its neighbour), and so do the softmax and p-norm families.  The norm
-// kernels with an activation epilogue keep one shape per row width there: four vectors per thread.
-#define THN_SCALAR_SHAPES(X)                                                         \
-    X(4, 8, 256) X(4, 16, 256) X(4, 32, 256) X(4, 64, 256) X(4, 128, 256)            \
-    X(4, 256, 256) X(4, 512, 512) X(4, 1024, 1024)
+// Rows off the 128-bit path (N not a whole number of 16-byte vectors, or a pointer or stride off 16 bytes) run every family in the
+// same shapes as rows on it: their slots are 16-byte windows at element-aligned addresses, the ragged last one overlapping its neighbour.
 
 // Return value of the launchers: 0 launched (or occupancy written), 1 no such instance, <0 HIP error.
 // When `occupancy` is not null the kernel is not launched; *occupancy receives the number of workgroups
