@@ -3,6 +3,7 @@ gelu.py:107-119, and the ``GeLU`` callable, :121-129)."""
 import torch
 
 from .. import _native
+from .._autograd import ACT, native_apply
 from ._launch import act_bwd, act_fwd
 
 
@@ -11,6 +12,8 @@ def _code(approximate):
 
 
 class gelu(torch.autograd.Function):
+    apply = native_apply(ACT, _native.ACT_GELU, ('approximate',))
+
     @staticmethod
     def forward(ctx, input, approximate):
         output = act_fwd(input, _code(approximate))

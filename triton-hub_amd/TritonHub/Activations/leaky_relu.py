@@ -3,10 +3,13 @@ Function, leaky_relu.py:85-97, and the ``LeakyReLU`` callable, :99-104)."""
 import torch
 
 from .. import _native
+from .._autograd import ACT, native_apply
 from ._launch import act_bwd, act_fwd
 
 
 class leakyrelu(torch.autograd.Function):
+    apply = native_apply(ACT, _native.ACT_LEAKY_RELU, ('negative_slope',))
+
     @staticmethod
     def forward(ctx, input, negative_slope):
         output = act_fwd(input, _native.ACT_LEAKY_RELU, negative_slope)

@@ -3,11 +3,14 @@
 import torch
 
 from .. import _native
+from .._autograd import SOFTMAX, native_apply
 from ._launch import softmax_bwd, softmax_fwd
 
 
 class logsoftmax(torch.autograd.Function):
     """forward(ctx, input) -> log_softmax(input, dim=-1); saves the OUTPUT; backward: dy - exp(y)*sum(dy)."""
+
+    apply = native_apply(SOFTMAX, _native.LOGSOFTMAX)
 
     @staticmethod
     def forward(ctx, input):

@@ -3,10 +3,13 @@ mish.py:91-102, and the ``Mish`` callable, :104-108).  The Function saves its in
 import torch
 
 from .. import _native
+from .._autograd import ACT, native_apply
 from ._launch import act_bwd, act_fwd
 
 
 class mish(torch.autograd.Function):
+    apply = native_apply(ACT, _native.ACT_MISH)
+
     @staticmethod
     def forward(ctx, input):
         output = act_fwd(input, _native.ACT_MISH)

@@ -3,10 +3,13 @@ relu.py:81-92, and the ``ReLU`` callable, :94-98).  The Function saves its input
 import torch
 
 from .. import _native
+from .._autograd import ACT, native_apply
 from ._launch import act_bwd, act_fwd
 
 
 class relu(torch.autograd.Function):
+    apply = native_apply(ACT, _native.ACT_RELU)
+
     @staticmethod
     def forward(ctx, input):
         output = act_fwd(input, _native.ACT_RELU)

@@ -3,10 +3,13 @@ relu6.py:83-94, and the ``ReLU6`` callable, :96-100).  The Function saves its in
 import torch
 
 from .. import _native
+from .._autograd import ACT, native_apply
 from ._launch import act_bwd, act_fwd
 
 
 class relu6(torch.autograd.Function):
+    apply = native_apply(ACT, _native.ACT_RELU6)
+
     @staticmethod
     def forward(ctx, input):
         output = act_fwd(input, _native.ACT_RELU6)

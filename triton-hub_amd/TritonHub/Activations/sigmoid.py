@@ -3,10 +3,13 @@ sigmoid.py:81-92, and the ``Sigmoid`` callable, :94-98).  The Function saves its
 import torch
 
 from .. import _native
+from .._autograd import ACT, native_apply
 from ._launch import act_bwd, act_fwd
 
 
 class sigmoid(torch.autograd.Function):
+    apply = native_apply(ACT, _native.ACT_SIGMOID, flag=True)
+
     @staticmethod
     def forward(ctx, input):
         output = act_fwd(input, _native.ACT_SIGMOID)

@@ -3,10 +3,13 @@ silu.py:82-93, and the ``SiLU`` callable, :95-99).  The Function saves its input
 import torch
 
 from .. import _native
+from .._autograd import ACT, native_apply
 from ._launch import act_bwd, act_fwd
 
 
 class silu(torch.autograd.Function):
+    apply = native_apply(ACT, _native.ACT_SILU)
+
     @staticmethod
     def forward(ctx, input):
         output = act_fwd(input, _native.ACT_SILU)

@@ -3,11 +3,14 @@
 import torch
 
 from .. import _native
+from .._autograd import SOFTMAX, native_apply
 from ._launch import softmax_bwd, softmax_fwd
 
 
 class softmax(torch.autograd.Function):
     """forward(ctx, input) -> softmax(input, dim=-1); saves the OUTPUT; backward: y*dy - y*sum(y*dy)."""
+
+    apply = native_apply(SOFTMAX, _native.SOFTMAX)
 
     @staticmethod
     def forward(ctx, input):

@@ -9,11 +9,14 @@ gives the same values and gradients as negating with a tensor op.
 import torch
 
 from .. import _native
+from .._autograd import SOFTMAX, native_apply
 from ._launch import softmax_bwd, softmax_fwd
 
 
 class softmin(torch.autograd.Function):
     """forward(ctx, input) -> softmax(input, dim=-1), exactly as in the reference; saves the output."""
+
+    apply = native_apply(SOFTMAX, _native.SOFTMAX)
 
     @staticmethod
     def forward(ctx, input):
@@ -29,6 +32,8 @@ class softmin(torch.autograd.Function):
 
 class _softmin_of(torch.autograd.Function):
     """forward(ctx, x) -> softmax(-x, dim=-1) in one pass; backward returns d/dx, sign included."""
+
+    apply = native_apply(SOFTMAX, _native.SOFTMIN)
 
     @staticmethod
     def forward(ctx, input):

@@ -3,10 +3,13 @@ Function, softplus.py:89-102, and the ``Softplus`` callable, :104-110)."""
 import torch
 
 from .. import _native
+from .._autograd import ACT, native_apply
 from ._launch import act_bwd, act_fwd
 
 
 class softplus(torch.autograd.Function):
+    apply = native_apply(ACT, _native.ACT_SOFTPLUS, ('beta', 'threshold'))
+
     @staticmethod
     def forward(ctx, input, beta, threshold):
         output = act_fwd(input, _native.ACT_SOFTPLUS, beta, threshold)

@@ -3,10 +3,13 @@ tanh.py:83-94, and the ``Tanh`` callable, :96-100).  The Function saves its OUTP
 import torch
 
 from .. import _native
+from .._autograd import ACT, native_apply
 from ._launch import act_bwd, act_fwd
 
 
 class tanh(torch.autograd.Function):
+    apply = native_apply(ACT, _native.ACT_TANH, flag=True)
+
     @staticmethod
     def forward(ctx, input):
         output = act_fwd(input, _native.ACT_TANH)

@@ -3,10 +3,13 @@ Function, threshold.py:85-100, and the ``Threshold`` callable, :102-108)."""
 import torch
 
 from .. import _native
+from .._autograd import ACT, native_apply
 from ._launch import act_bwd, act_fwd
 
 
 class threshold_fn(torch.autograd.Function):
+    apply = native_apply(ACT, _native.ACT_THRESHOLD, ('threshold', 'value'))
+
     @staticmethod
     def forward(ctx, input, threshold, value):
         output = act_fwd(input, _native.ACT_THRESHOLD, threshold, value)

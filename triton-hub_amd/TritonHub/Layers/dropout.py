@@ -11,6 +11,7 @@ import random
 import torch
 
 from .. import _native
+from .._autograd import PYTHON, native_apply
 from ..Activations._launch import _call
 
 
@@ -46,6 +47,8 @@ class dropout(torch.autograd.Function):
     gives them back; every other backward, a second one among them, regenerates the mask from the seed.  The two give the
     same bits.  The mask is no saved tensor, as the seed is none, so a graph can be walked again without retain_graph; under
     saved-tensor hooks, which would not see it, and so in a non-reentrant checkpoint, none is kept."""
+
+    apply = native_apply(PYTHON)
 
     @staticmethod
     def forward(ctx, input, p, training):

@@ -11,6 +11,7 @@ rounded to the storage type, results are closer to exact arithmetic than the cha
 import torch
 
 from .. import _native
+from .._autograd import LAYERNORM, RMSNORM, native_apply
 from ._launch import norm_bwd, norm_fwd
 from .layernorm import LayerNorm
 from .rmsnorm import RMSNorm
@@ -26,6 +27,8 @@ def _code(activation: str) -> int:
 
 class layernorm_act(torch.autograd.Function):
     """forward(ctx, input, weight, bias, eps, act) -> act(layernorm(input)); saves what ``layernorm`` saves."""
+
+    apply = native_apply(LAYERNORM, params=('eps', 'act'), flag=True)
 
     @staticmethod
     def forward(ctx, input, weight, bias, eps, act):
@@ -46,6 +49,8 @@ class layernorm_act(torch.autograd.Function):
 
 class rmsnorm_act(torch.autograd.Function):
     """forward(ctx, input, weight, eps, act) -> act(rmsnorm(input)); saves what ``rmsnorm`` saves."""
+
+    apply = native_apply(RMSNORM, params=('eps', 'act'), flag=True)
 
     @staticmethod
     def forward(ctx, input, weight, eps, act):

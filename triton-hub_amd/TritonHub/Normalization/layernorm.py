@@ -5,12 +5,15 @@ module (layernorm.py:225-252) -- with the Triton kernels replaced by HIP kernels
 """
 import torch
 
+from .._autograd import LAYERNORM, native_apply
 from ._launch import norm_bwd, norm_fwd
 
 
 class layernorm(torch.autograd.Function):
     """forward(ctx, input, weight, bias, eps) -> output; saves (input, weight, bias, mean, rstd), the last two
     being (M,) float32 row statistics: mean = sum(x)/N, rstd = 1/sqrt(biased variance + eps)."""
+
+    apply = native_apply(LAYERNORM, params=('eps',))
 
     @staticmethod
     def forward(ctx, input, weight, bias, eps):

@@ -5,12 +5,15 @@ Same public surface -- the ``rmsnorm`` autograd Function (rmsnorm.py:169-181) an
 """
 import torch
 
+from .._autograd import RMSNORM, native_apply
 from ._launch import norm_bwd, norm_fwd
 
 
 class rmsnorm(torch.autograd.Function):
     """forward(ctx, input, weight, eps) -> output; saves (input, weight, rstd) with rstd the (M,) float32
     row statistic 1/sqrt(mean(x^2) + eps)."""
+
+    apply = native_apply(RMSNORM, params=('eps',))
 
     @staticmethod
     def forward(ctx, input, weight, eps):

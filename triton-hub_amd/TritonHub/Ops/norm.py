@@ -2,14 +2,16 @@
 reference (the ``Norm`` autograd Function, norm.py:128-144, and the ``norm`` callable, :146-154)."""
 import torch
 
+from .._autograd import PNORM, native_apply
 from ._launch import norm_bwd, norm_fwd
 
 
 class Norm(torch.autograd.Function):
     """forward(ctx, x, p=2, eps=1e-6) -> max(||x||_p, eps) of shape (B, L) in x.dtype; saves (x, norms)."""
 
+    apply = native_apply(PNORM)
+
     @staticmethod
-    @torch.amp.custom_fwd(device_type='cuda')
     def forward(ctx, x, p=2, eps=1e-6):
         assert len(x.shape) == 3, "Expected Tensor to be 3D (B, L, D), add batch dim input is 2D"
         ctx.p = p
@@ -18,7 +20,6 @@ class Norm(torch.autograd.Function):
         return norms_x
 
     @staticmethod
-    @torch.amp.custom_bwd(device_type='cuda')
     def backward(ctx, grad_output):
         p = ctx.p
         x, norms_x = ctx.saved_tensors

@@ -3,14 +3,16 @@
 ``normalize`` callable, :162-170)."""
 import torch
 
+from .._autograd import NORMALIZE, native_apply
 from ._launch import normalize_bwd, normalize_fwd
 
 
 class Normalize(torch.autograd.Function):
     """forward(ctx, x, p=2, eps=1e-6) -> x_norm; saves (x, x_norm, norms) with the norms in x.dtype."""
 
+    apply = native_apply(NORMALIZE)
+
     @staticmethod
-    @torch.amp.custom_fwd(device_type='cuda')
     def forward(ctx, x, p=2, eps=1e-6):
         assert len(x.shape) == 3, "Expected Tensor to be 3D (B, L, D), add batch dim input is 2D"
         ctx.p = p
@@ -19,7 +21,6 @@ class Normalize(torch.autograd.Function):
         return x_norm
 
     @staticmethod
-    @torch.amp.custom_bwd(device_type='cuda')
     def backward(ctx, grad_output):
         p = ctx.p
         x, x_norm, norms_x = ctx.saved_tensors
