@@ -61,8 +61,9 @@ __device__ __forceinline__ float gelu_tanh_gate(float x) { return gelu_tanh_gate
 // LITERALS: |t| in a register of its own, an instruction more, and the coefficients in the instructions.  That is the faster
 // one where little else is in flight, without -> with, us: the element-wise forward of 2^23 and 2^24 bfloat16 elements 6.8-7.1 -> 6.3-6.7
 // and 12.0 -> 11.3 (2^26 42.6 -> 42.3; before degree 7 6.6, 11.5 and 43.7; float16 9.5 -> 9.5 and 12.4 -> 12.3, before 9.2 and 12.0), 2^22 float64
-// elements 10.1 -> 9.8, and the norm forwards off the 128-bit path (RMSNorm, 2^26 bfloat16 elements, 4098 columns 94.9 -> 92.1).  The
-// forwards on that path lose 2-4 % by it (RMSNorm + GeLU bfloat16 1536 columns 47.0 -> 49.0), and the backwards spill.
+// elements 10.1 -> 9.8, and the norm forwards off the 128-bit path.  Those on it lose 2-4 % by it, and the backwards spill.  (The norms over 16-bit
+// rows go by the tables of thn_gelu_table.h instead; the element-wise kernels gained with 2^26 elements, forward + backward 109 -> 106 us, but lost
+// up to 4 % at 2^22 and 2^24, where filling the table counts.)
 struct NormalParts {
     float tq, e, step;      // t_s*Q(t), exp(-x^2/2), x < 0 ? 0 : 1
 };

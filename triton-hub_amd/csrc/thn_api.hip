@@ -960,6 +960,9 @@ int plan_launch(int which, int flavour, bool aligned, int64_t M, int64_t N, int 
         // N = 1024 41.3 -> 39.5 us, 2048 43.2 -> 39.8, 4096 45.7 -> 40.3, RMSNorm 38.1 -> 36.2, 39.7 -> 38.1, 42.4 -> 38.4; 2^25 of them, RMSNorm 5120
         // 77.1 -> 71.4, 6000 80.2 -> 74.3; 2^25 bfloat16 elements, RMSNorm 2048 43.0 -> 40.0).
         if (which == kFusedBwd && s.block == 512 && thn::arithmetic_bound(flavour >> 1)) cap = 1;
+        // and in 256-thread workgroups over 16-bit rows on the 128-bit path for RMSNorm two, where the registers leave room for three (2^25 bfloat16 elements, three ->
+        // two: N = 256 43.6 -> 39.0 us, 512 43.4 -> 39.0, 1024 44.8 -> 38.9; LayerNorm the other way, 256 45.2 and 41.3).
+        if (which == kFusedBwd && s.block == 256 && aligned && bytes == 2 && flavour == 2 * thn::kGelu && cap > 2) cap = 2;
         if ((narrow_forward_pair || narrow_backward_pair) && cap < 2) cap = 2;
         if (which == kPnormFwd && s.k == 5) cap = 1;       // 1280 vectors per workgroup step: see THN_PN_SHAPES_FIVE above
     }

@@ -20,7 +20,7 @@
 
 #include <type_traits>
 
-#include "thn_act_math.h"
+#include "thn_gelu_table.h"
 #include "thn_device.h"
 
 namespace thn {
@@ -199,8 +199,9 @@ constexpr RowForm bwd_form() {
     return RowForm{true, !LN, true};     // K = 3, 4: rows of more than 32 KiB
 }
 
-// Epilogues that make the norm kernels arithmetic-bound: vector instructions issue in 98 % of the busy cycles of a LayerNorm + GeLU
-// forward and in 91 % of its backward's (bfloat16 16384 x 4096, 28.1 and 37.6 per element).  Two attempts to fill the rest measured slower, forward + backward
+// Epilogues with so much arithmetic that it shapes the kernels: with GeLU as a polynomial vector instructions issued in 98 % of the busy cycles
+// of a LayerNorm + GeLU forward and in 91 % of its backward's (bfloat16 16384 x 4096, 28.1 and 37.6 per element), the tanh form
+// needs as many.  By table (gelu_tabled below) the forward is at the rate of its memory.  Two attempts with the polynomial to fill the rest measured slower, forward + backward
 // against 139.8 us: requesting the next row into the registers of the present one, once that is unpacked (no copies,
 // 16 and 8 instructions per row fewer) 141.3 to 143.1; w and b in LDS, which makes room for four waves per SIMD instead of three and two,
 // 143.2.  Under a profiler, with pauses between the launches, the latter's backward is 7 % faster: back to back the clock falls.
@@ -222,6 +223,24 @@ template <typename T, bool LN, int ACT, bool ALIGNED, bool BWD> constexpr bool s
     if (T::kBytes != 2 || !arithmetic_bound(ACT) || threads_per_row < 64) return false;
     return LN ? ALIGNED || BWD : ALIGNED && BWD && ACT == kGelu && threads_per_row == 64;
 }
+
+// Which GeLU epilogues go by the tables of thn_gelu_table.h.  Polynomial -> table, us of 2^26 bfloat16 elements, forward and backward:
+// LayerNorm 256 columns 56.1 -> 44.1 and 84.3 -> 73.5, 1024 53.9 -> 44.3 and 81.8 -> 74.0, 4096 54.6 -> 44.5 and 88.0 -> 74.6, 8192 55.9 -> 44.5 and 90.6 -> 78.0, 16384
+// 56.8 -> 46.3 and 153.5 -> 117.7, 32768 61.6 -> 51.9 and 194.5 -> 180.0; RMSNorm 4096 48.0 -> 43.2 and 74.7 -> 70.4, 16384 50.1 -> 41.9 and 115.3 -> 83.3; off
+// the 128-bit path LayerNorm 250 88.3 -> 52.3 and 90.4 -> 82.8, 4098 76.4 -> 59.9 and 130.2 -> 98.6, RMSNorm 4098 60.7 -> 46.7 and 102 -> 82 (250 backward
+// 86.5 -> 88.4).  Calls of a few rows pay for filling the table: LayerNorm 200 x 8001 forward 5.3 -> 5.6, 128 x 256 the same.
+// Not: float64, whose backward adds in float64; 1024-thread backwards off the 128-bit path where its registers spill (LayerNorm 1973 x 17001
+// 139 -> 231 us), and float32, which waits for memory, but for the LayerNorm backward (2^25 elements, 8192 columns 80.3 -> 77.5,
+// 4099 93.5 -> 81.4, 1024 to 4096 the same; narrower ones, and the forward, lost 2 to 4 % by it).
+template <typename T, bool LN, int ACT, bool BWD, bool ALIGNED, int K, int TPR> constexpr bool gelu_tabled() {
+    if (ACT != kGelu || T::kBytes == 8) return false;
+    if (T::kBytes == 4) return LN && BWD && TPR >= 128 && (ALIGNED || TPR < 1024);
+    return !(BWD && !ALIGNED && TPR == 1024 && (K >= 3 || LN));
+}
+
+// All reads of a vector under way at once (gelu_by_table) where there are registers for it: 2^25 bfloat16 elements, RMSNorm forward 256
+// columns 23.3 -> 22.4 us, LayerNorm forward 1024 25.0 -> 24.3; the backward of 16384 columns 73 -> 85, of 32768 112 -> 126, both spilling.
+template <bool ALIGNED, int K> constexpr bool gelu_batched(int block) { return ALIGNED && block <= 512 && K <= 4; }
 
 // Makes the compiler forget what it has derived from the packed vectors, so that the next pass really
 // unpacks them again instead of keeping the float32 values of the previous pass in registers.  No instruction.
@@ -277,6 +296,18 @@ __global__ void __launch_bounds__(BLOCK) norm_fwd_kernel(const FwdArgs a) {
     float br[LN ? K : 1][VEC];
     slot_params<T, K, ALIGNED>(wr, a.w, a.w_dtype, voff, a.n_cols, 1.0f);
     if constexpr (LN) slot_params<T, K, ALIGNED>(br, a.b, a.w_dtype, voff, a.n_cols, 0.0f);
+
+    constexpr bool kTable = gelu_tabled<T, LN, ACT, false, ALIGNED, K, TPR>();
+    __shared__ f32x4 gelu_table[kTable ? kGeluNodes : 1];
+    if constexpr (kTable) fill_gelu_table<false, BLOCK>(gelu_table, tid);
+    auto activate = [&](float (&z)[VEC]) {
+        if constexpr (kTable) {
+            gelu_by_table<false, gelu_batched<ALIGNED, K>(BLOCK)>(z, gelu_table);
+        } else if constexpr (ACT != kNoAct) {
+#pragma unroll
+            for (int e = 0; e < VEC; ++e) z[e] = act_fwd<ACT, float, !ALIGNED>(z[e], 0.0f, 0.0f);
+        }
+    };
 
     drain_vector_memory(cur);
     constexpr RowForm kForm = fwd_form<T::kBytes, LN, K, BLOCK, ACT != kNoAct>();
@@ -358,8 +389,8 @@ __global__ void __launch_bounds__(BLOCK) norm_fwd_kernel(const FwdArgs a) {
                     } else {
                         yf[e] = xf[e] * rstd * wr[k][e];
                     }
-                    if constexpr (ACT != kNoAct) yf[e] = act_fwd<ACT, float, !ALIGNED>(yf[e], 0.0f, 0.0f);
                 }
+                activate(yf);
                 slot_store<T, ALIGNED>(yrow, voff[k], a.n_cols, yf);
                 if constexpr (kForm.ahead) cur[k] = nxt[k];
                 else cur[k] = slot_load<T, ALIGNED, kKeepX>(nxrow, voff[k], a.n_cols);
@@ -449,8 +480,8 @@ __global__ void __launch_bounds__(BLOCK) norm_fwd_kernel(const FwdArgs a) {
                 if constexpr (LN && arithmetic_bound(ACT)) yf[e] = fmaf(fmaf(xf[k][e], rstd, shift_y), wr[k][e], br[k][e]);
                 else if constexpr (LN) yf[e] = fmaf((xf[k][e] - delta) * rstd, wr[k][e], br[k][e]);
                 else yf[e] = xf[k][e] * rstd * wr[k][e];
-                if constexpr (ACT != kNoAct) yf[e] = act_fwd<ACT, float, !ALIGNED>(yf[e], 0.0f, 0.0f);
             }
+            activate(yf);
             slot_store<T, ALIGNED>(yrow, voff[k], a.n_cols, yf);
         }
         // Every thread of the row stores the same two words to the same address (one request per wave): a
@@ -593,6 +624,15 @@ __global__ void __launch_bounds__(BLOCK) norm_bwd_kernel(const BwdArgs a) {
         }
     }
 
+    constexpr bool kTable = gelu_tabled<T, LN, ACT, true, ALIGNED, K, TPR>();
+    __shared__ f32x4 gelu_table[kTable ? kGeluNodes : 1];
+    if constexpr (kTable) fill_gelu_table<true, BLOCK>(gelu_table, tid);
+    constexpr bool kBatched = kTable && gelu_batched<ALIGNED, K>(BLOCK);
+    auto through_activation = [&](float z, float dy) -> float {             // dy * act'(z)
+        if constexpr (kTable) return dy * gelu_by_table<true>(z, gelu_table);
+        else return act_bwd<ACT, float>(z, dy, 0.0f, 0.0f);
+    };
+
     // One grid-stride step.  MASKED is only needed for the last step of a workgroup, where some of its row
     // groups may have run past the end and mirror the last row: they must add nothing to dW / dB.
     auto step = [&](auto masked_tag) {
@@ -635,19 +675,30 @@ __global__ void __launch_bounds__(BLOCK) norm_bwd_kernel(const BwdArgs a) {
         for (int k = 0; k < K; ++k) {
             if constexpr (!(FUSED && LN)) T::unpack(cx[k], u[k]);
             T::unpack(cg[k], gf[k]);
+            float slope[kBatched ? VEC : 1];
+            if constexpr (kBatched) {
+#pragma unroll
+                for (int e = 0; e < VEC; ++e) {
+                    u[k][e] = LN ? fmaf(u[k][e], c_rstd, -dlt_fused) : u[k][e] * c_rstd;
+                    slope[e] = LN ? fmaf(u[k][e], wr[k][e], br[k][e]) : u[k][e] * wr[k][e];
+                }
+                gelu_by_table<true, true>(slope, gelu_table);
+            }
             float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f;
 #pragma unroll
             for (int e = 0; e < VEC; ++e) {
-                if constexpr (FUSED && LN) {
+                if constexpr (kBatched) {
+                    gf[k][e] *= slope[e];                               // dy * act'(z)
+                } else if constexpr (FUSED && LN) {
                     u[k][e] = fmaf(u[k][e], c_rstd, -dlt_fused);        // the corrected xhat
                 } else if constexpr (LN) {
                     u[k][e] = (u[k][e] - c_mean) * c_rstd;
                 } else {
                     u[k][e] *= c_rstd;
                 }
-                if constexpr (FUSED) {
+                if constexpr (FUSED && !kBatched) {
                     const float z = LN ? fmaf(u[k][e], wr[k][e], br[k][e]) : u[k][e] * wr[k][e];
-                    gf[k][e] = act_bwd<ACT, float>(z, gf[k][e], 0.0f, 0.0f);       // dy * act'(z)
+                    gf[k][e] = through_activation(z, gf[k][e]);
                 }
                 wdy[k][e] = wr[k][e] * gf[k][e];
                 const bool in = counts(k, e);
@@ -754,7 +805,7 @@ __global__ void __launch_bounds__(BLOCK) norm_bwd_kernel(const BwdArgs a) {
                 if constexpr (FUSED) {
                     if (corrected) {
                         const float z = LN ? fmaf(u[e], wr[k][e], br[k][e]) : u[e] * wr[k][e];
-                        gf[e] = act_bwd<ACT, float>(z, gf[e], 0.0f, 0.0f);
+                        gf[e] = through_activation(z, gf[e]);
                     }
                 }
             }
