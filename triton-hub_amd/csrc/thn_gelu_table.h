@@ -1,12 +1,16 @@
 // GeLU from tables in LDS, for the kernels over 16-bit rows in which vector instructions would bound it: the norms with a GeLU
 // epilogue.  The normal distribution function Phi and GeLU' = Phi(x) + x*phi(x) are cut into intervals of 1/32 between -14
-// and 6, each with a cubic of its own around its middle (10 KiB per table).  A value costs 8 vector instructions and one 16-byte
-// read of LDS, which another pipe carries out, where the polynomial of thn_act_math.h takes 19 and 20 slots.
+// and 6, each with a cubic of its own around its middle (10 KiB per table, which a workgroup fills while its first rows arrive).  A value costs 8
+// or 9 vector instructions and one 16-byte read of LDS, which another pipe carries out, where the polynomial of thn_act_math.h takes 19 and 20
+// slots: 2^25 normally distributed values in registers 15.2 -> 9.1 us, about 16 cycles of LDS per 64 lanes, more than half of them bank
+// conflicts of lanes at different nodes.  LayerNorm + GeLU bfloat16 16384 x 4096: 28.1 and 37.6 vector instructions per element -> 21.1 and 28.7,
+// forward + backward 145.4 -> 124.8 us, the forward then at the rate of its memory.  Intervals of 1/32 keep the tables small (finer
+// ones would be more to fill) at the accuracy below.  Which kernels use it, with both sides over other widths: gelu_tabled() in thn_kernels.h.
 //
 // The cubics are the Taylor polynomials of degree 5 economised over the interval (the Chebyshev polynomials of degree 4 and 5 taken
 // off), off by at most x^4 * 3.1e-10 of the value: below a rounded coefficient for |x| < 4.  Against float64, 2-norm, polynomial -> table: GeLU of
-// normal values 3.88e-8 -> 3.23e-8 (at 1.5 times their spread and an offset of 0.25 3.30e-8 -> 3.14e-8), GeLU' 4.83e-8 -> 3.80e-8 (4.26e-8 -> 4.13e-8); Phi in bands of x [-2, -1] 1.2e-7 -> 3.6e-8, [-6, -5] 1.1e-6 -> 1.4e-7, [-9, -8] 2.0e-6 -> 9.0e-7,
-// [-13, -12] 5.2e-6 -> 4.6e-6; GeLU' from 1 up, where it is 1 but for a rounded coefficient, 3.4e-8 -> 4.9e-8.
+// normal values 3.88e-8 -> 3.23e-8 (at 1.5 times their spread and an offset of 0.25 3.30e-8 -> 3.14e-8), GeLU' 4.83e-8 -> 3.80e-8 (4.26e-8 -> 4.13e-8);
+// Phi in bands of x [-2, -1] 1.2e-7 -> 3.6e-8, [-6, -5] 1.1e-6 -> 1.4e-7, [-9, -8] 2.0e-6 -> 9.0e-7, [-13, -12] 5.2e-6 -> 4.6e-6; GeLU' from 1 up, where it is 1 but for a rounded coefficient, 3.4e-8 -> 4.9e-8.
 #pragma once
 
 #include "thn_act_math.h"
