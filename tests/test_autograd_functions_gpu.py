@@ -108,3 +108,31 @@ def test_the_cache_policy_is_read_at_each_call(monkeypatch):
         seen.append(observed(function(NORMS + "layernorm", "layernorm").apply, (W, B, 1e-5), "bf16", True))
     for other in seen[1:]:
         assert all(torch.equal(a, b) for a, b in zip(seen[0], other) if isinstance(a, torch.Tensor))
+
+
+@pytest.mark.parametrize("form", ["f32", "strided"])
+@pytest.mark.parametrize("name", CASES)
+def test_saved_tensors_are_read_once(name, form):
+    """A non-reentrant checkpoint's hooks refuse a second reading, whichever way the backward of this input goes."""
+    from torch.utils.checkpoint import checkpoint
+    module, cls, args = CASES[name]
+    apply = function(module, cls).apply
+    print(f"{name} {form}", flush=True)
+    w, b = (torch.linspace(-1, 2, 68, device="cuda") for _ in range(2))
+    arguments = [w if a is W else b if a is B else a for a in args]
+    gradients = []
+    for run in (lambda t: apply(t, *arguments), lambda t: checkpoint(lambda u: apply(u, *arguments), t, use_reentrant=False)):
+        random.seed(5)
+        x = make_input(form).requires_grad_(True)
+        y = run(x)
+        random.seed(5)
+        gradients += torch.autograd.grad(y, x, torch.linspace(-1, 1, y.numel(), device="cuda").view(y.shape))
+    assert torch.equal(*gradients)
+    read = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: read.append(t) or t):
+        random.seed(5)
+        y = apply(make_input(form).requires_grad_(True), *arguments)
+    held = sum(t is not None for t in y.grad_fn.saved_tensors)
+    read.clear()
+    y.backward(torch.ones_like(y))
+    assert len(read) == held

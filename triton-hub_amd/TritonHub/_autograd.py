@@ -17,6 +17,17 @@ from . import _native
 LAYERNORM, RMSNORM, SOFTMAX, ACT, PNORM, NORMALIZE, PYTHON = range(7)       # enum Kind in csrc/thn_host.cpp
 
 
+class ReadContext:
+    """A Function's context whose saved tensors have been read already, for the Python backward to go on with."""
+    __slots__ = ("ctx", "saved_tensors")
+
+    def __init__(self, ctx, saved_tensors):
+        self.ctx, self.saved_tensors = ctx, saved_tensors
+
+    def __getattr__(self, name):
+        return getattr(self.ctx, name)
+
+
 class native_apply:
     """``kind`` and ``code``: which operator; ``params``: the names under which the context keeps the arguments behind the tensors;
     ``flag``: an activation code follows (norms), the output is saved (activations).  The class attribute is replaced when it is
@@ -46,6 +57,6 @@ class native_apply:
         quick._backward_cls = owner._backward_cls          # one class of nodes, whichever way they were made
         owner._backward_cls.apply = backward
         from .Normalization import _launch
-        _native.host().autograd_function_ready(capsule, super(torch.autograd.Function, quick).apply, _launch.__dict__)
+        _native.host().autograd_function_ready(capsule, super(torch.autograd.Function, quick).apply, _launch.__dict__, ReadContext)
         owner.apply = classmethod(apply)
         return getattr(cls, 'apply')

@@ -440,6 +440,7 @@ struct Ref {                                 // an owned reference
 
 PyObject *n_to_save, *n_saved_tensors, *n_needs_input_grad, *n_eps, *n_act, *n_p, *n_cache_policy;
 PyObject* g_norm_launch_dict = nullptr;      // TritonHub.Normalization._launch: its cache policy
+PyObject* g_read_context = nullptr;          // TritonHub._autograd.ReadContext
 
 Function* function_of(PyObject* capsule) { return static_cast<Function*>(PyCapsule_GetPointer(capsule, "TritonHub.Function")); }
 
@@ -594,8 +595,8 @@ template <size_t N> PyObject* gradients(const at::Tensor (&tensors)[N], Py_ssize
     return result;
 }
 
-// backward(ctx, d_out) -> gradients.  The Python backward takes every form that is not made here, the errors of freed or
-// changed saved tensors included.
+// backward(ctx, d_out) -> gradients.  The Python backward takes every form that is not made here.  The saved tensors are read once (a
+// checkpoint's hooks allow no second time): it gets a context that holds them.
 PyObject* function_backward(PyObject* self, PyObject* const* args, Py_ssize_t nargs) {
     HANDLE_TH_ERRORS
     const Function& f = *function_of(self);
@@ -649,8 +650,12 @@ PyObject* function_backward(PyObject* self, PyObject* const* args, Py_ssize_t na
             result = behind == 0 ? THPVariable_Wrap(dx[0]) : gradients(dx, 1, 1 + behind);
         }
     }
-    if (call == Call::kGeneral) return call_python(f.backward, args, nargs);
-    return result;
+    if (call != Call::kGeneral) return result;
+    PyObject* const parts[2] = {ctx, saved.p};
+    const Ref read(call_python(g_read_context, parts, 2));
+    if (!read) return nullptr;
+    PyObject* const again[2] = {read.p, d_out};
+    return call_python(f.backward, again, 2);
     END_HANDLE_TH_ERRORS
 }
 
@@ -722,13 +727,14 @@ PyObject* autograd_function(PyObject*, PyObject* const* args, Py_ssize_t nargs) 
     END_HANDLE_TH_ERRORS
 }
 
-// autograd_function_ready(capsule, torch's C apply of the class with the native forward, the module dictionary with the cache policy)
+// autograd_function_ready(capsule, torch's C apply of the class with the native forward, the module dictionary with the cache policy, ReadContext)
 PyObject* autograd_function_ready(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     HANDLE_TH_ERRORS
-    if (wrong_count(nargs, 3)) return nullptr;
+    if (wrong_count(nargs, 4)) return nullptr;
     Function* f = function_of(args[0]);
     if (f == nullptr) return nullptr;
     if (g_norm_launch_dict == nullptr) g_norm_launch_dict = Py_NewRef(args[2]);
+    if (g_read_context == nullptr) g_read_context = Py_NewRef(args[3]);
     f->apply = Py_NewRef(args[1]);
     Py_RETURN_NONE;
     END_HANDLE_TH_ERRORS
